@@ -18,7 +18,7 @@ the package's public classes (qcdgpu_amd.Lattice, Batch, flow.Flow):
   evaluate log density and action of given configurations (the inverse flow)
   learned  chains that alternate a heatbath sweep and a learned Metropolis
            sweep, measured every step
-  train    optimiser steps of the flow on given configurations
+  train    the flow's training objective and its gradient on given batches
 
 A lattice's links stay on the card between calls; a pass that ends a run
 reads them back, as a user who stores the configuration does.  Ensembles and
@@ -74,7 +74,9 @@ def listed():
         dict(name="flow_evaluate_1", kind="evaluate", n1=8, n2=8, n3=8, n4=4, layers=8, bins=4, batch=1, beta=2.2),
         # Heatbath + learned sweep chain at 8^3 x 4, beta 2.2.
         dict(name="flow_chain_8x8x8x4", kind="learned", n1=8, n2=8, n3=8, n4=4, layers=8, bins=4, beta=2.2, steps=50),
-        # Two optimiser steps on batches of 16 configurations.
+        # Loss and gradient of two batches of 16 configurations (forward and
+        # backward through every layer; the optimiser's element-wise step is
+        # left to the caller, since it scales vanishing components up).
         dict(name="flow_train_16", kind="train", n1=8, n2=8, n3=8, n4=4, layers=8, bins=4, batch=16, steps=2),
     ]
 
@@ -316,8 +318,8 @@ def run(state):
         return dict(plaquette=plq, polyakov=poly, wilson=lat.wilson_measurements(raw=True), links=lat.export_links(),
                     accepted=accepted, proposed=proposed)
     flow, B = state["flow"], case["batch"]
-    losses = [flow.train_step(state["data"][k * B:(k + 1) * B], 1e-3) for k in range(case["steps"])]
-    return dict(losses=np.array(losses), params=flow.get_params())
+    out = [flow.train_grad(state["data"][k * B:(k + 1) * B]) for k in range(case["steps"])]
+    return dict(losses=np.array([o[0] for o in out]), grads=[o[1] for o in out])
 
 
 # ------------------------------------------------------------------ work
@@ -353,7 +355,7 @@ def work(case):
     if kind == "learned":
         return dict(bytes=case["steps"] * (par + 2 * cfg + 4 * V * (9 * 16 + 32)), flops=case["steps"] * conv)
     if kind == "train":
-        return dict(bytes=case["steps"] * (case["batch"] * cfg + 14 * par), flops=case["steps"] * 3 * case["batch"] * conv)
+        return dict(bytes=case["steps"] * (case["batch"] * cfg + 3 * par), flops=case["steps"] * 3 * case["batch"] * conv)
     return dict(bytes=case["batch"] * cfg + par, flops=case["batch"] * conv)
 
 
@@ -593,8 +595,8 @@ def _exact_evaluate(case, seed):
 def _exact_train(case, seed):
     f, p = _Flow64(case), _flow_params(case, seed).double()
     data = _quaternions(case, seed + 1, case["batch"] * case["steps"]).double()
-    m, v, losses = torch.zeros_like(p), torch.zeros_like(p), []
-    for k, L in enumerate(data.split(case["batch"])):
+    losses, grads = [], []
+    for L in data.split(case["batch"]):
         grad, loss = torch.zeros_like(p), 0.0
         for l in range(case["layers"]):   # a layer's loss depends on its own parameters only
             for part in L.split(8):
@@ -603,7 +605,5 @@ def _exact_train(case, seed):
                 grad += torch.autograd.grad(lj, q)[0]
                 loss += float(lj.detach())
         losses.append(loss / case["batch"])
-        grad /= case["batch"]
-        m, v = 0.9 * m + 0.1 * grad, 0.999 * v + 0.001 * grad * grad
-        p = p - 1e-3 * (m / (1 - 0.9 ** (k + 1))) / (torch.sqrt(v / (1 - 0.999 ** (k + 1))) + 1e-8)
-    return dict(losses=np.array(losses), params=p.cpu().numpy())
+        grads.append(grad.cpu().numpy())
+    return dict(losses=np.array(losses), grads=grads)
