@@ -129,10 +129,12 @@ int  qcd_lattice_sync(qcd_lattice *lat);
                           workgroup b runs on XCD b mod 8) updates:
                           0: hardware order;
                           1: one contiguous range of compact site indices
-                          per XCD, an x-slab;
+                          per XCD, an x-slab (its x-values side by side where
+                          N1 is a multiple of 8);
                           2 (default): the same x-slabs, dispatched
-                          cross-section first (x offset, then t, then z)
-                          for L2 reuse;
+                          cross-section first (x offset, then t, then z; on
+                          large lattices four z-groups before t) for L2
+                          reuse;
                           3: each XCD owns a block of x-values and z-rows,
                           N1/ax x N3/az with ax*az = 8, chosen for the
                           fewest halo links (1/x-extent + 1/z-extent),

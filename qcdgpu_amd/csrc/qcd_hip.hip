@@ -78,26 +78,34 @@ struct UpdArgs {
     // ReTr(U' * sum_{nu<mu} S_nu); modes 1, 2, 3 = even Y, Z, T half-steps.
     double* partials;
     int meas_mode;
-    int xcd_map;          // 0: hardware order, 1: one x-slab per XCD, >= 2: blocks of (x, z) per XCD
-    // xcd_map >= 2: z-groups of the lattice, N4, x-values per XCD block,
-    // XCD blocks along x, z-groups per XCD block
-    uint32_t ord_ng, ord_nt, ord_xs, ord_ax, ord_zr;
+    int xcd_map;          // 0: hardware order, 1: one x-slab per XCD, 2, 3: blocks of (x, z) per XCD
+    // The unit of a workgroup (block_unit): z-groups of the lattice, N4,
+    // x-values per XCD block, XCD blocks along x and z-groups dispatched
+    // together (as powers of two), z-groups per XCD block; the divisors come
+    // with their multipliers.  dispatch_order gives the values of every map.
+    uint32_t ord_ng, ord_ax_log, ord_zb_log, ord_zr;
+    FastDiv ord_nt, ord_xs;
+    uint32_t nunits;      // 64-link units of the launch
     uint32_t unit0;       // first 64-link unit of the launch (an x-slab's first interior slice; else 0)
     Twist tw;             // twisted boundary (read only by the TW instantiations)
 };
 
 // 64-link unit handled by the l-th workgroup (or wavefront) dispatched to
-// XCD k, for xcd_map >= 2.  A unit is a group of rb = 64 / (N2 / 2) whole
-// z-rows, so unit u = zg + ng (t + N4 x).  XCD k = kx + ax kz owns the block
+// XCD k; hardware dispatches workgroup b to XCD b mod 8.  For xcd_map 2 and 3
+// a unit is a group of rb = 64 / (N2 / 2) whole z-rows, so unit
+// u = zg + ng (t + N4 x).  XCD k = kx + ax kz owns the block
 // x in [kx xs, (kx+1) xs), z-groups [kz zr, (kz+1) zr); within it the units
-// go x offset fastest, then t, then z-group, so a unit's x, t and z
-// neighbours are dispatched close to it.
+// go x offset fastest, then the zb z-groups of a z-block, then t, then
+// z-block, so a unit's x, z and t neighbours are dispatched close to it.
+// The other maps are the same expression with other values (dispatch_order),
+// so no workgroup branches on the map.
 __device__ __forceinline__ uint32_t block_unit(const UpdArgs& a, uint32_t k, uint32_t l)
 {
-    const uint32_t kx = k % a.ord_ax, kz = k / a.ord_ax;
-    const uint32_t c = l % a.ord_xs, r = l / a.ord_xs;
-    const uint32_t t = r % a.ord_nt, zl = r / a.ord_nt;
-    return kz * a.ord_zr + zl + a.ord_ng * (t + a.ord_nt * (kx * a.ord_xs + c));
+    const uint32_t kx = k & ((1u << a.ord_ax_log) - 1u), kz = k >> a.ord_ax_log;
+    const uint32_t r = a.ord_xs.div(l), c = l - r * a.ord_xs.d;
+    const uint32_t zi = r & ((1u << a.ord_zb_log) - 1u), r2 = r >> a.ord_zb_log;
+    const uint32_t zB = a.ord_nt.div(r2), t = r2 - zB * a.ord_nt.d;
+    return kz * a.ord_zr + (zB << a.ord_zb_log) + zi + a.ord_ng * (t + a.ord_nt.d * (kx * a.ord_xs.d + c));
 }
 
 // Hardware dispatches workgroup b to XCD (b mod 8).  Remap so that each XCD
@@ -541,20 +549,6 @@ __device__ __forceinline__ double update_link(const UpdArgs& a, const Table<R, N
     return trace;
 }
 
-// Workgroup -> 64-link block.  Mode 1: XCD k (hardware block b goes to XCD
-// b mod 8) gets the k-th contiguous eighth of the compact index range, an
-// x-slab of the lattice.  Modes 2 and 3: each XCD gets one block of x-values
-// and z-groups (block_unit; mode 2 the x-slabs of mode 1, mode 3 the block
-// shape with the fewest halo links), dispatched cross-section first.
-__device__ __forceinline__ uint32_t upd_block(const UpdArgs& a)
-{
-    const uint32_t b = blockIdx.x, nb = gridDim.x;
-    if (a.xcd_map == 0 || (nb % 8u)) return b;
-    const uint32_t per = nb / 8u, k = b % 8u, l = b / 8u;
-    if (a.xcd_map >= 2) return block_unit(a, k, l);
-    return k * per + l;
-}
-
 // Body of the three-wavefront update for 64-link unit `blk` of a lattice
 // with `nunits` units (the fused-plaquette partial of the unit goes to
 // partials[(meas_mode - 1) * nunits + blk]).
@@ -699,22 +693,22 @@ __device__ __forceinline__ void update3(const UpdArgs& a, uint32_t blk, uint32_t
 template <typename R, int N, int NREAL, bool OVER, int RK, bool MEAS, bool TW = false, int MU = -1>
 __global__ __launch_bounds__(kUpdThreads) void k_update(UpdArgs a)
 {
-    update3<R, N, NREAL, OVER, RK, MEAS, TW, MU>(a, upd_block(a), gridDim.x);
+    const uint32_t blk = block_unit(a, blockIdx.x & 7u, blockIdx.x >> 3);
+    if (blk >= a.nunits) return;   // whole workgroup: the grid is rounded up to the XCDs
+    update3<R, N, NREAL, OVER, RK, MEAS, TW, MU>(a, blk, a.nunits);
 }
 
 // One wavefront per 64 links: each wavefront gathers and sums the three
 // staple shares of its own links (one batch of gathers per direction) and
 // updates them; a workgroup is 4 independent wavefronts.  More links are in
 // flight per CU than with kUpdThreads workgroups, at the cost of a longer
-// path per wavefront.  The 64-link unit map is the same as upd_block's.
+// path per wavefront.  The 64-link unit map is k_update's.
 constexpr int kWaves1 = 4;
 __device__ __forceinline__ uint32_t upd_unit1(const UpdArgs& a, int w)
 {
     const uint32_t b = blockIdx.x, nb = gridDim.x;
     if (a.xcd_map == 0 || (nb % 8u)) return b * kWaves1 + (uint32_t)w;
-    const uint32_t per = nb * kWaves1 / 8u, k = b % 8u, l = (b / 8u) * kWaves1 + (uint32_t)w;
-    if (a.xcd_map >= 2) return block_unit(a, k, l);
-    return k * per + l;
+    return block_unit(a, b % 8u, (b / 8u) * kWaves1 + (uint32_t)w);
 }
 
 // Body of the one-wavefront update for 64-link unit `unit` of `units`.
@@ -1979,12 +1973,18 @@ uint32_t update_unit0(const qcd_lattice* L) { return L->slab ? L->g.vh / (uint32
 // 1 / z-extent) of the table for a block that is cut along both
 // (periodic full extents have no halo).  A mode that does not apply falls
 // back to mode 1 (and to 0 when shape1 needs whole workgroups of four
-// units per XCD and does not get them).
+// units per XCD and does not get them).  Mode 1 takes any number of units
+// (the XCDs' ranges differ by at most one); 20 x 12 x 28 x 10, 525 units,
+// against hardware order: FP64 overrelaxation half-step 16.7 -> 11.4 us,
+// heatbath 23.3 -> 18.0 us, 12-real FP32 8.5 -> 7.7 and 10.7 -> 10.0 us.
 void dispatch_order(const qcd_lattice* L, int want, bool shape1, UpdArgs& a)
 {
     if (L->slab && want > 1) want = 1;   // the block orders cover the whole lattice
     a.xcd_map = want;
-    a.ord_ng = a.ord_nt = a.ord_xs = a.ord_ax = a.ord_zr = 1;
+    a.nunits = update_units(L);
+    a.ord_ng = a.ord_zr = 1;
+    a.ord_ax_log = a.ord_zb_log = 0;
+    a.ord_nt = a.ord_xs = make_fastdiv(1);
     if (want >= 2) {
         const uint32_t h = (uint32_t)L->g.h, nb = L->g.vh / kLinks;
         const uint32_t rb = (h <= kLinks && kLinks % h == 0) ? kLinks / h : 0;
@@ -2006,26 +2006,55 @@ void dispatch_order(const qcd_lattice* L, int want, bool shape1, UpdArgs& a)
             ok = bax != 0;
             if (ok) {
                 a.ord_ng = ng;
-                a.ord_nt = (uint32_t)L->g.n4;
-                a.ord_ax = bax;
-                a.ord_xs = n1 / bax;
+                a.ord_nt = make_fastdiv((uint32_t)L->g.n4);
+                a.ord_ax_log = bax == 8 ? 3 : (bax == 4 ? 2 : bax - 1);
+                a.ord_xs = make_fastdiv(n1 / bax);
                 a.ord_zr = ng / (8 / bax);
+                // With one or two z-rows per unit and more than 256 units (what
+                // an XCD has in flight) from one z-group to the next, the z
+                // neighbours have left the XCD's L2 by then: four z-groups go
+                // together.  64^4 FP32: overrelaxation half-step 1334 -> 1253
+                // us, heatbath 1438 -> 1331 us; FP64 2845 -> 2563 and 2931 ->
+                // 2644 us.  Elsewhere it costs: 144 units apart (48 x 64 x 48
+                // x 24) 260 -> 262 us, four rows per unit (64 x 32 x 64 x 64)
+                // 584 -> 601 us.
+                if (rb <= 2 && a.ord_xs.d * a.ord_nt.d > 256 && a.ord_zr % 4 == 0) a.ord_zb_log = 2;
             }
         }
         if (!ok) a.xcd_map = 1;
     }
     if (shape1 && a.xcd_map != 0) {
         // four 64-link units per workgroup: the XCD blocks need whole workgroups
-        if (update_units(L) % (8u * kWaves1)) a.xcd_map = 0;
+        if (a.nunits % (8u * kWaves1)) a.xcd_map = 0;
+    }
+    if (a.xcd_map == 0) {   // unit 8 l + k: hardware order
+        a.ord_ng = 8;
+        a.ord_zr = 1;
+        a.ord_ax_log = 0;
+        a.ord_nt = make_fastdiv(0x7fffffffu);
+    } else if (a.xcd_map == 1) {   // unit l + k nt
+        a.ord_ax_log = 3;
+        a.ord_nt = make_fastdiv(align_up(a.nunits, 8) / 8u);
+        const uint32_t per_x = L->g.vh / (uint32_t)L->g.n1;
+        if (!shape1 && !L->slab && L->g.n1 % 8 == 0 && per_x % kLinks == 0) {
+            // whole units per x-value: the XCD's x-values side by side
+            // (24^3 x 12 FP64 overrelaxation half-step 26.4 -> 25.4 us)
+            a.ord_xs = make_fastdiv((uint32_t)L->g.n1 / 8u);
+            a.ord_nt = make_fastdiv(per_x / kLinks);
+        }
     }
 }
+
+// Workgroups of one update launch (three-wavefront shape).
+uint32_t update_grid(const UpdArgs& a) { return a.xcd_map ? align_up(a.nunits, 8) : a.nunits; }
 
 template <typename R, int N, int NREAL, bool OVER, int RK>
 void launch_update_t(qcd_lattice* L, const UpdArgs& a, const LaunchOpt& o)
 {
-    const uint32_t nb = update_units(L);   // 64-link units
+    const uint32_t nb = a.nunits;   // 64-link units
+    const dim3 grid3(update_grid(a)), block3(kUpdThreads);
     if (a.tw.on) {   // twisted boundary: three-wavefront shape, plaquette never fused
-        launch(k_update<R, N, NREAL, OVER, RK, false, true>, dim3(nb), dim3(kUpdThreads), L->stream, o, a);
+        launch(k_update<R, N, NREAL, OVER, RK, false, true>, grid3, block3, L->stream, o, a);
         return;
     }
     if (L->tune_update_shape == 1) {
@@ -2037,16 +2066,15 @@ void launch_update_t(qcd_lattice* L, const UpdArgs& a, const LaunchOpt& o)
         return;
     }
     if (o.meas_mode) {
-        launch(k_update<R, N, NREAL, OVER, RK, true>, dim3(nb), dim3(kUpdThreads), L->stream, o, a);
+        launch(k_update<R, N, NREAL, OVER, RK, true>, grid3, block3, L->stream, o, a);
         return;
     }
     // the plain half-steps, most launches of a cycle: one instance per direction
-    const dim3 grid(nb), block(kUpdThreads);
     switch (a.mu) {
-        case 0: launch(k_update<R, N, NREAL, OVER, RK, false, false, 0>, grid, block, L->stream, o, a); break;
-        case 1: launch(k_update<R, N, NREAL, OVER, RK, false, false, 1>, grid, block, L->stream, o, a); break;
-        case 2: launch(k_update<R, N, NREAL, OVER, RK, false, false, 2>, grid, block, L->stream, o, a); break;
-        default: launch(k_update<R, N, NREAL, OVER, RK, false, false, 3>, grid, block, L->stream, o, a); break;
+        case 0: launch(k_update<R, N, NREAL, OVER, RK, false, false, 0>, grid3, block3, L->stream, o, a); break;
+        case 1: launch(k_update<R, N, NREAL, OVER, RK, false, false, 1>, grid3, block3, L->stream, o, a); break;
+        case 2: launch(k_update<R, N, NREAL, OVER, RK, false, false, 2>, grid3, block3, L->stream, o, a); break;
+        default: launch(k_update<R, N, NREAL, OVER, RK, false, false, 3>, grid3, block3, L->stream, o, a); break;
     }
 }
 
@@ -2963,7 +2991,7 @@ int qcd_lattice_get_tune(const qcd_lattice* L, int knob, int* value, int* detail
             dispatch_order(L, L->tune_xcd_map, L->tune_update_shape == 1 && !L->tw.on, a);
             *value = a.xcd_map;
             if (detail) {   // XCD block: x-values, z-rows (modes 2 and 3)
-                detail[0] = a.xcd_map >= 2 ? (int)a.ord_xs : 0;
+                detail[0] = a.xcd_map >= 2 ? (int)a.ord_xs.d : 0;
                 detail[1] = a.xcd_map >= 2 ? (int)(a.ord_zr * ((uint32_t)L->g.n3 / a.ord_ng)) : 0;
             }
             break;
@@ -4144,7 +4172,10 @@ UpdArgs chain_base_args(const qcd_lattice* L)
     a.s_quads = (L->p.stream_mode == QCD_STREAM_REFERENCE) ? L->s_quads : 0u;
     a.partials = L->part_fused;
     a.xcd_map = 0;
-    a.ord_ng = a.ord_nt = a.ord_xs = a.ord_ax = a.ord_zr = 1;
+    a.ord_ng = a.ord_zr = 1;
+    a.ord_ax_log = a.ord_zb_log = 0;
+    a.ord_nt = a.ord_xs = make_fastdiv(1);
+    a.nunits = L->nb_fused;
     a.jump = L->jump_cols;
     a.pm_ak = L->pm_ak;
     a.prn = L->prn_buf;
