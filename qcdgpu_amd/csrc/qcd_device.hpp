@@ -160,9 +160,9 @@ template <typename R, int N> __device__ __forceinline__ void m_acc_dn(M<R, N>& a
 // matrices is in SU(3), so its third row is conj(row 1 x row 2).
 // F = f1 f2^+ f3^+: rows 0, 1 of f1 f2^+, then rows 0, 1 of that times f3^+.
 template <typename R>
-__device__ __forceinline__ M<R, 3> su3_fwd_term(const M<R, 3>& f1, const M<R, 3>& f2, const M<R, 3>& f3)
+__device__ __forceinline__ M<R, 3> su3_fwd_half(const M<R, 3>& f1, const M<R, 3>& f2)
 {
-    M<R, 3> t, F;
+    M<R, 3> t;
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
@@ -172,6 +172,12 @@ __device__ __forceinline__ M<R, 3> su3_fwd_term(const M<R, 3>& f1, const M<R, 3>
             cfmac(s, f1.e[i][2], f2.e[j][2]);
             t.e[i][j] = s;
         }
+    return t;
+}
+template <typename R>
+__device__ __forceinline__ M<R, 3> su3_fwd_rest(const M<R, 3>& t, const M<R, 3>& f3)
+{
+    M<R, 3> F;
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
@@ -181,8 +187,27 @@ __device__ __forceinline__ M<R, 3> su3_fwd_term(const M<R, 3>& f1, const M<R, 3>
             cfmac(s, t.e[i][2], f3.e[j][2]);
             F.e[i][j] = s;
         }
+    return F;
+}
+template <typename R>
+__device__ __forceinline__ M<R, 3> su3_fwd_term(const M<R, 3>& f1, const M<R, 3>& f2, const M<R, 3>& f3)
+{
+    M<R, 3> F = su3_fwd_rest(su3_fwd_half(f1, f2), f3);
     su3_row3(F);
     return F;
+}
+// Rows 0 and 1 are computed here and no later load is issued before them.
+template <typename R> __device__ __forceinline__ void pin_rows(M<R, 3>& a)
+{
+    asm volatile("" : "+v"(a.e[0][0].re), "+v"(a.e[0][0].im), "+v"(a.e[0][1].re), "+v"(a.e[0][1].im), "+v"(a.e[0][2].re),
+                 "+v"(a.e[0][2].im), "+v"(a.e[1][0].re), "+v"(a.e[1][0].im), "+v"(a.e[1][1].re), "+v"(a.e[1][1].im),
+                 "+v"(a.e[1][2].re), "+v"(a.e[1][2].im)::"memory");
+}
+template <typename R> __device__ __forceinline__ void pin(M<R, 3>& a)
+{
+    pin_rows(a);
+    asm volatile("" : "+v"(a.e[2][0].re), "+v"(a.e[2][0].im), "+v"(a.e[2][1].re), "+v"(a.e[2][1].im), "+v"(a.e[2][2].re),
+                 "+v"(a.e[2][2].im)::"memory");
 }
 // B = (b1 b2)^+ b3: columns 0, 1 of b1 b2 are rows 0, 1 of (b1 b2)^+.
 template <typename R>
@@ -428,40 +453,47 @@ __host__ __device__ __forceinline__ Site site_of(const Geom& g, uint32_t i, int 
     return s;
 }
 
-// Neighbour steps along a wavefront-uniform direction d (so every select on
-// d is scalar).  c = the site's coordinate along d, o = y & 1 of the site,
-// i = its compact index.  x, z and t steps move the compact index by the
-// direction's stride (wrapping at the boundary); a y step keeps or moves the
-// half-row index depending on o.  A step along one direction leaves the
-// coordinate along any other direction unchanged, and changes o only when
-// it is a y step, so two-step neighbours chain two calls with the original
-// c and o (the second direction is never y when the first one is).
+// Neighbour steps along a wavefront-uniform direction d, without a branch on
+// it (the direction only selects scalars; as branches the steps of a staple
+// were some 150 dependent scalar instructions in front of its first load).
+// c = the site's coordinate along d, o = y & 1 of the site, i = its compact
+// index.  x, z and t steps move the compact index by the direction's stride
+// (wrapping at the boundary); a y step keeps or moves the half-row index
+// depending on o.  A step along one direction leaves the coordinate along any
+// other direction unchanged, and changes o only when it is a y step, so
+// two-step neighbours chain two calls with the original c and o (the second
+// direction is never y when the first one is).
 __host__ __device__ __forceinline__ int coord(const Site& s, int d)
 {
-    return d == 0 ? s.x : (d == 1 ? s.y : (d == 2 ? s.z : s.t));
+    const int xy = d == 0 ? s.x : s.y, zt = d == 2 ? s.z : s.t;
+    return d < 2 ? xy : zt;
 }
-__host__ __device__ __forceinline__ uint32_t cstride(const Geom& g, int d)
+struct Step {
+    int last;            // extent - 1
+    bool y;
+    uint32_t st, wrap;   // compact stride (y: unused) and the distance across the boundary
+};
+__host__ __device__ __forceinline__ Step step_of(const Geom& g, int d)
 {
-    return d == 0 ? (uint32_t)g.h * (uint32_t)g.n3 * (uint32_t)g.n4
-                  : (d == 2 ? (uint32_t)g.h : (uint32_t)g.h * (uint32_t)g.n3);
+    const uint32_t h = (uint32_t)g.h, hz = h * (uint32_t)g.n3, hzt = hz * (uint32_t)g.n4;
+    const int nxy = d == 0 ? g.n1 : g.n2, nzt = d == 2 ? g.n3 : g.n4;
+    const uint32_t szt = d == 2 ? h : hz;
+    Step s;
+    s.last = (d < 2 ? nxy : nzt) - 1;
+    s.y = d == 1;
+    s.st = d == 0 ? hzt : szt;
+    s.wrap = s.y ? h - 1u : s.st * (uint32_t)s.last;
+    return s;
 }
-__host__ __device__ __forceinline__ int extent(const Geom& g, int d)
+__host__ __device__ __forceinline__ uint32_t step_fwd(const Step& s, uint32_t i, int c, uint32_t o)
 {
-    return d == 0 ? g.n1 : (d == 1 ? g.n2 : (d == 2 ? g.n3 : g.n4));
+    const uint32_t in = s.y ? o : s.st;
+    return i + (c < s.last ? in : 0u - s.wrap);
 }
-__host__ __device__ __forceinline__ uint32_t step_fwd(const Geom& g, uint32_t i, int d, int c, uint32_t o)
+__host__ __device__ __forceinline__ uint32_t step_bwd(const Step& s, uint32_t i, int c, uint32_t o)
 {
-    const int n = extent(g, d);
-    if (d == 1) return (c < n - 1) ? i + o : i - (uint32_t)(g.h - 1);
-    const uint32_t st = cstride(g, d);
-    return (c < n - 1) ? i + st : i - st * (uint32_t)(n - 1);
-}
-__host__ __device__ __forceinline__ uint32_t step_bwd(const Geom& g, uint32_t i, int d, int c, uint32_t o)
-{
-    const int n = extent(g, d);
-    if (d == 1) return (c > 0) ? i - (1u - o) : i + (uint32_t)(g.h - 1);
-    const uint32_t st = cstride(g, d);
-    return (c > 0) ? i - st : i + st * (uint32_t)(n - 1);
+    const uint32_t in = s.y ? o - 1u : 0u - s.st;
+    return i + (c > 0 ? in : s.wrap);
 }
 
 __host__ __device__ __forceinline__ uint32_t cindex(const Geom& g, int x, int y, int z, int t)
@@ -511,18 +543,22 @@ template <typename R, int N, int NREAL> struct Table {
     // SGPRs as an opaque value and selects the global_load saddr form
     // (scalar base + 32-bit lane offset) instead of a 64-bit add per load.
     using gchar = __attribute__((address_space(1))) char;
-    __device__ __forceinline__ static gchar* sbase(const V2* pl)
+    __device__ __forceinline__ static uint64_t scalar(uint64_t b)
     {
-        const uint64_t b = (uint64_t)pl;
         const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)b);
         const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(b >> 32));
-        return (gchar*)(((uint64_t)hi << 32) | lo);
+        return ((uint64_t)hi << 32) | lo;
     }
-    __device__ __forceinline__ V2 ld(const V2* pl, uint32_t i) const
+    // Address of (p, mu)'s first plane; the next plane is one stride further,
+    // so a matrix's planes are walked with one 64-bit scalar add each (a
+    // product per plane made 340 scalar instructions of an update's 54).
+    __device__ __forceinline__ uint64_t first(int p, int mu) const { return scalar((uint64_t)plane(p, mu, 0)); }
+    __device__ __forceinline__ uint64_t next(uint64_t b) const { return scalar(b + (uint64_t)vh_pad * sizeof(V2)); }
+    __device__ __forceinline__ static V2 ld(uint64_t b, uint32_t i)
     {
         using gR = __attribute__((address_space(1))) const R;
         const uint32_t off = i * (uint32_t)sizeof(V2);
-        const gR* q = (const gR*)(sbase(pl) + off);
+        const gR* q = (const gR*)((gchar*)b + off);
         V2 v;
         v.x = q[0];
         v.y = q[1];
@@ -536,16 +572,24 @@ template <typename R, int N, int NREAL> struct Table {
     __device__ __forceinline__ M<R, N> load_t(int p, int mu, uint32_t i) const
     {
         M<R, N> a;
-        if constexpr (N == 3) {
+        V2 v[NP];
+        if constexpr (UNIFORM) {
+            uint64_t b = first(p, mu);
 #pragma unroll
             for (int k = 0; k < NP; ++k) {
-                V2 v = UNIFORM ? ld(plane(p, mu, k), i) : ld_any(plane(p, mu, k), i);
-                a.e[k / 3][k % 3] = {v.x, v.y};
+                v[k] = ld(b, i);
+                if (k + 1 < NP) b = next(b);
             }
+        } else {
+#pragma unroll
+            for (int k = 0; k < NP; ++k) v[k] = ld_any(plane(p, mu, k), i);
+        }
+        if constexpr (N == 3) {
+#pragma unroll
+            for (int k = 0; k < NP; ++k) a.e[k / 3][k % 3] = {v[k].x, v[k].y};
             if constexpr (NP == 6) su3_row3(a);
         } else {
-            V2 v0 = UNIFORM ? ld(plane(p, mu, 0), i) : ld_any(plane(p, mu, 0), i);
-            V2 v1 = UNIFORM ? ld(plane(p, mu, 1), i) : ld_any(plane(p, mu, 1), i);
+            const V2 v0 = v[0], v1 = v[1];
             a.e[0][0] = {v0.x, v0.y};
             a.e[0][1] = {v1.x, v1.y};
             a.e[1][0] = {-v1.x, v1.y};
@@ -560,10 +604,12 @@ template <typename R, int N, int NREAL> struct Table {
     {
         M<R, N> a;
         if constexpr (N == 3) {
+            uint64_t b = first(p, mu);
 #pragma unroll
             for (int k = 0; k < NP; ++k) {
-                V2 v = ld(plane(p, mu, k), i);
+                V2 v = ld(b, i);
                 a.e[k / 3][k % 3] = {v.x, v.y};
+                if (k + 1 < NP) b = next(b);
             }
         } else {
             a = load_t<true>(p, mu, i);
@@ -584,15 +630,17 @@ template <typename R, int N, int NREAL> struct Table {
     __device__ __forceinline__ void store_u(int p, int mu, uint32_t i, const M<R, N>& a) const
     {
         const uint32_t off = i * (uint32_t)sizeof(V2);
+        uint64_t b = first(p, mu);
 #pragma unroll
         for (int k = 0; k < NP; ++k) {
             V2 v;
             v.x = a.e[k / N][k % N].re;
             v.y = a.e[k / N][k % N].im;
             using gRw = __attribute__((address_space(1))) R;
-            gRw* q = (gRw*)(sbase(plane(p, mu, k)) + off);
+            gRw* q = (gRw*)((gchar*)b + off);
             q[0] = v.x;
             q[1] = v.y;
+            if (k + 1 < NP) b = next(b);
         }
     }
 };

@@ -329,18 +329,43 @@ __device__ __forceinline__ M<R, N> staple_nu(const Table<R, N, NREAL>& T, const 
 {
     using Tab = Table<R, N, NREAL>;
     const int q = p ^ 1;
-    // The six gathers go out as two batches of three (forward, backward
-    // term): three matrices in flight per wavefront keep the register count
-    // low enough for six to eight wavefronts per SIMD, which hides more
-    // latency than a single batch of six at four wavefronts per SIMD.
+    // The gathers are spread so that the register count stays low enough for
+    // six to eight wavefronts per SIMD, which hides more latency than all six
+    // matrices in flight at four wavefronts per SIMD.
     const int cmu = coord(s, mu), cnu = coord(s, nu);
     const uint32_t o = (uint32_t)s.y & 1u;
-    const uint32_t i_pmu = step_fwd(g, i, mu, cmu, o);
-    const uint32_t i_pnu = step_fwd(g, i, nu, cnu, o);
-    const uint32_t i_mnu = step_bwd(g, i, nu, cnu, o);
-    const uint32_t i_pmu_mnu = step_bwd(g, i_pmu, nu, cnu, o);
+    const Step smu = step_of(g, mu), snu = step_of(g, nu);
+    const uint32_t i_pmu = step_fwd(smu, i, cmu, o);
+    const uint32_t i_pnu = step_fwd(snu, i, cnu, o);
+    const uint32_t i_mnu = step_bwd(snu, i, cnu, o);
+    const uint32_t i_pmu_mnu = step_bwd(snu, i_pmu, cnu, o);
     M<R, N> S;
-    if constexpr (N == 3 && NREAL == 18 && sizeof(R) == 4) {
+    if constexpr (N == 3 && NREAL == 12 && sizeof(R) == 4 && !TW) {
+        // FP32, 12 reals: each product is formed before the gathers that
+        // follow it are issued, 64 VGPRs (32^3 x 8 overrelaxation 14.1 ->
+        // 13.5 us, heatbath 19.0 -> 17.5 us against two batches of three).
+        M<R, N> f2 = T.load_raw_u(q, mu, i_pnu);
+        M<R, N> f1 = T.load_raw_u(q, nu, i_pmu);
+        M<R, N> f3 = T.load_raw_u(p, nu, i);
+        Tab::finish(f2);
+        M<R, 3> t = su3_fwd_half(f1, f2);
+        pin_rows(t);
+        M<R, N> b1 = T.load_raw_u(q, mu, i_mnu);
+        M<R, N> b2 = T.load_raw_u(p, nu, i_pmu_mnu);
+        Tab::finish(f3);
+        M<R, 3> F = su3_fwd_rest(t, f3);
+        pin_rows(F);
+        M<R, N> b3 = T.load_raw_u(q, nu, i_mnu);
+        Tab::finish(b1);
+        Tab::finish(b2);
+        Tab::finish(b3);
+        su3_row3(F);
+        const M<R, 3> B = su3_bwd_term(b1, b2, b3);
+#pragma unroll
+        for (int r = 0; r < 3; ++r)
+#pragma unroll
+            for (int c = 0; c < 3; ++c) S.e[r][c] = cadd(F.e[r][c], B.e[r][c]);
+    } else if constexpr (N == 3 && NREAL == 18 && sizeof(R) == 4) {
         // FP32, 18 reals: the forward and then the backward three gathers as
         // two batches, scheduled freely (the peak holds three matrices in
         // flight, 78 VGPRs: six wavefronts per SIMD instead of four).
@@ -568,7 +593,11 @@ __device__ __forceinline__ void update3(const UpdArgs& a, uint32_t blk, uint32_t
     const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int lane = threadIdx.x & 63;
     const uint32_t i = (a.unit0 + blk) * kLinks + lane;
-    const bool active = i < a.g.vh;
+    // The grid is rounded up to the XCDs: a workgroup past the last unit runs
+    // through with no active lane (a return here would put a second round of
+    // argument loads behind the unit's arithmetic).
+    const bool live = blk < nunits;
+    const bool active = live && i < a.g.vh;
     Table<R, N, NREAL> Tb{(typename Vec2<R>::T*)a.table, a.g.vh_pad};
     const Table<R, N, NREAL> Ts{(typename Vec2<R>::T*)a.src, a.g.vh_pad};
     const int p = a.parity, mu = (MU >= 0) ? MU : a.mu;
@@ -585,7 +614,7 @@ __device__ __forceinline__ void update3(const UpdArgs& a, uint32_t blk, uint32_t
     constexpr bool kStream = (RK == RK_XOR128 || RK == RK_PM);
     uint4 rs = make_uint4(0, 0, 0, 0);
     if constexpr (kStream) {
-        if ((w == 0 && active) || (w > 0 && a.s_quads)) rs = a.rng[i];
+        if ((w == 0 && active) || (w > 0 && live && a.s_quads)) rs = a.rng[i];
     }
     // XOR128 jump table (8 KiB) staged in LDS by the whole workgroup with
     // direct global -> LDS loads (global_load_lds_dwordx4: lane l of a
@@ -602,9 +631,15 @@ __device__ __forceinline__ void update3(const UpdArgs& a, uint32_t blk, uint32_t
                                                  (__attribute__((address_space(3))) void*)&jtab[c * 64], 16, 0, 0);
         }
     }
-    M<R, N> S;
-    if (active) S = staple_nu<R, N, NREAL, TW>(Ts, a.g, s, i, p, mu, nu, a.tw);
-    else m_zero(S);
+    // a lane past the last link gathers link 0's neighbours, unused
+    M<R, N> S = staple_nu<R, N, NREAL, TW>(Ts, a.g, s, active ? i : 0u, p, mu, nu, a.tw);
+    // The share is complete here: without this the compiler puts the link's
+    // load and all gathers in flight ahead of the products, 126 VGPRs instead
+    // of 78, and 2048 workgroups no longer fit the chip at once (32^3 x 8
+    // FP32: overrelaxation 17.9 us, 16.9 with it; heatbath 21.0 and 20.1).
+    // FP64 overrelaxation has too few wavefronts either way and gains from
+    // the loads in flight (24^3 x 12: 24.9 us with it, 22.7 without).
+    if constexpr (N == 3 && !(OVER && sizeof(R) == 8)) pin(S);
     // Wavefront 0 issues the load of the link it updates before the
     // barrier, so its latency overlaps the wait for the other shares rather
     // than following it.
@@ -623,7 +658,7 @@ __device__ __forceinline__ void update3(const UpdArgs& a, uint32_t blk, uint32_t
     __syncthreads();
     if (w > 0) {
         if constexpr (kStream) {
-            if (a.s_quads) {
+            if (a.s_quads && live) {
                 const int half = w - 1;
                 uint2 o;
                 if constexpr (RK == RK_XOR128) {
@@ -686,16 +721,14 @@ __device__ __forceinline__ void update3(const UpdArgs& a, uint32_t blk, uint32_t
         trace = wave_sum(trace);
         // slot = 64-link unit, so the final sum runs in lattice order
         // whatever the launch order or kernel shape
-        if (lane == 0) a.partials[(size_t)(a.meas_mode - 1) * nunits + blk] = trace;
+        if (lane == 0 && live) a.partials[(size_t)(a.meas_mode - 1) * nunits + blk] = trace;
     }
 }
 
 template <typename R, int N, int NREAL, bool OVER, int RK, bool MEAS, bool TW = false, int MU = -1>
 __global__ __launch_bounds__(kUpdThreads) void k_update(UpdArgs a)
 {
-    const uint32_t blk = block_unit(a, blockIdx.x & 7u, blockIdx.x >> 3);
-    if (blk >= a.nunits) return;   // whole workgroup: the grid is rounded up to the XCDs
-    update3<R, N, NREAL, OVER, RK, MEAS, TW, MU>(a, blk, a.nunits);
+    update3<R, N, NREAL, OVER, RK, MEAS, TW, MU>(a, block_unit(a, blockIdx.x & 7u, blockIdx.x >> 3), a.nunits);
 }
 
 // One wavefront per 64 links: each wavefront gathers and sums the three
