@@ -41,6 +41,7 @@
 #include "../../include/qcd_hip.h"
 #include "qcd_device.hpp"
 #include "qcd_internal.h"
+#include "qcd_ranlux.hpp"
 
 using namespace qcd;
 
@@ -922,8 +923,27 @@ __global__ __launch_bounds__(kBlock) void k_ranlux_produce(float4* state, uint32
     ranlux_body<LUX>(state, n, samples, quads, g);
 }
 
-void launch_ranlux_produce(int lux, float4* state, uint32_t n, uint32_t samples, float4* quads, hipStream_t st)
+// The same produce() with the blocks in parallel (qcd_ranlux.hpp): one
+// workgroup of W wavefronts per 64 streams.
+__global__ __launch_bounds__(kRlWaves * 64) void k_ranlux_jump(float4* state, uint32_t n, uint32_t samples, uint32_t keep,
+                                                               float4* quads, const uint4* tab)
 {
+    extern __shared__ uint32_t rl_lds[];
+    rl_produce(state, n, samples, keep, quads, blockIdx.x, tab, rl_lds, blockDim.x / 64u);
+}
+
+// produce() of `samples` quads per stream; the first `keep` go to `quads`
+// (null: none).  tab: the lattice's jump tables.
+void launch_ranlux_produce(int lux, float4* state, uint32_t n, uint32_t samples, uint32_t keep, float4* quads,
+                           const uint4* tab, hipStream_t st)
+{
+    if (!quads) keep = 0;
+    const uint32_t W = rl_waves(lux, samples, keep, n);
+    if (W) {
+        hipLaunchKernelGGL(k_ranlux_jump, dim3((n + 63u) / 64u), dim3(64u * W), rl_lds_bytes(W), st, state, n, samples,
+                           keep, quads, tab);
+        return;
+    }
     const uint32_t nb = (n + kBlock - 1) / kBlock;
     switch (lux) {
         case 0: hipLaunchKernelGGL(k_ranlux_produce<0>, dim3(nb), dim3(kBlock), 0, st, state, n, samples, quads); break;
@@ -932,6 +952,17 @@ void launch_ranlux_produce(int lux, float4* state, uint32_t n, uint32_t samples,
         case 3: hipLaunchKernelGGL(k_ranlux_produce<3>, dim3(nb), dim3(kBlock), 0, st, state, n, samples, quads); break;
         default: hipLaunchKernelGGL(k_ranlux_produce<4>, dim3(nb), dim3(kBlock), 0, st, state, n, samples, quads); break;
     }
+}
+
+// Device copy of the jump tables of one luxury level (96 kB).
+bool alloc_rl_tables(int lux, uint4** tab)
+{
+    const std::vector<uint32_t>& h = rl_tables(lux >= 0 && lux < 4 ? lux : 4);   // as the kernels take it
+    if (hipMalloc((void**)tab, sizeof(uint32_t) * h.size()) != hipSuccess) {
+        *tab = nullptr;
+        return false;
+    }
+    return hipMemcpy(*tab, h.data(), sizeof(uint32_t) * h.size(), hipMemcpyHostToDevice) == hipSuccess;
 }
 
 // Host seeding of the RANLUX table as PRNG::initialize / RL_initialize
@@ -1747,7 +1778,19 @@ __global__ __launch_bounds__(kWaves1 * kLinks) void k_update_batch1(const ChainD
     update1<R, N, NREAL, OVER, RK, MEAS>(a, u, cd[c].nunits);
 }
 
-// RANLUX produce for every chain: one wavefront-sized workgroup per unit.
+// RANLUX produce for every chain, one workgroup per unit: W wavefronts with
+// the blocks in parallel, or one wavefront stepping through them.
+__global__ __launch_bounds__(kRlWaves * 64) void k_ranlux_jump_batch(const ChainDesc* cd, const uint2* map,
+                                                                     uint32_t samples, uint32_t keep, const uint4* tab)
+{
+    extern __shared__ uint32_t rl_lds[];
+    const uint32_t c = __builtin_amdgcn_readfirstlane(map[blockIdx.x].x);
+    const uint32_t u = __builtin_amdgcn_readfirstlane(map[blockIdx.x].y);
+    if (c == ~0u) return;
+    rl_produce(cd[c].rl_state, cd[c].nunits * kLinks, samples, keep, const_cast<float4*>(cd[c].a.prn), u, tab, rl_lds,
+               blockDim.x / 64u);
+}
+
 template <int LUX>
 __global__ __launch_bounds__(kLinks) void k_ranlux_produce_batch(const ChainDesc* cd, const uint2* map, uint32_t samples)
 {
@@ -1795,6 +1838,7 @@ struct qcd_lattice {
     uint4* rng_buf[2] = {nullptr, nullptr};   // generator states; rng_buf[rng_cur] is current
     uint4* jump_cols = nullptr;               // XOR128 jump-ahead matrix: 128 columns, then the 4-bit table
     float4* rl_state = nullptr;               // RANLUX: 7 float4 per stream
+    uint4* rl_tab = nullptr;                  // RANLUX: jump tables of its luxury level
     float4* prn_buf = nullptr;                // RANLUX: produced quads, prn_quads per stream
     uint32_t prn_quads = 0;
     uint32_t pm_ak = 1;                       // Park-Miller jump multiplier
@@ -2111,14 +2155,26 @@ void launch_update_t(qcd_lattice* L, const UpdArgs& a, const LaunchOpt& o)
     }
 }
 
+// Quads per instance a heatbath half-step can read: a link's SU(2) updates
+// take at most NHIT tries and one more each (kp_update), quad k of link i
+// being quad i + k PRNGSTEP of the buffer.  The reference sizes every
+// produce() for three of them, also SU(2)'s.
+uint32_t update_quads(const qcd_lattice* L)
+{
+    const uint64_t k = (uint64_t)(L->p.sun == 3 ? 3 : 1) * (uint64_t)(L->p.nhit + 1);
+    const uint64_t per = (k * L->n_streams + L->n_inst - 1) / L->n_inst;
+    return (uint32_t)std::min<uint64_t>(per, L->s_quads);
+}
+
 // One produce() of `samples` quads per generator instance into `out` (quad
 // q = sample * n_inst + instance), or a skip of as many when out is null;
-// XOR128 / PM states advance in place in the current state buffer.
-void produce_quads_into(qcd_lattice* L, uint32_t samples, float4* out)
+// XOR128 / PM states advance in place in the current state buffer.  RANLUX may
+// leave out the quads from `keep` on.
+void produce_quads_into(qcd_lattice* L, uint32_t samples, uint32_t keep, float4* out)
 {
     const uint32_t n = L->n_inst, nb = align_up(n, kBlock) / kBlock;
     if (L->p.prng == QCD_PRNG_RANLUX) {
-        launch_ranlux_produce(L->p.ranlux_luxury, L->rl_state, n, samples, out, L->stream);
+        launch_ranlux_produce(L->p.ranlux_luxury, L->rl_state, n, samples, keep, out, L->rl_tab, L->stream);
     } else if (L->p.prng == QCD_PRNG_XOR128) {
         if (out)
             hipLaunchKernelGGL(k_xor128_produce, dim3(nb), dim3(kBlock), 0, L->stream, L->rng_buf[L->rng_cur], n,
@@ -2182,7 +2238,7 @@ int launch_update_rn(qcd_lattice* L, int parity, int mu, int kind, int start_gid
             // reads quad k of link i at k * PRNGSTEP + i
             {
                 ProfScope ps(L, "PRNG produce");
-                produce_quads_into(L, L->s_quads, L->prn_buf);
+                produce_quads_into(L, L->s_quads, update_quads(L), L->prn_buf);
             }
             a.prn = L->prn_buf;
             a.prn_stride = L->n_streams;
@@ -2273,7 +2329,7 @@ int launch_simple(qcd_lattice* L, int which, const LaunchOpt& o)
                                    L->g, L->rng_buf[L->rng_cur], (const float4*)nullptr, 0u);
             } else if (L->p.prng == QCD_PRNG_RANLUX) {
                 const uint32_t q = (N == 3) ? 24u : 8u;   // 8 links x 3 or 1 quads
-                launch_ranlux_produce(L->p.ranlux_luxury, L->rl_state, L->n_streams, q, L->prn_buf, L->stream);
+                launch_ranlux_produce(L->p.ranlux_luxury, L->rl_state, L->n_streams, q, q, L->prn_buf, L->rl_tab, L->stream);
                 hipLaunchKernelGGL((k_init_hot<R, N, NREAL, RK_BUF>), dim3(nb), dim3(kBlock), 0, L->stream, L->table,
                                    L->g, (uint4*)nullptr, (const float4*)L->prn_buf, L->n_streams);
             } else {
@@ -2583,7 +2639,8 @@ int qcd_lattice_create(const qcd_params* pp, qcd_lattice** out)
         // PRNGSTEP instances, per Haar start (8 links x 3 quads for SU(3)).
         L->prn_quads = L->s_quads > 24u ? L->s_quads : 24u;
         if ((p.prng == QCD_PRNG_RANLUX &&
-             hipMalloc((void**)&L->rl_state, sizeof(float4) * 7 * L->n_inst) != hipSuccess) ||
+             (hipMalloc((void**)&L->rl_state, sizeof(float4) * 7 * L->n_inst) != hipSuccess ||
+              !alloc_rl_tables(p.ranlux_luxury, &L->rl_tab))) ||
             hipMalloc((void**)&L->prn_buf, sizeof(float4) * (size_t)L->prn_quads * L->n_inst) != hipSuccess) {
             qcd_lattice_destroy(L);
             return fail(QCD_E_NOMEM, "PRN quad buffer");
@@ -2633,6 +2690,7 @@ int qcd_lattice_destroy(qcd_lattice* L)
     (void)hipFree(L->rng_buf[1]);
     (void)hipFree(L->jump_cols);
     (void)hipFree(L->rl_state);
+    (void)hipFree(L->rl_tab);
     (void)hipFree(L->prn_buf);
     (void)hipFree(L->partials);
     (void)hipFree(L->rec_index);
@@ -3074,8 +3132,9 @@ static int random_start(qcd_lattice* L)
     const uint32_t nb = align_up(n, kBlock) / kBlock;
     for (int d = 0; d < 4 && rc == QCD_OK; ++d) {
         if (L->p.prng == QCD_PRNG_RANLUX) {
-            launch_ranlux_produce(L->p.ranlux_luxury, L->rl_state, n, need, buf, L->stream);
-            if (S > need) launch_ranlux_produce(L->p.ranlux_luxury, L->rl_state, n, S - need, nullptr, L->stream);
+            launch_ranlux_produce(L->p.ranlux_luxury, L->rl_state, n, need, need, buf, L->rl_tab, L->stream);
+            if (S > need)
+                launch_ranlux_produce(L->p.ranlux_luxury, L->rl_state, n, S - need, 0, nullptr, L->rl_tab, L->stream);
         } else if (L->p.prng == QCD_PRNG_XOR128) {
             hipLaunchKernelGGL(k_xor128_produce, dim3(nb), dim3(kBlock), 0, L->stream, L->rng_buf[L->rng_cur], n, need,
                                buf);
@@ -3150,7 +3209,7 @@ int qcd_prng_init(qcd_lattice* L)
         srand(seed);
         ranlux_seed_table(L->n_inst, tab);
         HIPCHK(hipMemcpyAsync(L->rl_state, tab.data(), sizeof(float) * tab.size(), hipMemcpyHostToDevice, L->stream));
-        launch_ranlux_produce(L->p.ranlux_luxury, L->rl_state, L->n_inst, L->s_quads, nullptr, L->stream);
+        launch_ranlux_produce(L->p.ranlux_luxury, L->rl_state, L->n_inst, L->s_quads, 0, nullptr, L->rl_tab, L->stream);
         HIPCHK(hipGetLastError());
         HIPCHK(hipStreamSynchronize(L->stream));
         L->rng_ready = true;
@@ -3793,14 +3852,22 @@ int qcd_prng_produce_host(int prng, int ranlux_luxury, unsigned n, unsigned samp
             (void)hipFree(ds);
             return fail(QCD_E_NOMEM, "quads buffer");
         }
+        uint4* tab = nullptr;
+        if (!alloc_rl_tables(ranlux_luxury, &tab)) {
+            (void)hipFree(tab);
+            (void)hipFree(ds);
+            (void)hipFree(dq);
+            return fail(QCD_E_NOMEM, "RANLUX jump tables");
+        }
         hipError_t e = hipMemcpy(ds, table, sbytes, hipMemcpyHostToDevice);
         if (e == hipSuccess) {
-            launch_ranlux_produce(ranlux_luxury, ds, n, samples, dq, 0);
+            launch_ranlux_produce(ranlux_luxury, ds, n, samples, samples, dq, tab, 0);
             e = hipGetLastError();
         }
         if (e == hipSuccess) e = hipDeviceSynchronize();
         if (e == hipSuccess && qbytes) e = hipMemcpy(quads, dq, qbytes, hipMemcpyDeviceToHost);
         if (e == hipSuccess) e = hipMemcpy(table, ds, sbytes, hipMemcpyDeviceToHost);
+        (void)hipFree(tab);
         (void)hipFree(ds);
         (void)hipFree(dq);
         if (e != hipSuccess) return fail(QCD_E_HIP, "ranlux produce: %s", hipGetErrorString(e));
@@ -4093,7 +4160,7 @@ int qcd_prng_replay(qcd_lattice* L, unsigned counter, int start)
         if (left < 4) return fail(QCD_E_ARG, "counter %u cannot follow a hot start (it takes 4 productions)", counter);
         const uint32_t q = (L->p.sun == 3) ? 24u : 8u;
         if (ranlux) {
-            launch_ranlux_produce(L->p.ranlux_luxury, L->rl_state, L->n_inst, q, nullptr, L->stream);
+            launch_ranlux_produce(L->p.ranlux_luxury, L->rl_state, L->n_inst, q, 0, nullptr, L->rl_tab, L->stream);
         } else {
             const uint32_t nv = L->g.vh, nbv = align_up(nv, kBlock) / kBlock;
             if (L->p.prng == QCD_PRNG_XOR128)
@@ -4107,7 +4174,7 @@ int qcd_prng_replay(qcd_lattice* L, unsigned counter, int start)
     if (left > 0) {
         if (ranlux) {
             for (uint32_t k = 0; k < left; ++k)
-                launch_ranlux_produce(L->p.ranlux_luxury, L->rl_state, L->n_inst, L->s_quads, nullptr, L->stream);
+                launch_ranlux_produce(L->p.ranlux_luxury, L->rl_state, L->n_inst, L->s_quads, 0, nullptr, L->rl_tab, L->stream);
             HIPCHK(hipGetLastError());
         } else if (L->p.stream_mode != QCD_STREAM_REFERENCE) {
             return fail(QCD_E_UNSUPPORTED,
@@ -4399,7 +4466,11 @@ int batch_halfstep_rn(qcd_batch* B, int parity, int mu, int kind, int meas_mode,
         const uint32_t S = B->chains[0]->s_quads;
         const dim3 grid(B->len_units), block(kLinks);
         const uint2* map = B->d_map + B->off_units;
-        switch (p.ranlux_luxury) {
+        const uint32_t keep = update_quads(B->chains[0]), W = rl_waves(p.ranlux_luxury, S, keep, (uint64_t)B->len_units * kLinks);
+        if (W)
+            hipLaunchKernelGGL(k_ranlux_jump_batch, grid, dim3(64u * W), rl_lds_bytes(W), B->stream, B->d_desc, map, S, keep,
+                               B->chains[0]->rl_tab);
+        else switch (p.ranlux_luxury) {
             case 0: hipLaunchKernelGGL(k_ranlux_produce_batch<0>, grid, block, 0, B->stream, B->d_desc, map, S); break;
             case 1: hipLaunchKernelGGL(k_ranlux_produce_batch<1>, grid, block, 0, B->stream, B->d_desc, map, S); break;
             case 2: hipLaunchKernelGGL(k_ranlux_produce_batch<2>, grid, block, 0, B->stream, B->d_desc, map, S); break;
