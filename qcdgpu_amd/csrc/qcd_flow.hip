@@ -47,6 +47,7 @@
 #include <vector>
 
 #include "../../include/qcd_hip.h"
+#include "qcd_device.hpp"
 #include "qcd_internal.h"
 
 namespace {
@@ -65,6 +66,7 @@ typedef float f4 __attribute__((ext_vector_type(4)));
 struct FGeom {
     int n1, n2, n3, n4;   // extents along x, y, z, t
     uint32_t V;
+    qcd::FastDiv d2, d3, d4, dV;   // division by N2, N3, N4, V
 };
 
 __host__ __device__ inline uint16_t f2bf(float f)
@@ -84,12 +86,11 @@ __device__ inline float bf2f(uint16_t h)
 
 __device__ inline void coords(const FGeom& g, uint32_t s, int c[4])
 {
-    c[1] = (int)(s % (uint32_t)g.n2);
-    uint32_t r = s / (uint32_t)g.n2;
-    c[2] = (int)(r % (uint32_t)g.n3);
-    r /= (uint32_t)g.n3;
-    c[3] = (int)(r % (uint32_t)g.n4);
-    c[0] = (int)(r / (uint32_t)g.n4);
+    const uint32_t r = g.d2.div(s), r2 = g.d3.div(r), r3 = g.d4.div(r2);
+    c[1] = (int)(s - r * (uint32_t)g.n2);
+    c[2] = (int)(r - r2 * (uint32_t)g.n3);
+    c[3] = (int)(r2 - r3 * (uint32_t)g.n4);
+    c[0] = (int)r3;
 }
 __device__ inline uint32_t site(const FGeom& g, const int c[4])
 {
@@ -120,28 +121,51 @@ __device__ inline float4 link(const float4* L, const FGeom& g, uint32_t b, int m
     return L[((size_t)b * 4 + mu) * g.V + s];
 }
 
-// staple sum of U_mu(x) (see the file comment)
-__device__ float4 staple(const float4* L, const FGeom& g, uint32_t b, int mu, const int c[4])
+// staple sum of U_mu(x) (see the file comment).  The direction is a template
+// parameter and the 18 links are all asked for first: a previous kernel's
+// links come from beyond this XCD's L2, so each round of loads that waits for
+// the one before costs a microsecond or two.
+struct StapleLinks {
+    float4 l[3][6];
+};
+template <int mu>
+__device__ __forceinline__ void load_staple(StapleLinks& sl, const float4* L, const FGeom& g, uint32_t b, const int c[4])
 {
-    float4 A = make_float4(0.f, 0.f, 0.f, 0.f);
     const uint32_t x = site(g, c);
     const uint32_t xp = shifted(g, c, mu, 1);
-    for (int nu = 0; nu < 4; ++nu) {
-        if (nu == mu) continue;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        const int nu = k + (k >= mu ? 1 : 0);
         const uint32_t xpn = shifted(g, c, nu, 1), xmn = shifted(g, c, nu, -1);
         int cm[4] = {c[0], c[1], c[2], c[3]};
         const int n[4] = {g.n1, g.n2, g.n3, g.n4};
         cm[nu] = wrap(cm[nu] - 1, n[nu]);
         const uint32_t xpmn = shifted(g, cm, mu, 1);   // x + mu - nu
-        const float4 f = qmul(qmul(link(L, g, b, nu, xp), qdag(link(L, g, b, mu, xpn))), qdag(link(L, g, b, nu, x)));
-        const float4 r = qmul(qmul(qdag(link(L, g, b, nu, xpmn)), qdag(link(L, g, b, mu, xmn))), link(L, g, b, nu, xmn));
+        sl.l[k][0] = link(L, g, b, nu, xp);
+        sl.l[k][1] = link(L, g, b, mu, xpn);
+        sl.l[k][2] = link(L, g, b, nu, x);
+        sl.l[k][3] = link(L, g, b, nu, xpmn);
+        sl.l[k][4] = link(L, g, b, mu, xmn);
+        sl.l[k][5] = link(L, g, b, nu, xmn);
+    }
+}
+__device__ __forceinline__ float4 staple_sum(const StapleLinks& sl)
+{
+    float4 A = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        const float4* l = sl.l[k];
+        const float4 f = qmul(qmul(l[0], qdag(l[1])), qdag(l[2]));
+        const float4 r = qmul(qmul(qdag(l[3]), qdag(l[4])), l[5]);
         A = qadd(A, qadd(f, r));
     }
     return A;
 }
+// Nothing after this line is loaded before it, nothing before it later.
+__device__ __forceinline__ void loads_issued() { asm volatile("" ::: "memory"); }
 
 // (U_nu(x) U_rho(x+nu) U_nu(x+rho)^+ U_rho(x)^+)_0
-__device__ float plaq0(const float4* L, const FGeom& g, uint32_t b, int nu, int rho, const int c[4])
+__device__ __forceinline__ float plaq0(const float4* L, const FGeom& g, uint32_t b, int nu, int rho, const int c[4])
 {
     const uint32_t x = site(g, c);
     const float4 p = qmul(qmul(link(L, g, b, nu, x), link(L, g, b, rho, shifted(g, c, nu, 1))),
@@ -198,103 +222,367 @@ __global__ void k_flow_haar(float4* L, uint64_t n, uint64_t seed)
     L[j] = make_float4(q.x * nrm, q.y * nrm, q.z * nrm, q.w * nrm);
 }
 
-__global__ void k_flow_features(const float4* L, uint16_t* feat, FGeom g, uint32_t B, int mu, int par)
+template <int mu>
+__global__ __launch_bounds__(256) void k_flow_features(const float4* L, uint16_t* feat, FGeom g, uint32_t B, int par)
 {
     const uint32_t j = blockIdx.x * blockDim.x + threadIdx.x;
     if (j >= B * g.V) return;
-    const uint32_t b = j / g.V, s = j % g.V;
+    const uint32_t b = g.dV.div(j), s = j - b * g.V;
     int c[4];
     coords(g, s, c);
     const bool act = is_active(c, mu, par);
+    StapleLinks sl;
+    load_staple<mu>(sl, L, g, b, c);
+    // the three planes orthogonal to mu: U_nu(x), U_rho(x) are among the staple's links
+    float4 un[3], ur[3];
+    int k = 0;
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+#pragma unroll
+        for (int j2 = i + 1; j2 < 3; ++j2) {
+            const int nu = i + (i >= mu ? 1 : 0), rho = j2 + (j2 >= mu ? 1 : 0);
+            ur[k] = link(L, g, b, rho, shifted(g, c, nu, 1));
+            un[k] = link(L, g, b, nu, shifted(g, c, rho, 1));
+            ++k;
+        }
+    loads_issued();
     float f[kCin0] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     if (act) {
-        const float4 A = staple(L, g, b, mu, c);
+        const float4 A = staple_sum(sl);
         f[0] = sqrtf(A.x * A.x + A.y * A.y + A.z * A.z + A.w * A.w) * (1.f / 6.f);
         f[4] = 1.f;
     }
-    int k = 1;
-    for (int nu = 0; nu < 4; ++nu)
-        for (int rho = nu + 1; rho < 4; ++rho)
-            if (nu != mu && rho != mu) f[k++] = plaq0(L, g, b, nu, rho, c);
-    uint16_t* o = feat + (size_t)j * kCin0;
-    for (int q = 0; q < kCin0; ++q) o[q] = f2bf(f[q]);
+    k = 0;
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+#pragma unroll
+        for (int j2 = i + 1; j2 < 3; ++j2) {
+            const float4 p = qmul(qmul(sl.l[i][2], ur[k]), qmul(qdag(un[k]), qdag(sl.l[j2][2])));
+            f[++k] = p.x;
+        }
+    uint4 o;   // 8 channels, 16 bytes
+    o.x = f2bf(f[0]) | (uint32_t)f2bf(f[1]) << 16;
+    o.y = f2bf(f[2]) | (uint32_t)f2bf(f[3]) << 16;
+    o.z = f2bf(f[4]) | (uint32_t)f2bf(f[5]) << 16;
+    o.w = f2bf(f[6]) | (uint32_t)f2bf(f[7]) << 16;
+    reinterpret_cast<uint4*>(feat)[j] = o;
 }
 
-// One wavefront: a tile of 16 sites x 16 output channels.  in[(row) * cin +
-// channel] (BF16), wt[n * (81 cin) + k] (BF16, k = st * cin + channel),
-// out: tanh -> BF16 [row * cout + n] (act) or FP32 [row * cout + n].
-template <int CIN>
-__global__ __launch_bounds__(256) void k_flow_conv(const uint16_t* in, int cin, const uint16_t* wt, const float* bias,
-                                                   int cout, uint16_t* out_bf, float* out_f, FGeom g, uint32_t B,
-                                                   int act)
+// ---------------------------------------------------------------- convolution
+// Operand orders of the implicit GEMM.  A k-step is 16 consecutive k =
+// st * cin + channel; lane (n, q) = (lane % 16, lane / 16) holds the four k
+// at 4 q of row / column n.  Weights are stored in the order the lanes load
+// them, whole cache lines per wavefront; with 32 input channels a stencil
+// point's two k-steps come in one 16-byte load, so hidden channel c sits at
+// hid_pos(c) of its site.
+constexpr int kSteps1 = 41;   // conv1: 81 * 8 / 16, the last half empty
+constexpr size_t kW1Pack = (size_t)2 * kSteps1 * 64 * 4;
+__host__ __device__ constexpr int hid_pos(int c) { return 8 * ((c % 16) / 4) + 4 * (c / 16) + c % 4; }
+__host__ __device__ constexpr size_t w1_pos(int n, int k)
 {
-    static_assert(CIN % 4 == 0, "a lane's 4 values stay inside one stencil point");
-    (void)cin;   // == CIN (the host dispatches on it)
+    return ((size_t)((n / 16) * kSteps1 + k / 16) * 64 + n % 16 + 16 * ((k % 16) / 4)) * 4 + k % 4;
+}
+__host__ __device__ constexpr size_t w2_pos(int n, int k) { return ((size_t)(k / 32) * 64 + n + 16 * ((k % 16) / 4)) * 8 + 4 * ((k % 32) / 16) + k % 4; }
+__host__ __device__ constexpr size_t w2t_pos(int c, int k)   // k = st * 16 + n
+{
+    return ((size_t)((c / 16) * kStencil + k / 16) * 64 + c % 16 + 16 * ((k % 16) / 4)) * 4 + k % 4;
+}
+
+template <int CIN> struct ConvOp {
+    static constexpr int loads = CIN == 8 ? kSteps1 : kStencil;   // operand loads along k
+    static constexpr int per = CIN == 32 ? 2 : 1;                 // k-steps per load
+    static constexpr int ntiles = CIN == 32 ? 1 : 2;              // output tiles of 16 channels
+    typedef short V __attribute__((ext_vector_type(4 * per)));
+};
+
+// One wavefront: MT tiles of 16 sites x NT tiles of 16 output channels.
+// in[row * CIN + channel] (BF16), out: tanh -> BF16 at hid_pos (ACT) or FP32
+// [row * cout + n].  The loads of BS operand steps are issued before the
+// matrix instructions of the previous BS, which run in k order whatever the
+// shape, so every shape gives the same sums.
+template <int CIN, int MT, int NT, int BS, bool ACT>
+__global__ __launch_bounds__(256) void k_flow_conv(const uint16_t* in, const uint16_t* wt, const float* bias,
+                                                   uint16_t* out_bf, float* out_f, FGeom g, uint32_t ntile_m)
+{
+    using Op = ConvOp<CIN>;
+    using V = typename Op::V;
+    constexpr int COUT = 16 * Op::ntiles, NL = Op::loads, NB = (NL + BS - 1) / BS;
     const uint32_t wave = __builtin_amdgcn_readfirstlane((int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6));
-    const int lane = threadIdx.x & 63;
-    const uint32_t ntile_m = B * g.V / 16, ntile_n = (uint32_t)cout / 16;
-    if (wave >= ntile_m * ntile_n) return;   // whole wavefront
-    const uint32_t tm = wave % ntile_m, tn = wave / ntile_m;
-    const uint32_t row = tm * 16 + (lane & 15);   // A row of this lane
-    const uint32_t b = row / g.V, s = row % g.V;
-    int c[4];
-    coords(g, s, c);
+    const int lane = threadIdx.x & 63, q = lane >> 4;
+    const uint32_t groups = (ntile_m + MT - 1) / MT;
+    if (wave >= groups * (Op::ntiles / NT)) return;   // whole wavefront
+    const uint32_t tm = wave % groups, tn = (wave / groups) * NT;
+    // byte offsets of the 3 neighbour positions along each direction, per tile; the tile's configuration is the base
+    const char* base[MT];
+    uint32_t xo[MT][3], yo[MT][3], zo[MT][3], to[MT][3];
     const int n[4] = {g.n1, g.n2, g.n3, g.n4};
-    const int kq = 4 * (lane >> 4);                // k offset of this lane's 4 values
-    const uint32_t ncol = tn * 16 + (lane & 15);   // B column of this lane
-    constexpr int K = kStencil * CIN;
-    const uint16_t* wrow = wt + (size_t)ncol * K;
-    const uint16_t* inb = in + (size_t)b * g.V * CIN;
-    f4 acc = {0.f, 0.f, 0.f, 0.f};
-    // The operands of U consecutive k-steps are loaded before their MFMAs,
-    // so U gathers are in flight at once; the MFMAs run in k order, as one
-    // step at a time would.
-    constexpr int U = 8;
-    for (int k0 = 0; k0 < K; k0 += 16 * U) {
-        s4 av[U], bv[U];
+    constexpr uint32_t B = 2u * CIN;
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const int k = k0 + 16 * u + kq;   // K is a multiple of 4: a lane's 4 values are all inside or all past K
-            av[u] = s4{0, 0, 0, 0};
-            bv[u] = s4{0, 0, 0, 0};
-            if (k < K) {
-                const int st = k / CIN, ch = k % CIN;
-                const int o[4] = {st / 27 - 1, (st / 9) % 3 - 1, (st / 3) % 3 - 1, st % 3 - 1};
-                int e[4];
+    for (int m = 0; m < MT; ++m) {
+        const uint32_t tile = min(tm * MT + m, ntile_m - 1u);
+        const uint32_t b = g.dV.div(tile * 16);   // 16 divides V: a tile is inside one configuration
+        base[m] = reinterpret_cast<const char*>(in) + (size_t)b * g.V * B;
+        int c[4];
+        coords(g, tile * 16 - b * g.V + (uint32_t)(lane & 15), c);
 #pragma unroll
-                for (int d = 0; d < 4; ++d) e[d] = wrap(c[d] + o[d], n[d]);
-                av[u] = *reinterpret_cast<const s4*>(inb + (size_t)site(g, e) * CIN + ch);
-                bv[u] = *reinterpret_cast<const s4*>(wrow + k);
+        for (int o = 0; o < 3; ++o) {
+            // the lane's 4 (or 2 x 4) channels of a point: 8 q bytes on, or 16 q
+            // for two k-steps; with 8 channels a k-step is two points
+            xo[m][o] = (uint32_t)wrap(c[0] + o - 1, n[0]) * (uint32_t)(n[1] * n[2] * n[3]) * B +
+                       (CIN == 8 ? 8u * (q & 1) : 8u * Op::per * (uint32_t)q);
+            yo[m][o] = (uint32_t)wrap(c[1] + o - 1, n[1]) * B;
+            zo[m][o] = (uint32_t)wrap(c[2] + o - 1, n[2]) * (uint32_t)n[1] * B;
+            to[m][o] = (uint32_t)wrap(c[3] + o - 1, n[3]) * (uint32_t)(n[1] * n[2]) * B;
+        }
+    }
+    auto point = [&](int m, int st) { return xo[m][st / 27] + yo[m][(st / 9) % 3] + zo[m][(st / 3) % 3] + to[m][st % 3]; };
+    auto offset = [&](int m, int l) -> uint32_t {
+        if constexpr (CIN == 8) {
+            const uint32_t a = point(m, 2 * l), b = 2 * l + 1 < kStencil ? point(m, 2 * l + 1) : a;
+            return q < 2 ? a : b;
+        } else {
+            return point(m, l);
+        }
+    };
+    const V* wl[NT];
+#pragma unroll
+    for (int t = 0; t < NT; ++t) wl[t] = reinterpret_cast<const V*>(wt) + (size_t)(tn + t) * NL * 64 + lane;
+    f4 acc[MT][NT];
+#pragma unroll
+    for (int m = 0; m < MT; ++m)
+#pragma unroll
+        for (int t = 0; t < NT; ++t) acc[m][t] = f4{0.f, 0.f, 0.f, 0.f};
+    V av[2][BS][MT], bv[2][BS][NT];
+    auto issue = [&](int bt) {
+#pragma unroll
+        for (int i = 0; i < BS; ++i) {
+            const int l = bt * BS + i;
+            if (l >= NL) break;
+#pragma unroll
+            for (int t = 0; t < NT; ++t) bv[bt & 1][i][t] = wl[t][(size_t)l * 64];
+#pragma unroll
+            for (int m = 0; m < MT; ++m) av[bt & 1][i][m] = *reinterpret_cast<const V*>(base[m] + offset(m, l));
+        }
+        asm volatile("" ::: "memory");   // these loads before, the next batch's after
+    };
+    issue(0);
+#pragma unroll
+    for (int bt = 0; bt < NB; ++bt) {
+        if (bt + 1 < NB) issue(bt + 1);
+#pragma unroll
+        for (int i = 0; i < BS; ++i) {
+            if (bt * BS + i >= NL) break;
+#pragma unroll
+            for (int h = 0; h < Op::per; ++h)
+#pragma unroll
+                for (int m = 0; m < MT; ++m)
+#pragma unroll
+                    for (int t = 0; t < NT; ++t) {
+                        s4 a, b;
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) {
+                            a[j] = av[bt & 1][i][m][4 * h + j];
+                            b[j] = bv[bt & 1][i][t][4 * h + j];
+                        }
+                        acc[m][t] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, acc[m][t], 0, 0, 0);
+                    }
+        }
+    }
+    // lane holds D[4 * (lane / 16) + i][lane % 16]
+#pragma unroll
+    for (int m = 0; m < MT; ++m) {
+        if (tm * MT + m >= ntile_m) break;
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+            const int ncol = (int)(tn + t) * 16 + (lane & 15);
+            const float bs = bias[ncol];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const size_t r = (size_t)(tm * MT + m) * 16 + 4 * q + i;
+                const float v = acc[m][t][i] + bs;
+                if constexpr (ACT) out_bf[r * COUT + hid_pos(ncol)] = f2bf(tanhf(v));
+                else out_f[r * COUT + ncol] = v;
+            }
+        }
+    }
+}
+
+// The same sums with the input in LDS: one workgroup of 4 wavefronts per
+// x-plane of a configuration stages the plane and its two neighbours (`plane`
+// sites each, contiguous) and every one of the 81 gathers of a site reads
+// from there.  A wavefront takes MT tiles of 16 sites at a time.
+template <int CIN, int MT, int BS, int WV, bool ACT>
+__global__ __launch_bounds__(64 * WV) void k_flow_conv_plane(const uint16_t* in, const uint16_t* wt, const float* bias,
+                                                         uint16_t* out_bf, float* out_f, FGeom g, uint32_t plane)
+{
+    using Op = ConvOp<CIN>;
+    using V = typename Op::V;
+    constexpr int COUT = 16 * Op::ntiles, NL = Op::loads, NB = (NL + BS - 1) / BS, NT = Op::ntiles;
+    constexpr uint32_t B = 2u * CIN;
+    extern __shared__ uint4 planes[];
+    const uint32_t b = blockIdx.x / (uint32_t)g.n1, x = blockIdx.x % (uint32_t)g.n1;
+    const uint32_t pv = plane * B / 16u;   // 16-byte vectors of a plane
+#pragma unroll
+    for (int o = 0; o < 3; ++o) {
+        const uint4* src = reinterpret_cast<const uint4*>(in) +
+                           ((size_t)b * (uint32_t)g.n1 + (uint32_t)wrap((int)x + o - 1, g.n1)) * pv;
+#pragma unroll 4
+        for (uint32_t i = threadIdx.x; i < pv; i += 64u * WV) planes[o * pv + i] = src[i];
+    }
+    __syncthreads();
+    const char* sm = reinterpret_cast<const char*>(planes);
+    const uint32_t w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), tiles = plane / 16u;
+    const int lane = threadIdx.x & 63, q = lane >> 4;
+    const int n[4] = {g.n1, g.n2, g.n3, g.n4};
+    const V* wl[NT];
+#pragma unroll
+    for (int t = 0; t < NT; ++t) wl[t] = reinterpret_cast<const V*>(wt) + (size_t)t * NL * 64 + lane;
+    for (uint32_t t0 = w * MT; t0 < tiles; t0 += WV * MT) {
+        uint32_t yo[MT][3], zo[MT][3], to[MT][3];
+#pragma unroll
+        for (int m = 0; m < MT; ++m) {
+            int c[4];
+            coords(g, min(t0 + m, tiles - 1u) * 16u + (uint32_t)(lane & 15), c);
+#pragma unroll
+            for (int o = 0; o < 3; ++o) {
+                yo[m][o] = (uint32_t)wrap(c[1] + o - 1, n[1]) * B + (CIN == 8 ? 8u * (q & 1) : 8u * Op::per * (uint32_t)q);
+                zo[m][o] = (uint32_t)wrap(c[2] + o - 1, n[2]) * (uint32_t)n[1] * B;
+                to[m][o] = (uint32_t)wrap(c[3] + o - 1, n[3]) * (uint32_t)(n[1] * n[2]) * B;
+            }
+        }
+        auto point = [&](int m, int st) {
+            return (uint32_t)(st / 27) * plane * B + yo[m][(st / 9) % 3] + zo[m][(st / 3) % 3] + to[m][st % 3];
+        };
+        auto offset = [&](int m, int l) -> uint32_t {
+            if constexpr (CIN == 8) {
+                const uint32_t a0 = point(m, 2 * l), a1 = 2 * l + 1 < kStencil ? point(m, 2 * l + 1) : a0;
+                return q < 2 ? a0 : a1;
+            } else {
+                return point(m, l);
+            }
+        };
+        f4 acc[MT][NT];
+#pragma unroll
+        for (int m = 0; m < MT; ++m)
+#pragma unroll
+            for (int t = 0; t < NT; ++t) acc[m][t] = f4{0.f, 0.f, 0.f, 0.f};
+        V av[2][BS][MT], bv[2][BS][NT];
+        auto issue = [&](int bt) {
+#pragma unroll
+            for (int i = 0; i < BS; ++i) {
+                const int l = bt * BS + i;
+                if (l >= NL) break;
+#pragma unroll
+                for (int t = 0; t < NT; ++t) bv[bt & 1][i][t] = wl[t][(size_t)l * 64];
+#pragma unroll
+                for (int m = 0; m < MT; ++m) av[bt & 1][i][m] = *reinterpret_cast<const V*>(sm + offset(m, l));
+            }
+            asm volatile("" ::: "memory");
+        };
+        issue(0);
+#pragma unroll
+        for (int bt = 0; bt < NB; ++bt) {
+            if (bt + 1 < NB) issue(bt + 1);
+#pragma unroll
+            for (int i = 0; i < BS; ++i) {
+                if (bt * BS + i >= NL) break;
+#pragma unroll
+                for (int h = 0; h < Op::per; ++h)
+#pragma unroll
+                    for (int m = 0; m < MT; ++m)
+#pragma unroll
+                        for (int t = 0; t < NT; ++t) {
+                            s4 av4, bv4;
+#pragma unroll
+                            for (int j = 0; j < 4; ++j) {
+                                av4[j] = av[bt & 1][i][m][4 * h + j];
+                                bv4[j] = bv[bt & 1][i][t][4 * h + j];
+                            }
+                            acc[m][t] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(av4, bv4, acc[m][t], 0, 0, 0);
+                        }
             }
         }
 #pragma unroll
-        for (int u = 0; u < U; ++u) acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(av[u], bv[u], acc, 0, 0, 0);
-    }
-    // lane holds D[4 * (lane / 16) + i][lane % 16]
-    for (int i = 0; i < 4; ++i) {
-        const uint32_t r = tm * 16 + 4 * (lane >> 4) + i;
-        float v = acc[i] + bias[ncol];
-        if (act) out_bf[(size_t)r * cout + ncol] = f2bf(tanhf(v));
-        else out_f[(size_t)r * cout + ncol] = v;
+        for (int m = 0; m < MT; ++m) {
+            if (t0 + m >= tiles) break;
+#pragma unroll
+            for (int t = 0; t < NT; ++t) {
+                const int ncol = t * 16 + (lane & 15);
+                const float bs = bias[ncol];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const size_t r = (size_t)blockIdx.x * plane + (size_t)(t0 + m) * 16 + 4 * q + i;
+                    const float v = acc[m][t][i] + bs;
+                    if constexpr (ACT) out_bf[r * COUT + hid_pos(ncol)] = f2bf(tanhf(v));
+                    else out_f[r * COUT + ncol] = v;
+                }
+            }
+        }
     }
 }
 
-struct Spline {
-    float xk[kMaxBins + 1], yk[kMaxBins + 1], d[kMaxBins + 1];
-    int K;
+// Launch for `rows` sites.  Measured for 32 -> 16 channels on 8^3 x 4 sites
+// (one wavefront per tile and eight gathers in flight before: 33 us for one
+// configuration, 159 us for 64, bound by the gathers' latency and the L1):
+//   one configuration (128 tiles)    4.0 us as one tile per wavefront, 14 in planes
+//   8 (64 planes)                   10.2                             12.2
+//   16 (128 planes)                 16.6                             12.6
+//   64 (512 planes)                 45.7 with four tiles             25.1, with 8 wavefronts 29.3
+// The matrix instructions of 64 configurations take 8.6 us.
+template <int CIN, bool ACT>
+void launch_conv(const uint16_t* in, const uint16_t* wt, const float* bias, uint16_t* out_bf, float* out_f, const FGeom& g,
+                 uint32_t rows, hipStream_t st)
+{
+    constexpr int NTT = ConvOp<CIN>::ntiles, BS = CIN == 16 ? 3 : 6;   // 16 channels: 6 would spill
+    const uint32_t tiles = rows / 16, plane = g.V / (uint32_t)g.n1, planes = rows / plane, lds = 3u * plane * 2u * CIN;
+    if (plane % 16 == 0 && lds <= 64u * 1024u && planes >= 96u) {
+        if (planes <= 256u)
+            hipLaunchKernelGGL((k_flow_conv_plane<CIN, 2, BS, 8, ACT>), dim3(planes), dim3(512), lds, st, in, wt, bias,
+                               out_bf, out_f, g, plane);
+        else
+            hipLaunchKernelGGL((k_flow_conv_plane<CIN, 2, BS, 4, ACT>), dim3(planes), dim3(256), lds, st, in, wt, bias,
+                               out_bf, out_f, g, plane);
+    } else if (tiles <= 4096u) {
+        hipLaunchKernelGGL((k_flow_conv<CIN, 1, 1, 9, ACT>), dim3(tiles * NTT), dim3(64), 0, st, in, wt, bias, out_bf,
+                           out_f, g, tiles);
+    } else {
+        hipLaunchKernelGGL((k_flow_conv<CIN, 4, NTT, 3, ACT>), dim3((tiles + 15) / 16), dim3(256), 0, st, in, wt, bias,
+                           out_bf, out_f, g, tiles);
+    }
+}
+
+// The number of bins is a template parameter, so that the knots live in
+// registers and a site's 16 raw parameters are four loads (with a run-time
+// count every one of them was a load of its own, waited for in turn).
+template <int K> struct Spline {
+    float xk[K + 1], yk[K + 1], d[K + 1];
 };
 
 __device__ inline float softplus(float x) { return x > 20.f ? x : log1pf(expf(x)); }
 
-__device__ void make_spline(const float* r, int K, Spline& sp)
+__device__ __forceinline__ void load_raw(float (&r)[kOut], const float* prm, size_t row)
 {
-    sp.K = K;
+    const float4* v = reinterpret_cast<const float4*>(prm) + 4 * row;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const float4 a = v[q];
+        r[4 * q] = a.x;
+        r[4 * q + 1] = a.y;
+        r[4 * q + 2] = a.z;
+        r[4 * q + 3] = a.w;
+    }
+}
+
+template <int K> __device__ __forceinline__ void make_spline(const float (&r)[kOut], Spline<K>& sp)
+{
     float mw = r[0], mh = r[K];
+#pragma unroll
     for (int i = 1; i < K; ++i) {
         mw = fmaxf(mw, r[i]);
         mh = fmaxf(mh, r[K + i]);
     }
-    float ew[kMaxBins], eh[kMaxBins], sw = 0.f, sh = 0.f;
+    float ew[K], eh[K], sw = 0.f, sh = 0.f;
+#pragma unroll
     for (int i = 0; i < K; ++i) {
         ew[i] = expf(r[i] - mw);
         eh[i] = expf(r[K + i] - mh);
@@ -302,76 +590,100 @@ __device__ void make_spline(const float* r, int K, Spline& sp)
         sh += eh[i];
     }
     sp.xk[0] = sp.yk[0] = 0.f;
+#pragma unroll
     for (int i = 0; i < K; ++i) {
         sp.xk[i + 1] = sp.xk[i] + kPi * (kMinW + (1.f - K * kMinW) * ew[i] / sw);
         sp.yk[i + 1] = sp.yk[i] + kPi * (kMinW + (1.f - K * kMinW) * eh[i] / sh);
     }
     sp.xk[K] = sp.yk[K] = kPi;
+#pragma unroll
     for (int i = 0; i <= K; ++i) sp.d[i] = kMinD + (1.f - kMinD) * softplus(r[2 * K + i]) * 1.4426950408889634f;
 }
 
-// forward: y = f(x), dlog = log f'(x)
-__device__ float spline_fwd(const Spline& sp, float x, float& dlog)
+// Bin of v among the knots (the first whose upper knot exceeds v) and its corner values.
+template <int K> struct Bin {
+    float x0, x1, y0, y1, d0, d1;
+};
+template <int K> __device__ __forceinline__ Bin<K> find_bin(const Spline<K>& sp, const float (&knots)[K + 1], float v)
 {
-    int k = 0;
-    while (k < sp.K - 1 && x >= sp.xk[k + 1]) ++k;
-    const float w = sp.xk[k + 1] - sp.xk[k], h = sp.yk[k + 1] - sp.yk[k], s = h / w;
-    const float xi = fminf(fmaxf((x - sp.xk[k]) / w, 0.f), 1.f), om = 1.f - xi;
-    const float den = s + (sp.d[k + 1] + sp.d[k] - 2.f * s) * xi * om;
-    const float y = sp.yk[k] + h * (s * xi * xi + sp.d[k] * xi * om) / den;
-    const float num = s * s * (sp.d[k + 1] * xi * xi + 2.f * s * xi * om + sp.d[k] * om * om);
+    Bin<K> b{sp.xk[0], sp.xk[1], sp.yk[0], sp.yk[1], sp.d[0], sp.d[1]};
+    bool go = true;
+#pragma unroll
+    for (int i = 1; i < K; ++i) {
+        go = go && v >= knots[i];
+        if (go) b = Bin<K>{sp.xk[i], sp.xk[i + 1], sp.yk[i], sp.yk[i + 1], sp.d[i], sp.d[i + 1]};
+    }
+    return b;
+}
+
+// forward: y = f(x), dlog = log f'(x)
+template <int K> __device__ __forceinline__ float spline_fwd(const Spline<K>& sp, float x, float& dlog)
+{
+    const Bin<K> b = find_bin<K>(sp, sp.xk, x);
+    const float w = b.x1 - b.x0, h = b.y1 - b.y0, s = h / w;
+    const float xi = fminf(fmaxf((x - b.x0) / w, 0.f), 1.f), om = 1.f - xi;
+    const float den = s + (b.d1 + b.d0 - 2.f * s) * xi * om;
+    const float y = b.y0 + h * (s * xi * xi + b.d0 * xi * om) / den;
+    const float num = s * s * (b.d1 * xi * xi + 2.f * s * xi * om + b.d0 * om * om);
     dlog = logf(num) - 2.f * logf(den);
     return y;
 }
 
 // inverse: x = f^-1(y), dlog = log f'(x)
-__device__ float spline_inv(const Spline& sp, float y, float& dlog)
+template <int K> __device__ __forceinline__ float spline_inv(const Spline<K>& sp, float y, float& dlog)
 {
-    int k = 0;
-    while (k < sp.K - 1 && y >= sp.yk[k + 1]) ++k;
-    const float w = sp.xk[k + 1] - sp.xk[k], h = sp.yk[k + 1] - sp.yk[k], s = h / w;
-    const float dy = y - sp.yk[k], dd = sp.d[k + 1] + sp.d[k] - 2.f * s;
-    const float a = h * (s - sp.d[k]) + dy * dd;
-    const float bq = h * sp.d[k] - dy * dd;
+    const Bin<K> b = find_bin<K>(sp, sp.yk, y);
+    const float w = b.x1 - b.x0, h = b.y1 - b.y0, s = h / w;
+    const float dy = y - b.y0, dd = b.d1 + b.d0 - 2.f * s;
+    const float a = h * (s - b.d0) + dy * dd;
+    const float bq = h * b.d0 - dy * dd;
     const float cq = -s * dy;
     const float disc = fmaxf(bq * bq - 4.f * a * cq, 0.f);
     const float xi = fminf(fmaxf(2.f * cq / (-bq - sqrtf(disc)), 0.f), 1.f), om = 1.f - xi;
     const float den = s + dd * xi * om;
-    const float num = s * s * (sp.d[k + 1] * xi * xi + 2.f * s * xi * om + sp.d[k] * om * om);
+    const float num = s * s * (b.d1 * xi * xi + 2.f * s * xi * om + b.d0 * om * om);
     dlog = logf(num) - 2.f * logf(den);
-    return sp.xk[k] + xi * w;
+    return b.x0 + xi * w;
 }
 
 // Coupling of layer (mu, par): forward (inverse = 0) maps theta -> f(theta),
 // inverse maps theta' -> f^-1(theta'); both add log J = log f'(theta) +
 // 2 log(sin f(theta) / sin theta) of the forward map to logj[row].
-__global__ void k_flow_couple(float4* L, const float* prm, float* logj, FGeom g, uint32_t B, int mu, int par, int K,
-                              int inverse)
+template <int mu, int K>
+__global__ __launch_bounds__(256) void k_flow_couple(float4* L, const float* prm, float* logj, FGeom g, uint32_t B, int par,
+                                                     int inverse)
 {
     const uint32_t j = blockIdx.x * blockDim.x + threadIdx.x;
     if (j >= B * g.V) return;
-    const uint32_t b = j / g.V, s = j % g.V;
+    const uint32_t b = g.dV.div(j), s = j - b * g.V;
     int c[4];
     coords(g, s, c);
     if (!is_active(c, mu, par)) return;
-    const float4 A = staple(L, g, b, mu, c);
+    StapleLinks sl;
+    load_staple<mu>(sl, L, g, b, c);
+    float4& U = L[((size_t)b * 4 + mu) * g.V + s];
+    const float4 U0 = U;
+    float raw[kOut];
+    load_raw(raw, prm, j);
+    const float lj0 = logj[j];
+    loads_issued();
+    const float4 A = staple_sum(sl);
     const float k = sqrtf(A.x * A.x + A.y * A.y + A.z * A.z + A.w * A.w);
     if (!(k > 1e-20f)) return;
     const float ik = 1.f / k;
     const float4 Vq = make_float4(A.x * ik, A.y * ik, A.z * ik, A.w * ik);
-    float4& U = L[((size_t)b * 4 + mu) * g.V + s];
-    const float4 W = qmul(U, Vq);
+    const float4 W = qmul(U0, Vq);
     const float sn = sqrtf(W.y * W.y + W.z * W.z + W.w * W.w);
     const float th = atan2f(sn, W.x);
-    Spline sp;
-    make_spline(prm + (size_t)j * kOut, K, sp);
+    Spline<K> sp;
+    make_spline<K>(raw, sp);
     float dlog, th2;
     if (!inverse) th2 = spline_fwd(sp, th, dlog);
     else th2 = spline_inv(sp, th, dlog);
     const float th_in = inverse ? th2 : th, th_out = inverse ? th : th2;   // theta and f(theta)
     const float si = sinf(th_in), so = sinf(th_out);
     const float ratio = (si > 1e-6f && so > 1e-6f) ? so / si : expf(dlog);   // limit at the poles: f'(theta)
-    logj[j] += dlog + 2.f * logf(ratio);
+    logj[j] = lj0 + (dlog + 2.f * logf(ratio));
     float4 Wn;
     if (sn > 1e-12f) {
         const float f = sinf(th2) / sn;
@@ -413,7 +725,8 @@ __global__ void k_flow_imh_key(unsigned long long* imh, unsigned long long seed,
     }
 }
 
-__global__ __launch_bounds__(256) void k_flow_imh_couple(float4* L, const float* prm, FGeom g, int mu, int par, int K,
+template <int mu, int K>
+__global__ __launch_bounds__(256) void k_flow_imh_couple(float4* L, const float* prm, FGeom g, int par,
                                                          float beta, uint64_t lmix, unsigned long long* imh)
 {
     const uint32_t s = blockIdx.x * blockDim.x + threadIdx.x;
@@ -425,16 +738,22 @@ __global__ __launch_bounds__(256) void k_flow_imh_couple(float4* L, const float*
         int c[4];
         coords(g, s, c);
         if (is_active(c, mu, par)) {
-            const float4 A = staple(L, g, 0, mu, c);
+            StapleLinks sl;
+            load_staple<mu>(sl, L, g, 0, c);
+            float4& U = L[(size_t)mu * g.V + s];
+            const float4 U0 = U;
+            float raw[kOut];
+            load_raw(raw, prm, s);
+            loads_issued();
+            const float4 A = staple_sum(sl);
             const float k = sqrtf(A.x * A.x + A.y * A.y + A.z * A.z + A.w * A.w);
             if (k > 1e-20f) {
                 const float ik = 1.f / k;
                 const float4 Vq = make_float4(A.x * ik, A.y * ik, A.z * ik, A.w * ik);
-                float4& U = L[(size_t)mu * g.V + s];
-                const float4 W = qmul(U, Vq);
+                const float4 W = qmul(U0, Vq);
                 const float th = atan2f(sqrtf(W.y * W.y + W.z * W.z + W.w * W.w), W.x);
-                Spline sp;
-                make_spline(prm + (size_t)s * kOut, K, sp);
+                Spline<K> sp;
+                make_spline<K>(raw, sp);
                 float dlog;
                 const float thz = spline_inv(sp, th, dlog);
                 const float lj_cur = log_jac(dlog, thz, th);
@@ -531,19 +850,22 @@ __device__ double nll_link(const double* r, int K, double th)
 // precision, step 1e-5; the map is smooth except at bin edges, a set of
 // measure zero) into g (BF16, [row][16], zero at inactive sites and for
 // the unused channels); loss[row] = -log q_a (0 at inactive sites).
+template <int mu>
 __global__ void k_flow_nll_grad(const float4* L, const float* prm, uint16_t* g, float* loss, FGeom g4, uint32_t B,
-                                int mu, int par, int K)
+                                int par, int K)
 {
     const uint32_t j = blockIdx.x * blockDim.x + threadIdx.x;
     if (j >= B * g4.V) return;
-    const uint32_t b = j / g4.V, s = j % g4.V;
+    const uint32_t b = g4.dV.div(j), s = j - b * g4.V;
     int c[4];
     coords(g4, s, c);
     float gr[kOut];
     for (int q = 0; q < kOut; ++q) gr[q] = 0.f;
     float lo = 0.f;
     if (is_active(c, mu, par)) {
-        const float4 A = staple(L, g4, b, mu, c);
+        StapleLinks sl;
+        load_staple<mu>(sl, L, g4, b, c);
+        const float4 A = staple_sum(sl);
         const float k = sqrtf(A.x * A.x + A.y * A.y + A.z * A.z + A.w * A.w);
         if (k > 1e-20f) {
             const float ik = 1.f / k;
@@ -604,7 +926,7 @@ __global__ __launch_bounds__(256) void k_flow_wgrad(const uint16_t* gout, int co
                 coords(g, s, c);
                 int e[4];
                 for (int d = 0; d < 4; ++d) e[d] = wrap(c[d] + o[d], n[d]);
-                bv[q] = (short)in[((size_t)b * g.V + site(g, e)) * cin + ch];
+                bv[q] = (short)in[((size_t)b * g.V + site(g, e)) * cin + (cin == kHidden ? hid_pos(ch) : ch)];
             }
         }
         acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(av, bv, acc, 0, 0, 0);
@@ -641,7 +963,7 @@ __global__ __launch_bounds__(256) void k_flow_colsum(const uint16_t* gout, int c
     if (threadIdx.x == 0) out[blockIdx.x] = red[0];
 }
 
-// transposed conv2 weights for the input gradient: wt[c][st * 16 + n] =
+// transposed conv2 weights for the input gradient: entry (c, st * 16 + n) =
 // W2[n][(80 - st) * 32 + c] (the stencil point of offset -o)
 __global__ void k_flow_w2_transpose(const uint16_t* w2, uint16_t* wt)
 {
@@ -649,7 +971,7 @@ __global__ void k_flow_w2_transpose(const uint16_t* w2, uint16_t* wt)
     if (i >= (uint32_t)(kHidden * kStencil * kOut)) return;
     const uint32_t c = i / (kStencil * kOut), rest = i % (kStencil * kOut);
     const uint32_t st = rest / kOut, nn = rest % kOut;
-    wt[i] = w2[(size_t)nn * (kStencil * kHidden) + (kStencil - 1 - st) * kHidden + c];
+    wt[w2t_pos((int)c, (int)rest)] = w2[w2_pos((int)nn, (int)((kStencil - 1 - st) * kHidden + c))];
 }
 
 // dpre = dhid (1 - h^2), h the tanh output (BF16)
@@ -657,7 +979,7 @@ __global__ void k_flow_tanh_back(const float* dhid, const uint16_t* h, uint16_t*
 {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
-    const float hv = bf2f(h[i]);
+    const float hv = bf2f(h[i - i % kHidden + hid_pos((int)(i % kHidden))]);
     dpre[i] = f2bf(dhid[i] * (1.f - hv * hv));
 }
 
@@ -683,11 +1005,11 @@ __global__ void k_flow_unpack_params(const float* p, uint32_t layers, uint16_t* 
     const uint32_t l = (uint32_t)(i / per);
     uint64_t o = i % per;
     const uint64_t n1 = (uint64_t)kHidden * kStencil * kCin0, n2 = (uint64_t)kOut * kStencil * kHidden;
-    if (o < n1) { w1[l * n1 + o] = f2bf(p[i]); return; }
+    if (o < n1) { w1[l * kW1Pack + w1_pos((int)(o / (kStencil * kCin0)), (int)(o % (kStencil * kCin0)))] = f2bf(p[i]); return; }
     o -= n1;
     if (o < kHidden) { b1[l * kHidden + o] = p[i]; return; }
     o -= kHidden;
-    if (o < n2) { w2[l * n2 + o] = f2bf(p[i]); return; }
+    if (o < n2) { w2[l * n2 + w2_pos((int)(o / (kStencil * kHidden)), (int)(o % (kStencil * kHidden)))] = f2bf(p[i]); return; }
     o -= n2;
     b2[l * kOut + o] = p[i];
 }
@@ -697,7 +1019,7 @@ __global__ void k_flow_action_sites(const float4* L, double* out, FGeom g, uint3
 {
     const uint32_t j = blockIdx.x * blockDim.x + threadIdx.x;
     if (j >= B * g.V) return;
-    const uint32_t b = j / g.V, s = j % g.V;
+    const uint32_t b = g.dV.div(j), s = j - b * g.V;
     int c[4];
     coords(g, s, c);
     double acc = 0.0;
@@ -731,6 +1053,7 @@ struct qcd_flow {
     qcd_flow_desc d;
     FGeom g;
     size_t nparam = 0;
+    float* staged = nullptr;   // parameters as uploaded, FP32
     std::vector<float> host_params;
     uint16_t* w1 = nullptr;    // [layers][32][81 * 8]
     float* b1 = nullptr;       // [layers][32]
@@ -777,22 +1100,60 @@ constexpr size_t kLayerParams = kW1 + kHidden + kW2 + kOut;
         if (e_ != hipSuccess) return err(QCD_E_HIP, std::string(#x) + ": " + hipGetErrorString(e_)); \
     } while (0)
 
+// Calls f with the direction as a compile-time constant.
+template <typename Fn> void with_mu(int mu, Fn f)
+{
+    switch (mu) {
+        case 0: f(std::integral_constant<int, 0>{}); break;
+        case 1: f(std::integral_constant<int, 1>{}); break;
+        case 2: f(std::integral_constant<int, 2>{}); break;
+        default: f(std::integral_constant<int, 3>{}); break;
+    }
+}
+
+// The same with the number of spline bins.
+template <typename Fn> void with_mu_bins(int mu, int bins, Fn f)
+{
+    with_mu(mu, [&](auto m) {
+        switch (bins) {
+            case 1: f(m, std::integral_constant<int, 1>{}); break;
+            case 2: f(m, std::integral_constant<int, 2>{}); break;
+            case 3: f(m, std::integral_constant<int, 3>{}); break;
+            case 4: f(m, std::integral_constant<int, 4>{}); break;
+            default: f(m, std::integral_constant<int, kMaxBins>{}); break;
+        }
+    });
+}
+
+// Workgroup of the one-thread-per-site kernels: few sites go to as many CUs
+// as there are wavefronts.
+dim3 site_block(uint32_t n) { return dim3(n <= 65536u ? 64u : 256u); }
+dim3 site_grid(uint32_t n) { return dim3((n + site_block(n).x - 1) / site_block(n).x); }
+
+// Spline parameters (F->prm) of layer l from the features in F->feat.
+void conditioner(qcd_flow* F, int l, uint32_t rows, hipStream_t st)
+{
+    launch_conv<kCin0, true>(F->feat, F->w1 + l * kW1Pack, F->b1 + l * kHidden, F->hid, nullptr, F->g, rows, st);
+    launch_conv<kHidden, false>(F->hid, F->w2 + l * kW2, F->b2 + l * kOut, nullptr, F->prm, F->g, rows, st);
+}
+
 int run_layers(qcd_flow* F, uint32_t B, bool inverse)
 {
     const FGeom g = F->g;
-    const uint32_t n = B * g.V, nb = (n + 255) / 256;
+    const uint32_t n = B * g.V;
     FCHK(hipMemsetAsync(F->logj, 0, sizeof(float) * n, F->stream));
     for (int step = 0; step < F->d.layers; ++step) {
         const int l = inverse ? F->d.layers - 1 - step : step;
         const int mu = l % 4, par = (l / 4) % 2;
-        hipLaunchKernelGGL(k_flow_features, dim3(nb), dim3(256), 0, F->stream, F->links, F->feat, g, B, mu, par);
-        const uint32_t w1n = (n / 16) * (kHidden / 16), w2n = (n / 16) * (kOut / 16);
-        hipLaunchKernelGGL(k_flow_conv<kCin0>, dim3((w1n + 3) / 4), dim3(256), 0, F->stream, F->feat, kCin0, F->w1 + l * kW1,
-                           F->b1 + l * kHidden, kHidden, F->hid, (float*)nullptr, g, B, 1);
-        hipLaunchKernelGGL(k_flow_conv<kHidden>, dim3((w2n + 3) / 4), dim3(256), 0, F->stream, F->hid, kHidden, F->w2 + l * kW2,
-                           F->b2 + l * kOut, kOut, (uint16_t*)nullptr, F->prm, g, B, 0);
-        hipLaunchKernelGGL(k_flow_couple, dim3(nb), dim3(256), 0, F->stream, F->links, F->prm, F->logj, g, B, mu, par,
-                           F->d.bins, inverse ? 1 : 0);
+        with_mu(mu, [&](auto m) {
+            hipLaunchKernelGGL(k_flow_features<decltype(m)::value>, site_grid(n), site_block(n), 0, F->stream, F->links,
+                               F->feat, g, B, par);
+        });
+        conditioner(F, l, n, F->stream);
+        with_mu_bins(mu, F->d.bins, [&](auto m, auto k) {
+            hipLaunchKernelGGL((k_flow_couple<decltype(m)::value, decltype(k)::value>), site_grid(n), site_block(n), 0,
+                               F->stream, F->links, F->prm, F->logj, g, B, par, inverse ? 1 : 0);
+        });
     }
     FCHK(hipGetLastError());
     return QCD_OK;
@@ -851,11 +1212,14 @@ int qcd_flow_create(const qcd_flow_desc* desc, qcd_flow** out)
     if (V * (uint64_t)d.max_batch > (1ull << 26)) return err(QCD_E_ARG, "max_batch x sites above 2^26");
     qcd_flow* F = new qcd_flow();
     F->d = d;
-    F->g = FGeom{d.n[0], d.n[1], d.n[2], d.n[3], (uint32_t)V};
+    F->g = FGeom{d.n[0], d.n[1], d.n[2], d.n[3], (uint32_t)V, qcd::make_fastdiv((uint32_t)d.n[1]),
+                 qcd::make_fastdiv((uint32_t)d.n[2]), qcd::make_fastdiv((uint32_t)d.n[3]), qcd::make_fastdiv((uint32_t)V)};
     F->nparam = kLayerParams * (size_t)d.layers;
     const size_t n = V * (size_t)d.max_batch;
     bool ok = hipStreamCreateWithFlags(&F->stream, hipStreamNonBlocking) == hipSuccess;
-    ok = ok && hipMalloc((void**)&F->w1, sizeof(uint16_t) * kW1 * d.layers) == hipSuccess;
+    ok = ok && hipMalloc((void**)&F->w1, sizeof(uint16_t) * kW1Pack * d.layers) == hipSuccess;
+    ok = ok && hipMemset(F->w1, 0, sizeof(uint16_t) * kW1Pack * d.layers) == hipSuccess;   // the padded k
+    ok = ok && hipMalloc((void**)&F->staged, sizeof(float) * F->nparam) == hipSuccess;
     ok = ok && hipMalloc((void**)&F->b1, sizeof(float) * kHidden * d.layers) == hipSuccess;
     ok = ok && hipMalloc((void**)&F->w2, sizeof(uint16_t) * kW2 * d.layers) == hipSuccess;
     ok = ok && hipMalloc((void**)&F->b2, sizeof(float) * kOut * d.layers) == hipSuccess;
@@ -881,6 +1245,7 @@ int qcd_flow_destroy(qcd_flow* F)
     if (!F) return QCD_OK;
     if (F->stream) (void)hipStreamSynchronize(F->stream);
     (void)hipFree(F->w1);
+    (void)hipFree(F->staged);
     (void)hipFree(F->b1);
     (void)hipFree(F->w2);
     (void)hipFree(F->b2);
@@ -912,20 +1277,12 @@ int qcd_flow_set_params(qcd_flow* F, const float* p, size_t n)
 {
     if (!F || !p) return err(QCD_E_ARG, "null argument");
     if (n != F->nparam) return err(QCD_E_ARG, "expected " + std::to_string(F->nparam) + " parameters, got " + std::to_string(n));
-    const int Ln = F->d.layers;
-    std::vector<uint16_t> w1(kW1 * Ln), w2(kW2 * Ln);
-    std::vector<float> b1(kHidden * Ln), b2(kOut * Ln);
-    for (int l = 0; l < Ln; ++l) {
-        const float* q = p + l * kLayerParams;
-        for (size_t i = 0; i < kW1; ++i) w1[l * kW1 + i] = f2bf(q[i]);
-        for (int i = 0; i < kHidden; ++i) b1[l * kHidden + i] = q[kW1 + i];
-        for (size_t i = 0; i < kW2; ++i) w2[l * kW2 + i] = f2bf(q[kW1 + kHidden + i]);
-        for (int i = 0; i < kOut; ++i) b2[l * kOut + i] = q[kW1 + kHidden + kW2 + i];
-    }
-    FCHK(hipMemcpy(F->w1, w1.data(), sizeof(uint16_t) * w1.size(), hipMemcpyHostToDevice));
-    FCHK(hipMemcpy(F->w2, w2.data(), sizeof(uint16_t) * w2.size(), hipMemcpyHostToDevice));
-    FCHK(hipMemcpy(F->b1, b1.data(), sizeof(float) * b1.size(), hipMemcpyHostToDevice));
-    FCHK(hipMemcpy(F->b2, b2.data(), sizeof(float) * b2.size(), hipMemcpyHostToDevice));
+    // uploaded as they are; the device makes the BF16 operand orders
+    FCHK(hipMemcpyAsync(F->staged, p, sizeof(float) * n, hipMemcpyHostToDevice, F->stream));
+    hipLaunchKernelGGL(k_flow_unpack_params, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, F->stream,
+                       (const float*)F->staged, (uint32_t)F->d.layers, F->w1, F->b1, F->w2, F->b2);
+    FCHK(hipGetLastError());
+    FCHK(hipStreamSynchronize(F->stream));
     F->host_params.assign(p, p + n);
     F->host_stale = false;
     if (F->tp) {   // training continues from these parameters, fresh moments
@@ -979,17 +1336,18 @@ int imh_sweep(qcd_flow* F, qcd_lattice* lat, unsigned long long seed, int mode, 
     if ((rc = qcdhip::su2_quats(lat, F->links, true, &st))) return rc;   // the lattice's stream from here on
     hipLaunchKernelGGL(k_flow_imh_key, dim3(1), dim3(64), 0, st, F->imh, seed, mode);
     const FGeom g = F->g;
-    const uint32_t nb = (g.V + 255) / 256;
-    const uint32_t w1n = (g.V / 16) * (kHidden / 16), w2n = (g.V / 16) * (kOut / 16);
     for (int l = 0; l < F->d.layers; ++l) {
         const int mu = l % 4, par = (l / 4) % 2;
-        hipLaunchKernelGGL(k_flow_features, dim3(nb), dim3(256), 0, st, F->links, F->feat, g, 1u, mu, par);
-        hipLaunchKernelGGL(k_flow_conv<kCin0>, dim3((w1n + 3) / 4), dim3(256), 0, st, F->feat, kCin0, F->w1 + l * kW1,
-                           F->b1 + l * kHidden, kHidden, F->hid, (float*)nullptr, g, 1u, 1);
-        hipLaunchKernelGGL(k_flow_conv<kHidden>, dim3((w2n + 3) / 4), dim3(256), 0, st, F->hid, kHidden, F->w2 + l * kW2,
-                           F->b2 + l * kOut, kOut, (uint16_t*)nullptr, F->prm, g, 1u, 0);
-        hipLaunchKernelGGL(k_flow_imh_couple, dim3(nb), dim3(256), 0, st, F->links, F->prm, g, mu, par, F->d.bins,
-                           (float)beta, ((uint64_t)l + 1) * 0xD1B54A32D192ED03ull, F->imh);
+        with_mu(mu, [&](auto m) {
+            hipLaunchKernelGGL(k_flow_features<decltype(m)::value>, site_grid(g.V), site_block(g.V), 0, st, F->links, F->feat,
+                               g, 1u, par);
+        });
+        conditioner(F, l, g.V, st);
+        with_mu_bins(mu, F->d.bins, [&](auto m, auto k) {
+            hipLaunchKernelGGL((k_flow_imh_couple<decltype(m)::value, decltype(k)::value>), site_grid(g.V), site_block(g.V),
+                               0, st, F->links, F->prm, g, par, (float)beta, ((uint64_t)l + 1) * 0xD1B54A32D192ED03ull,
+                               F->imh);
+        });
     }
     FCHK(hipGetLastError());
     return qcdhip::su2_quats(lat, F->links, false, nullptr);
@@ -1056,20 +1414,21 @@ int train_grad(qcd_flow* F, const float* links, int batch, double* loss)
     }
     const uint64_t nl = (uint64_t)B * 4 * g.V;
     FCHK(hipMemcpyAsync(F->links, links, sizeof(float4) * nl, hipMemcpyHostToDevice, F->stream));
-    const uint32_t w1n = (R / 16) * (kHidden / 16), w2n = (R / 16) * (kOut / 16);
     const uint32_t nchunk = (R + kChunk - 1) / kChunk;
     for (int l = 0; l < F->d.layers; ++l) {
         const int mu = l % 4, par = (l / 4) % 2;
         float* gl = F->tgrad + (size_t)l * kLayerParams;   // W1, b1, W2, b2 of layer l
         // forward of the conditioner on the data configurations
-        hipLaunchKernelGGL(k_flow_features, dim3(nb), dim3(256), 0, F->stream, F->links, F->feat, g, B, mu, par);
-        hipLaunchKernelGGL(k_flow_conv<kCin0>, dim3((w1n + 3) / 4), dim3(256), 0, F->stream, F->feat, kCin0, F->w1 + l * kW1,
-                           F->b1 + l * kHidden, kHidden, F->hid, (float*)nullptr, g, B, 1);
-        hipLaunchKernelGGL(k_flow_conv<kHidden>, dim3((w2n + 3) / 4), dim3(256), 0, F->stream, F->hid, kHidden, F->w2 + l * kW2,
-                           F->b2 + l * kOut, kOut, (uint16_t*)nullptr, F->prm, g, B, 0);
+        with_mu(mu, [&](auto m) {
+            hipLaunchKernelGGL(k_flow_features<decltype(m)::value>, site_grid(R), site_block(R), 0, F->stream, F->links,
+                               F->feat, g, B, par);
+        });
+        conditioner(F, l, R, F->stream);
         // -log q_a and its gradient with respect to the spline parameters
-        hipLaunchKernelGGL(k_flow_nll_grad, dim3(nb), dim3(256), 0, F->stream, (const float4*)F->links, F->prm, F->tg,
-                           F->tloss, g, B, mu, par, F->d.bins);
+        with_mu(mu, [&](auto m) {
+            hipLaunchKernelGGL(k_flow_nll_grad<decltype(m)::value>, dim3(nb), dim3(256), 0, F->stream,
+                               (const float4*)F->links, F->prm, F->tg, F->tloss, g, B, par, F->d.bins);
+        });
         hipLaunchKernelGGL((k_flow_rowsum<float>), dim3(B), dim3(256), 0, F->stream, F->tloss, g.V,
                            F->tsums + (size_t)l * F->d.max_batch);
         // conv2: weight and bias gradients, then the hidden gradient through the transposed convolution
@@ -1085,10 +1444,7 @@ int train_grad(qcd_flow* F, const float* links, int batch, double* loss)
             const uint32_t nt = (uint32_t)(kHidden * kStencil * kOut);
             hipLaunchKernelGGL(k_flow_w2_transpose, dim3((nt + 255) / 256), dim3(256), 0, F->stream,
                                (const uint16_t*)(F->w2 + l * kW2), F->tw2t);
-            const uint32_t wtn = (R / 16) * (kHidden / 16);
-            hipLaunchKernelGGL(k_flow_conv<kOut>, dim3((wtn + 3) / 4), dim3(256), 0, F->stream, (const uint16_t*)F->tg, kOut,
-                               (const uint16_t*)F->tw2t, (const float*)F->tzero, kHidden, (uint16_t*)nullptr, F->tdhid,
-                               g, B, 0);
+            launch_conv<kOut, false>(F->tg, F->tw2t, F->tzero, nullptr, F->tdhid, g, R, F->stream);
             hipLaunchKernelGGL(k_flow_tanh_back, dim3((R * kHidden + 255) / 256), dim3(256), 0, F->stream,
                                (const float*)F->tdhid, (const uint16_t*)F->hid, F->tdpre, R * (uint32_t)kHidden);
         }
