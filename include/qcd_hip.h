@@ -593,7 +593,7 @@ int  qcd_flow_imh_seed(qcd_flow *flow, unsigned long long seed);
    the sample / evaluate layout) -- for every coupling layer, the sum over
    its active links of -log q_a(U_a | frozen links) on the data itself, the
    density the learned Metropolis sweep proposes with -- and its gradient:
-   the spline part by central differences in double precision, then conv2,
+   the spline part in closed form in double precision, then conv2,
    tanh and conv1 backwards (weight gradients as MFMA GEMMs over the sites,
    the hidden gradient as the transposed stencil convolution).
    qcd_flow_train_grad returns the loss per configuration and the gradient

@@ -62,6 +62,9 @@ constexpr float kMinW = 1e-3f, kMinD = 1e-3f;
 
 typedef short s4 __attribute__((ext_vector_type(4)));
 typedef float f4 __attribute__((ext_vector_type(4)));
+typedef short s8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
+__device__ __forceinline__ bf8 as_bf(s8 v) { return __builtin_bit_cast(bf8, v); }
 
 struct FGeom {
     int n1, n2, n3, n4;   // extents along x, y, z, t
@@ -295,14 +298,31 @@ template <int CIN> struct ConvOp {
     typedef short V __attribute__((ext_vector_type(4 * per)));
 };
 
+// What becomes of output n of a row: the hidden layer (tanh, BF16 at
+// hid_pos), the spline parameters (FP32), or, given the hidden layer h, the
+// gradient before its tanh (v (1 - h^2), BF16).
+enum ConvOut { CONV_TANH, CONV_RAW, CONV_TANH_BACK };
+template <int ACT, int COUT>
+__device__ __forceinline__ void conv_store(float v, size_t r, int n, const uint16_t* h, uint16_t* out_bf, float* out_f)
+{
+    if constexpr (ACT == CONV_TANH) {
+        out_bf[r * COUT + hid_pos(n)] = f2bf(tanhf(v));
+    } else if constexpr (ACT == CONV_RAW) {
+        out_f[r * COUT + n] = v;
+    } else {
+        const float hv = bf2f(h[r * COUT + hid_pos(n)]);
+        out_bf[r * COUT + n] = f2bf(v * (1.f - hv * hv));
+    }
+}
+
 // One wavefront: MT tiles of 16 sites x NT tiles of 16 output channels.
-// in[row * CIN + channel] (BF16), out: tanh -> BF16 at hid_pos (ACT) or FP32
-// [row * cout + n].  The loads of BS operand steps are issued before the
-// matrix instructions of the previous BS, which run in k order whatever the
-// shape, so every shape gives the same sums.
-template <int CIN, int MT, int NT, int BS, bool ACT>
+// in[row * CIN + channel] (BF16); outputs as conv_store.  The loads of BS
+// operand steps are issued before the matrix instructions of the previous BS,
+// which run in k order whatever the shape, so every shape gives the same sums.
+template <int CIN, int MT, int NT, int BS, int ACT>
 __global__ __launch_bounds__(256) void k_flow_conv(const uint16_t* in, const uint16_t* wt, const float* bias,
-                                                   uint16_t* out_bf, float* out_f, FGeom g, uint32_t ntile_m)
+                                                   const uint16_t* h, uint16_t* out_bf, float* out_f, FGeom g,
+                                                   uint32_t ntile_m)
 {
     using Op = ConvOp<CIN>;
     using V = typename Op::V;
@@ -400,8 +420,7 @@ __global__ __launch_bounds__(256) void k_flow_conv(const uint16_t* in, const uin
             for (int i = 0; i < 4; ++i) {
                 const size_t r = (size_t)(tm * MT + m) * 16 + 4 * q + i;
                 const float v = acc[m][t][i] + bs;
-                if constexpr (ACT) out_bf[r * COUT + hid_pos(ncol)] = f2bf(tanhf(v));
-                else out_f[r * COUT + ncol] = v;
+                conv_store<ACT, COUT>(v, r, ncol, h, out_bf, out_f);
             }
         }
     }
@@ -411,9 +430,10 @@ __global__ __launch_bounds__(256) void k_flow_conv(const uint16_t* in, const uin
 // x-plane of a configuration stages the plane and its two neighbours (`plane`
 // sites each, contiguous) and every one of the 81 gathers of a site reads
 // from there.  A wavefront takes MT tiles of 16 sites at a time.
-template <int CIN, int MT, int BS, int WV, bool ACT>
+template <int CIN, int MT, int BS, int WV, int ACT>
 __global__ __launch_bounds__(64 * WV) void k_flow_conv_plane(const uint16_t* in, const uint16_t* wt, const float* bias,
-                                                         uint16_t* out_bf, float* out_f, FGeom g, uint32_t plane)
+                                                             const uint16_t* h, uint16_t* out_bf, float* out_f, FGeom g,
+                                                             uint32_t plane)
 {
     using Op = ConvOp<CIN>;
     using V = typename Op::V;
@@ -513,8 +533,7 @@ __global__ __launch_bounds__(64 * WV) void k_flow_conv_plane(const uint16_t* in,
                 for (int i = 0; i < 4; ++i) {
                     const size_t r = (size_t)blockIdx.x * plane + (size_t)(t0 + m) * 16 + 4 * q + i;
                     const float v = acc[m][t][i] + bs;
-                    if constexpr (ACT) out_bf[r * COUT + hid_pos(ncol)] = f2bf(tanhf(v));
-                    else out_f[r * COUT + ncol] = v;
+                    conv_store<ACT, COUT>(v, r, ncol, h, out_bf, out_f);
                 }
             }
         }
@@ -529,25 +548,30 @@ __global__ __launch_bounds__(64 * WV) void k_flow_conv_plane(const uint16_t* in,
 //   16 (128 planes)                 16.6                             12.6
 //   64 (512 planes)                 45.7 with four tiles             25.1, with 8 wavefronts 29.3
 // The matrix instructions of 64 configurations take 8.6 us.
-template <int CIN, bool ACT>
-void launch_conv(const uint16_t* in, const uint16_t* wt, const float* bias, uint16_t* out_bf, float* out_f, const FGeom& g,
-                 uint32_t rows, hipStream_t st)
+// 16 -> 32 channels (backward) has twice the weights to read per input byte:
+// 16 configurations 21.4 us as one tile per wavefront, 46.7 in planes (it has
+// no such kernel); 64: 56 with four tiles, 76 with one, 78 in planes.
+template <int CIN, int ACT>
+void launch_conv(const uint16_t* in, const uint16_t* wt, const float* bias, const uint16_t* h, uint16_t* out_bf, float* out_f,
+                 const FGeom& g, uint32_t rows, hipStream_t st)
 {
-    constexpr int NTT = ConvOp<CIN>::ntiles, BS = CIN == 16 ? 3 : 6;   // 16 channels: 6 would spill
+    constexpr int NTT = ConvOp<CIN>::ntiles;
     const uint32_t tiles = rows / 16, plane = g.V / (uint32_t)g.n1, planes = rows / plane, lds = 3u * plane * 2u * CIN;
-    if (plane % 16 == 0 && lds <= 64u * 1024u && planes >= 96u) {
-        if (planes <= 256u)
-            hipLaunchKernelGGL((k_flow_conv_plane<CIN, 2, BS, 8, ACT>), dim3(planes), dim3(512), lds, st, in, wt, bias,
-                               out_bf, out_f, g, plane);
-        else
-            hipLaunchKernelGGL((k_flow_conv_plane<CIN, 2, BS, 4, ACT>), dim3(planes), dim3(256), lds, st, in, wt, bias,
-                               out_bf, out_f, g, plane);
+    if (CIN != 16 && plane % 16 == 0 && lds <= 64u * 1024u && planes >= 96u) {
+        if constexpr (CIN != 16) {
+            if (planes <= 256u)
+                hipLaunchKernelGGL((k_flow_conv_plane<CIN, 2, 6, 8, ACT>), dim3(planes), dim3(512), lds, st, in, wt, bias, h,
+                                   out_bf, out_f, g, plane);
+            else
+                hipLaunchKernelGGL((k_flow_conv_plane<CIN, 2, 6, 4, ACT>), dim3(planes), dim3(256), lds, st, in, wt, bias, h,
+                                   out_bf, out_f, g, plane);
+        }
     } else if (tiles <= 4096u) {
-        hipLaunchKernelGGL((k_flow_conv<CIN, 1, 1, 9, ACT>), dim3(tiles * NTT), dim3(64), 0, st, in, wt, bias, out_bf,
-                           out_f, g, tiles);
+        hipLaunchKernelGGL((k_flow_conv<CIN, 1, 1, 9, ACT>), dim3(tiles * NTT), dim3(64), 0, st, in, wt, bias, h,
+                           out_bf, out_f, g, tiles);
     } else {
         hipLaunchKernelGGL((k_flow_conv<CIN, 4, NTT, 3, ACT>), dim3((tiles + 15) / 16), dim3(256), 0, st, in, wt, bias,
-                           out_bf, out_f, g, tiles);
+                           h, out_bf, out_f, g, tiles);
     }
 }
 
@@ -800,59 +824,114 @@ __global__ __launch_bounds__(256) void k_flow_imh_couple(float4* L, const float*
 // configuration itself, so a layer's loss depends on its own parameters
 // only, and the gradient flows back through conv2, tanh and conv1 alone.
 
-// -log q_a of one active link in double precision (the map of
-// make_spline / spline_inv / log_jac, written for double): theta = angle of
-// U V, r = the 3K + 1 raw spline parameters.
-__device__ double nll_link(const double* r, int K, double th)
+// -log q_a of one active link in double precision (the map of make_spline /
+// spline_inv / log_jac, written for double) and its gradient gr with respect to
+// the 3K + 1 raw spline parameters r; th = angle of U V.  In the bin of th with
+// corners (x0, y0), sizes (w, h), slope s = h / w and end derivatives d0, d1
+// the inverse xi solves y0 + h A / den = th, and
+//   nll = log f' + 2 log(sin th / sin(x0 + xi w)),  f' = s^2 N / den^2,
+// so a parameter p moves it by its direct derivative plus, through xi,
+// -(dy/dp) / (w f') times the derivative in xi.  (Differences of nll at r +- h
+// were 27 evaluations per link: 231 us for 32768 sites, now 8 us.)
+template <int K> __device__ __forceinline__ double nll_grad_link(const float (&rf)[kOut], double th, float (&gr)[kOut])
 {
-    const double pi = 3.14159265358979323846;
-    double mw = r[0], mh = r[K];
+    const double pi = 3.14159265358979323846, ln2i = 1.4426950408889634;
+    double mw = rf[0], mh = rf[K];
+#pragma unroll
     for (int i = 1; i < K; ++i) {
-        mw = fmax(mw, r[i]);
-        mh = fmax(mh, r[K + i]);
+        mw = fmax(mw, (double)rf[i]);
+        mh = fmax(mh, (double)rf[K + i]);
     }
-    double ew[kMaxBins], eh[kMaxBins], sw = 0.0, sh = 0.0;
+    double pw[K], ph[K], sw = 0.0, sh = 0.0;
+#pragma unroll
     for (int i = 0; i < K; ++i) {
-        ew[i] = exp(r[i] - mw);
-        eh[i] = exp(r[K + i] - mh);
-        sw += ew[i];
-        sh += eh[i];
+        pw[i] = exp((double)rf[i] - mw);
+        ph[i] = exp((double)rf[K + i] - mh);
+        sw += pw[i];
+        sh += ph[i];
     }
-    double xk[kMaxBins + 1], yk[kMaxBins + 1], d[kMaxBins + 1];
-    xk[0] = yk[0] = 0.0;
+#pragma unroll
     for (int i = 0; i < K; ++i) {
-        xk[i + 1] = xk[i] + pi * (kMinW + (1.0 - K * kMinW) * ew[i] / sw);
-        yk[i + 1] = yk[i] + pi * (kMinW + (1.0 - K * kMinW) * eh[i] / sh);
+        pw[i] /= sw;
+        ph[i] /= sh;
     }
-    xk[K] = yk[K] = pi;
-    for (int i = 0; i <= K; ++i) {
-        const double x = r[2 * K + i];
-        d[i] = kMinD + (1.0 - kMinD) * (x > 30.0 ? x : log1p(exp(x))) * 1.4426950408889634;
+    const double scale = pi * (1.0 - K * (double)kMinW);
+    // the bin of th among the heights' knots, and its corners
+    double x0 = 0.0, y0 = 0.0, w = 0.0, h = 0.0, xa = 0.0, ya = 0.0;
+    float r0 = rf[2 * K], r1 = rf[2 * K + 1];
+    int bin = 0;
+    bool go = true;
+#pragma unroll
+    for (int i = 0; i < K; ++i) {
+        const double xb = i == K - 1 ? pi : xa + pi * (double)kMinW + scale * pw[i];
+        const double yb = i == K - 1 ? pi : ya + pi * (double)kMinW + scale * ph[i];
+        if (i > 0) go = go && th >= ya;
+        if (go) {
+            bin = i;
+            x0 = xa;
+            y0 = ya;
+            w = xb - xa;
+            h = yb - ya;
+            r0 = rf[2 * K + i];
+            r1 = rf[2 * K + i + 1];
+        }
+        xa = xb;
+        ya = yb;
     }
-    int k = 0;
-    while (k < K - 1 && th >= yk[k + 1]) ++k;
-    const double w = xk[k + 1] - xk[k], h = yk[k + 1] - yk[k], sl = h / w;
-    const double dy = th - yk[k], dd = d[k + 1] + d[k] - 2.0 * sl;
-    const double a = h * (sl - d[k]) + dy * dd, bq = h * d[k] - dy * dd, cq = -sl * dy;
+    auto sp = [&](double x) { return x > 30.0 ? x : log1p(exp(x)); };
+    auto sg = [&](double x) { return x > 30.0 ? 1.0 : 1.0 / (1.0 + exp(-x)); };
+    const double dk = (1.0 - (double)kMinD) * ln2i;
+    const double d0 = (double)kMinD + dk * sp((double)r0), d1 = (double)kMinD + dk * sp((double)r1);
+    const double s = h / w, dy = th - y0, dd = d1 + d0 - 2.0 * s;
+    const double a = h * (s - d0) + dy * dd, bq = h * d0 - dy * dd, cq = -s * dy;
     const double disc = fmax(bq * bq - 4.0 * a * cq, 0.0);
     const double xi = fmin(fmax(2.0 * cq / (-bq - sqrt(disc)), 0.0), 1.0), om = 1.0 - xi;
-    const double den = sl + dd * xi * om;
-    const double num = sl * sl * (d[k + 1] * xi * xi + 2.0 * sl * xi * om + d[k] * om * om);
-    const double dlog = log(num) - 2.0 * log(den);
-    const double thz = xk[k] + xi * w;
-    const double si = sin(thz), so = sin(th);
-    const double ratio = (si > 1e-9 && so > 1e-9) ? so / si : exp(dlog);
-    return dlog + 2.0 * log(ratio);
+    const double xo = xi * om;
+    const double den = s + dd * xo, N = d1 * xi * xi + 2.0 * s * xo + d0 * om * om, A = s * xi * xi + d0 * xo;
+    const double iden = 1.0 / den, iN = 1.0 / N;
+    const double dlog = log(s * s * N) - 2.0 * log(den);
+    const double thz = x0 + xi * w, si = sin(thz), so = sin(th);
+    const bool pole = !(si > 1e-9 && so > 1e-9);   // there the ratio's limit f' stands for sin th / sin thz
+    const double nll = pole ? 3.0 * dlog : dlog + 2.0 * log(so / si);
+    const double c1 = pole ? 3.0 : 1.0, cot = pole ? 0.0 : cos(thz) / si;
+    // direct derivatives of log f' and of y = y0 + h A / den
+    const double den_s = 1.0 - 2.0 * xo;
+    const double l_s = 2.0 / s + 2.0 * xo * iN - 2.0 * den_s * iden;
+    const double l_d0 = om * om * iN - 2.0 * xo * iden, l_d1 = xi * xi * iN - 2.0 * xo * iden;
+    const double l_xi = (2.0 * d1 * xi + 2.0 * s * (1.0 - 2.0 * xi) - 2.0 * d0 * om) * iN - 2.0 * dd * (1.0 - 2.0 * xi) * iden;
+    const double y_s = h * (xi * xi * den - A * den_s) * iden * iden;
+    const double y_d0 = h * xo * (den - A) * iden * iden, y_d1 = -h * A * xo * iden * iden;
+    const double y_h = A * iden + y_s / w, y_w = -y_s * s / w;
+    // d nll / d xi over dy / d xi = w f'
+    const double f1 = s * s * N * iden * iden, q = (c1 * l_xi - 2.0 * cot * w) / (w * f1);
+    const double g_x0 = -2.0 * cot, g_w = -c1 * l_s * s / w - 2.0 * cot * xi - q * y_w;
+    const double g_y0 = -q, g_h = c1 * l_s / w - q * y_h;
+    const double g_d0 = c1 * l_d0 - q * y_d0, g_d1 = c1 * l_d1 - q * y_d1;
+    // softmax: x0 is the sum of the widths below the bin
+    double mwg = 0.0, mhg = 0.0;
+#pragma unroll
+    for (int i = 0; i < K; ++i) {
+        mwg += pw[i] * (i < bin ? g_x0 : (i == bin ? g_w : 0.0));
+        mhg += ph[i] * (i < bin ? g_y0 : (i == bin ? g_h : 0.0));
+    }
+#pragma unroll
+    for (int i = 0; i < K; ++i) {
+        gr[i] = (float)(scale * pw[i] * ((i < bin ? g_x0 : (i == bin ? g_w : 0.0)) - mwg));
+        gr[K + i] = (float)(scale * ph[i] * ((i < bin ? g_y0 : (i == bin ? g_h : 0.0)) - mhg));
+    }
+#pragma unroll
+    for (int i = 0; i <= K; ++i)
+        gr[2 * K + i] = i == bin ? (float)(g_d0 * dk * sg((double)r0)) : (i == bin + 1 ? (float)(g_d1 * dk * sg((double)r1)) : 0.f);
+    return nll;
 }
 
 // Per site of a batch: at active sites, -log q_a and its gradient with
-// respect to the raw spline parameters (central differences in double
-// precision, step 1e-5; the map is smooth except at bin edges, a set of
-// measure zero) into g (BF16, [row][16], zero at inactive sites and for
-// the unused channels); loss[row] = -log q_a (0 at inactive sites).
-template <int mu>
-__global__ void k_flow_nll_grad(const float4* L, const float* prm, uint16_t* g, float* loss, FGeom g4, uint32_t B,
-                                int par, int K)
+// respect to the raw spline parameters into g (BF16, [row][16], zero at
+// inactive sites and for the unused channels); loss[row] = -log q_a (0 at
+// inactive sites).
+template <int mu, int K>
+__global__ __launch_bounds__(256) void k_flow_nll_grad(const float4* L, const float* prm, uint16_t* g, float* loss, FGeom g4,
+                                                       uint32_t B, int par)
 {
     const uint32_t j = blockIdx.x * blockDim.x + threadIdx.x;
     if (j >= B * g4.V) return;
@@ -860,35 +939,193 @@ __global__ void k_flow_nll_grad(const float4* L, const float* prm, uint16_t* g, 
     int c[4];
     coords(g4, s, c);
     float gr[kOut];
+#pragma unroll
     for (int q = 0; q < kOut; ++q) gr[q] = 0.f;
     float lo = 0.f;
     if (is_active(c, mu, par)) {
         StapleLinks sl;
         load_staple<mu>(sl, L, g4, b, c);
+        const float4 U = L[((size_t)b * 4 + mu) * g4.V + s];
+        float raw[kOut];
+        load_raw(raw, prm, j);
+        loads_issued();
         const float4 A = staple_sum(sl);
         const float k = sqrtf(A.x * A.x + A.y * A.y + A.z * A.z + A.w * A.w);
         if (k > 1e-20f) {
             const float ik = 1.f / k;
-            const float4 W = qmul(L[((size_t)b * 4 + mu) * g4.V + s], make_float4(A.x * ik, A.y * ik, A.z * ik, A.w * ik));
+            const float4 W = qmul(U, make_float4(A.x * ik, A.y * ik, A.z * ik, A.w * ik));
             const double th = atan2((double)sqrtf(W.y * W.y + W.z * W.z + W.w * W.w), (double)W.x);
-            double r[3 * kMaxBins + 1];
-            const int np = 3 * K + 1;
-            for (int q = 0; q < np; ++q) r[q] = (double)prm[(size_t)j * kOut + q];
-            lo = (float)nll_link(r, K, th);
-            const double hstep = 1e-5;
-            for (int q = 0; q < np; ++q) {
-                const double r0 = r[q];
-                r[q] = r0 + hstep;
-                const double up = nll_link(r, K, th);
-                r[q] = r0 - hstep;
-                const double dn = nll_link(r, K, th);
-                r[q] = r0;
-                gr[q] = (float)((up - dn) / (2.0 * hstep));
-            }
+            lo = (float)nll_grad_link<K>(raw, th, gr);
         }
     }
     loss[j] = lo;
-    for (int q = 0; q < kOut; ++q) g[(size_t)j * kOut + q] = f2bf(gr[q]);
+    uint4* o = reinterpret_cast<uint4*>(g) + 2 * (size_t)j;
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+        uint32_t v[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = f2bf(gr[8 * q + 2 * i]) | (uint32_t)f2bf(gr[8 * q + 2 * i + 1]) << 16;
+        o[q] = make_uint4(v[0], v[1], v[2], v[3]);
+    }
+}
+
+// Weight and bias gradients from x-planes in LDS: dW[n][st * C + ch] = sum over
+// rows r of gout[r][n] X[r + st][ch] and db[n] = sum of gout[r][n], as
+// v_mfma_f32_16x16x32_bf16 tiles with 32 rows (sites) per step.  Both operands
+// run along the rows, so they are read transposed (ds_read_b64_tr_b16: lane l
+// of 16 gives the address of columns 4 (l % 4) .. + 3 of row l / 4 and gets
+// column l of the four rows), at any stencil offset.  One workgroup of 8
+// wavefronts stages three planes of X and its rows of the plane of gout; `segs`
+// workgroups share a plane's rows.  Wavefront w takes the offsets (oy, oz, ot) =
+// w, w + 8, .. with all three ox, and goes on to further units with the same
+// sums; one partial array per workgroup.
+// For 16 configurations of 8^3 x 4 (128 planes): 32 -> 16 channels 15 us, 8 ->
+// 32 channels 9 us, against 240 and 142 us of k_flow_wgrad, whose every operand
+// element is a load; 23 and 19 with one workgroup per plane and 16-row steps.
+// The matrix instructions take 2.6 us of the 15, the transposed reads 6 (25 of
+// 512 bytes per wavefront and 16 rows).
+constexpr int kGradWaves = 8, kGradOffs = 4;   // 27 offsets over 8 wavefronts
+constexpr uint32_t kGradRows = 32;
+template <int C, int N>
+__global__ __launch_bounds__(64 * kGradWaves) void k_flow_wgrad_plane(const uint16_t* gout, const uint16_t* in, float* part,
+                                                                      FGeom g, uint32_t plane, uint32_t segs, uint32_t len,
+                                                                      uint32_t units)
+{
+    constexpr int CT = C == 32 ? 6 : 2, NT = N / 16;   // tiles of 16 columns per offset: 3 x 2 halves, or ox pairs
+    constexpr uint32_t BX = 2u * C, BG = 2u * N, K = kStencil * C;
+    extern __shared__ uint4 planes[];
+    const uint32_t w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int lane = threadIdx.x & 63, q = lane >> 4;
+    const uint32_t row4 = (uint32_t)(lane & 15) >> 2, chunk = (uint32_t)lane & 3u;
+    const uint32_t xv = plane * BX / 16u;
+    const char* sx = reinterpret_cast<const char*>(planes);
+    const char* sg = sx + 3u * plane * BX;
+    const int n[4] = {g.n1, g.n2, g.n3, g.n4};
+    typedef __attribute__((address_space(3))) s4 ls4;
+    auto tr = [&](const char* a) { return __builtin_amdgcn_ds_read_tr16_b64_v4i16((ls4*)a); };
+    // rows of 64 bytes: their halves change places every four rows, or the
+    // eight rows of half a wavefront would meet in half the banks
+    auto swz = [](uint32_t byte, uint32_t stride) { return stride == 64u ? byte ^ ((byte >> 3) & 32u) : byte; };
+    auto stage = [&](uint4* dst, const uint4* src, uint32_t nv, uint32_t stride) {
+#pragma unroll 2
+        for (uint32_t i = threadIdx.x; i < nv; i += 64u * kGradWaves) dst[swz(16u * i, stride) / 16u] = src[i];
+    };
+    f4 acc[kGradOffs][CT][NT], accb[NT];
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+        accb[t] = f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int i = 0; i < kGradOffs; ++i)
+#pragma unroll
+            for (int c = 0; c < CT; ++c) acc[i][c][t] = f4{0.f, 0.f, 0.f, 0.f};
+    }
+    for (uint32_t un = blockIdx.x; un < units; un += gridDim.x) {
+        const uint32_t pl = un / segs, first = (un - pl * segs) * len, last = min(first + len, plane);
+        const uint32_t b = pl / (uint32_t)g.n1, x = pl % (uint32_t)g.n1;
+        __syncthreads();   // the previous unit has been read
+#pragma unroll
+        for (int o = 0; o < 3; ++o)
+            stage(planes + o * xv, reinterpret_cast<const uint4*>(in) +
+                                       ((size_t)b * (uint32_t)g.n1 + (uint32_t)wrap((int)x + o - 1, g.n1)) * xv, xv, BX);
+        stage(planes + 3 * xv, reinterpret_cast<const uint4*>(gout + ((size_t)pl * plane + first) * N), (last - first) * BG / 16u,
+              BG);
+        __syncthreads();
+        for (uint32_t r0 = first; r0 < last; r0 += kGradRows) {
+            // two groups of 16 rows; a plane of an odd number of them ends in
+            // half a step, the other half zero in both operands
+            const bool two = r0 + 16u < last;
+            uint32_t yo[2][3], zo[2][3], to[2][3];
+            s8 a[NT];
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const uint32_t r = r0 + (two ? 16u * h : 0u) + 4u * (uint32_t)q + row4;
+                int c[4];
+                coords(g, r, c);
+#pragma unroll
+                for (int o = 0; o < 3; ++o) {
+                    yo[h][o] = (uint32_t)wrap(c[1] + o - 1, n[1]) * BX;
+                    zo[h][o] = (uint32_t)wrap(c[2] + o - 1, n[2]) * (uint32_t)n[1] * BX;
+                    to[h][o] = (uint32_t)wrap(c[3] + o - 1, n[3]) * (uint32_t)(n[1] * n[2]) * BX;
+                }
+#pragma unroll
+                for (int t = 0; t < NT; ++t) {
+                    const s4 v = tr(sg + swz((r - first) * BG + 32u * t + 8u * chunk, BG));
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) a[t][4 * h + j] = h == 0 || two ? v[j] : (short)0;
+                }
+            }
+            auto pick = [](const uint32_t (&v)[3], uint32_t i) { return i == 0 ? v[0] : (i == 1 ? v[1] : v[2]); };
+            s8 bv[2][CT];
+            auto issue = [&](int i) {
+                const uint32_t m = w + kGradWaves * i;
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    const uint32_t row = pick(yo[h], m / 9u) + pick(zo[h], (m / 3u) % 3u) + pick(to[h], m % 3u);
+#pragma unroll
+                    for (int t = 0; t < CT; ++t) {
+                        s4 v;
+                        if constexpr (C == 32)
+                            v = tr(sx + (uint32_t)(t >> 1) * plane * BX + swz(row + 32u * (t & 1) + 8u * chunk, BX));
+                        else
+                            v = tr(sx + (uint32_t)(t == 0 ? chunk >> 1 : 2) * plane * BX + row + 8u * (chunk & 1));
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) bv[i & 1][t][4 * h + j] = h == 0 || two ? v[j] : (short)0;
+                    }
+                }
+            };
+            issue(0);
+#pragma unroll
+            for (int i = 0; i < kGradOffs; ++i) {
+                if (i + 1 < kGradOffs && w + kGradWaves * (i + 1) < 27u) issue(i + 1);
+                if (w + kGradWaves * i >= 27u) break;   // uniform
+#pragma unroll
+                for (int t = 0; t < CT; ++t)
+#pragma unroll
+                    for (int u = 0; u < NT; ++u)
+                        acc[i][t][u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf(a[u]), as_bf(bv[i & 1][t]),
+                                                                               acc[i][t][u], 0, 0, 0);
+            }
+            if (w == kGradWaves - 1u) {   // three offsets only: the bias sums, times ones
+                s8 one;
+#pragma unroll
+                for (int j = 0; j < 8; ++j) one[j] = 0x3f80;
+#pragma unroll
+                for (int u = 0; u < NT; ++u)
+                    accb[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf(a[u]), as_bf(one), accb[u], 0, 0, 0);
+            }
+        }
+    }
+    // lane holds D[4 (lane / 16) + i][lane % 16]: rows are output channels
+    float* o = part + (size_t)blockIdx.x * (N * K + N);
+#pragma unroll
+    for (int i = 0; i < kGradOffs; ++i) {
+        const uint32_t m = w + kGradWaves * i;
+        if (m >= 27u) break;
+#pragma unroll
+        for (int t = 0; t < CT; ++t) {
+            const int col = lane & 15;
+            uint32_t ox, ch;
+            if constexpr (C == 32) {
+                ox = (uint32_t)t >> 1;
+                const int ps = 16 * (t & 1) + col;   // stored position -> channel (hid_pos)
+                ch = (uint32_t)(16 * ((ps >> 2) & 1) + 4 * (ps >> 3) + (ps & 3));
+            } else {
+                ox = t == 0 ? (uint32_t)col >> 3 : 2u;
+                ch = (uint32_t)col & 7u;
+                if (t == 1 && col >= 8) continue;
+            }
+            const uint32_t k = (27u * ox + m) * C + ch;
+#pragma unroll
+            for (int u = 0; u < NT; ++u)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) o[(size_t)(16 * u + 4 * q + e) * K + k] = acc[i][t][u][e];
+        }
+    }
+    if (w == kGradWaves - 1u && (lane & 15) == 0)
+#pragma unroll
+        for (int u = 0; u < NT; ++u)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) o[(size_t)N * K + 16 * u + 4 * q + e] = accb[u][e];
 }
 
 // Weight gradient dW[n][k] = sum over rows r of gout[r][n] X[r][k], X the
@@ -939,12 +1176,21 @@ __global__ __launch_bounds__(256) void k_flow_wgrad(const uint16_t* gout, int co
 }
 
 // out[i] = sum over the nchunk partial arrays (fixed order)
-__global__ void k_flow_sum_parts(const float* part, uint32_t nchunk, uint32_t n, float* out)
+__global__ __launch_bounds__(256) void k_flow_sum_parts(const float* __restrict__ part, uint32_t nchunk, uint32_t n,
+                                                        float* __restrict__ out)
 {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     float a = 0.f;
-    for (uint32_t c = 0; c < nchunk; ++c) a += part[(size_t)c * n + i];
+    uint32_t c = 0;
+    for (; c + 16 <= nchunk; c += 16) {
+        float v[16];
+#pragma unroll
+        for (int k = 0; k < 16; ++k) v[k] = part[(size_t)(c + k) * n + i];
+#pragma unroll
+        for (int k = 0; k < 16; ++k) a += v[k];
+    }
+    for (; c < nchunk; ++c) a += part[(size_t)c * n + i];
     out[i] = a;
 }
 
@@ -965,22 +1211,15 @@ __global__ __launch_bounds__(256) void k_flow_colsum(const uint16_t* gout, int c
 
 // transposed conv2 weights for the input gradient: entry (c, st * 16 + n) =
 // W2[n][(80 - st) * 32 + c] (the stencil point of offset -o)
-__global__ void k_flow_w2_transpose(const uint16_t* w2, uint16_t* wt)
+__global__ void k_flow_w2_transpose(const uint16_t* w2, uint16_t* wt)   // blockIdx.y: the layer
 {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    w2 += (size_t)blockIdx.y * (kHidden * kStencil * kOut);
+    wt += (size_t)blockIdx.y * (kHidden * kStencil * kOut);
     if (i >= (uint32_t)(kHidden * kStencil * kOut)) return;
     const uint32_t c = i / (kStencil * kOut), rest = i % (kStencil * kOut);
     const uint32_t st = rest / kOut, nn = rest % kOut;
     wt[w2t_pos((int)c, (int)rest)] = w2[w2_pos((int)nn, (int)((kStencil - 1 - st) * kHidden + c))];
-}
-
-// dpre = dhid (1 - h^2), h the tanh output (BF16)
-__global__ void k_flow_tanh_back(const float* dhid, const uint16_t* h, uint16_t* dpre, uint32_t n)
-{
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const float hv = bf2f(h[i - i % kHidden + hid_pos((int)(i % kHidden))]);
-    dpre[i] = f2bf(dhid[i] * (1.f - hv * hv));
 }
 
 // Adam (Kingma and Ba 2015) on the FP32 parameters, then the device copies
@@ -1076,10 +1315,9 @@ struct qcd_flow {
     float* tm = nullptr;        // Adam moments
     float* tv = nullptr;
     uint16_t* tg = nullptr;     // d loss / d spline parameters [max_batch * V][16] (BF16)
-    float* tdhid = nullptr;     // d loss / d hidden [max_batch * V][32]
     uint16_t* tdpre = nullptr;  // d loss / d pre-activation (BF16)
     float* tloss = nullptr;     // -log q_a per site
-    uint16_t* tw2t = nullptr;   // transposed conv2 weights of one layer
+    uint16_t* tw2t = nullptr;   // transposed conv2 weights, every layer
     float* tpart = nullptr;     // weight-gradient partial sums
     float* tzero = nullptr;     // zero bias of the transposed convolution
     double* tsums = nullptr;    // per layer and configuration loss
@@ -1133,8 +1371,8 @@ dim3 site_grid(uint32_t n) { return dim3((n + site_block(n).x - 1) / site_block(
 // Spline parameters (F->prm) of layer l from the features in F->feat.
 void conditioner(qcd_flow* F, int l, uint32_t rows, hipStream_t st)
 {
-    launch_conv<kCin0, true>(F->feat, F->w1 + l * kW1Pack, F->b1 + l * kHidden, F->hid, nullptr, F->g, rows, st);
-    launch_conv<kHidden, false>(F->hid, F->w2 + l * kW2, F->b2 + l * kOut, nullptr, F->prm, F->g, rows, st);
+    launch_conv<kCin0, CONV_TANH>(F->feat, F->w1 + l * kW1Pack, F->b1 + l * kHidden, nullptr, F->hid, nullptr, F->g, rows, st);
+    launch_conv<kHidden, CONV_RAW>(F->hid, F->w2 + l * kW2, F->b2 + l * kOut, nullptr, nullptr, F->prm, F->g, rows, st);
 }
 
 int run_layers(qcd_flow* F, uint32_t B, bool inverse)
@@ -1257,8 +1495,7 @@ int qcd_flow_destroy(qcd_flow* F)
     (void)hipFree(F->act);
     (void)hipFree(F->sums);
     (void)hipFree(F->imh);
-    for (void* q : {(void*)F->tp, (void*)F->tgrad, (void*)F->tm, (void*)F->tv, (void*)F->tg, (void*)F->tdhid,
-                    (void*)F->tdpre, (void*)F->tloss, (void*)F->tw2t, (void*)F->tpart, (void*)F->tzero,
+    for (void* q : {(void*)F->tp, (void*)F->tgrad, (void*)F->tm, (void*)F->tv, (void*)F->tg, (void*)F->tdpre, (void*)F->tloss, (void*)F->tw2t, (void*)F->tpart, (void*)F->tzero,
                     (void*)F->tsums})
         (void)hipFree(q);
     if (F->stream) (void)hipStreamDestroy(F->stream);
@@ -1386,11 +1623,21 @@ int train_grad(qcd_flow* F, const float* links, int batch, double* loss)
     int rc = check_batch(F, batch);
     if (rc) return rc;
     const FGeom g = F->g;
-    const uint32_t B = (uint32_t)batch, R = B * g.V, nb = (R + 255) / 256;
+    const uint32_t B = (uint32_t)batch, R = B * g.V;
     const size_t nmax = (size_t)F->d.max_batch * g.V;
-    constexpr uint32_t kChunk = 512;
-    const size_t nchunk_max = (nmax + kChunk - 1) / kChunk;
-    const size_t part_max = nchunk_max * std::max((size_t)kOut * kStencil * kHidden, (size_t)kHidden * 656);
+    // weight gradients from x-planes in LDS where those fit, one partial
+    // array per workgroup; else from chunks of rows
+    constexpr uint32_t kChunk = 512, kGradGroups = 256;   // one workgroup per CU
+    const uint32_t plane = g.V / (uint32_t)g.n1, lds2 = plane * (3u * 2 * kHidden + 2 * kOut),
+                   lds1 = plane * (3u * 2 * kCin0 + 2 * kHidden);
+    const bool by_plane = plane % 16 == 0 && lds2 <= 64u * 1024u;
+    // segments of a plane, a multiple of kGradRows rows each
+    auto seg_len = [&](uint32_t nplanes) {
+        const uint32_t steps = (plane + kGradRows - 1) / kGradRows, segs = std::clamp(kGradGroups / nplanes, 1u, steps);
+        return (steps + segs - 1) / segs * kGradRows;
+    };
+    const size_t nchunk_max = by_plane ? std::min<size_t>(kGradGroups, nmax / 16) : (nmax + kChunk - 1) / kChunk;
+    const size_t part_max = nchunk_max * (kW2 + kHidden);
     if (!F->tp) {   // first step: training buffers and the FP32 parameters from the host copy
         bool ok = true;
         ok = ok && hipMalloc((void**)&F->tp, sizeof(float) * F->nparam) == hipSuccess;
@@ -1398,10 +1645,9 @@ int train_grad(qcd_flow* F, const float* links, int batch, double* loss)
         ok = ok && hipMalloc((void**)&F->tm, sizeof(float) * F->nparam) == hipSuccess;
         ok = ok && hipMalloc((void**)&F->tv, sizeof(float) * F->nparam) == hipSuccess;
         ok = ok && hipMalloc((void**)&F->tg, sizeof(uint16_t) * kOut * nmax) == hipSuccess;
-        ok = ok && hipMalloc((void**)&F->tdhid, sizeof(float) * kHidden * nmax) == hipSuccess;
         ok = ok && hipMalloc((void**)&F->tdpre, sizeof(uint16_t) * kHidden * nmax) == hipSuccess;
         ok = ok && hipMalloc((void**)&F->tloss, sizeof(float) * nmax) == hipSuccess;
-        ok = ok && hipMalloc((void**)&F->tw2t, sizeof(uint16_t) * kHidden * kStencil * kOut) == hipSuccess;
+        ok = ok && hipMalloc((void**)&F->tw2t, sizeof(uint16_t) * kW2 * F->d.layers) == hipSuccess;
         ok = ok && hipMalloc((void**)&F->tpart, sizeof(float) * part_max) == hipSuccess;
         ok = ok && hipMalloc((void**)&F->tzero, sizeof(float) * kHidden) == hipSuccess;
         ok = ok && hipMalloc((void**)&F->tsums, sizeof(double) * F->d.layers * F->d.max_batch) == hipSuccess;
@@ -1414,7 +1660,32 @@ int train_grad(qcd_flow* F, const float* links, int batch, double* loss)
     }
     const uint64_t nl = (uint64_t)B * 4 * g.V;
     FCHK(hipMemcpyAsync(F->links, links, sizeof(float4) * nl, hipMemcpyHostToDevice, F->stream));
-    const uint32_t nchunk = (R + kChunk - 1) / kChunk;
+    const uint32_t nplanes = R / plane, nchunk = (R + kChunk - 1) / kChunk;
+    const uint32_t len = seg_len(nplanes), segs = (plane + len - 1) / len, groups = std::min(nplanes * segs, kGradGroups);
+    // dW and db of one convolution, gout [R][N] and its input [R][C], to gw
+    // (the bias follows the weights)
+    auto weight_grad = [&](auto cc, auto nn, const uint16_t* gout, const uint16_t* in, uint32_t lds, float* gw) {
+        constexpr int C = decltype(cc)::value, N = decltype(nn)::value, K = kStencil * C;
+        if (by_plane) {
+            hipLaunchKernelGGL((k_flow_wgrad_plane<C, N>), dim3(groups), dim3(64 * kGradWaves), lds, F->stream, gout, in,
+                               F->tpart, g, plane, segs, len, nplanes * segs);
+            const uint32_t n = N * K + N;
+            hipLaunchKernelGGL(k_flow_sum_parts, dim3((n + 255) / 256), dim3(256), 0, F->stream, (const float*)F->tpart,
+                               groups, n, gw);
+            return;
+        }
+        const uint32_t tiles = (uint32_t)((K + 15) / 16) * (N / 16) * nchunk;
+        hipLaunchKernelGGL(k_flow_wgrad, dim3((tiles + 3) / 4), dim3(256), 0, F->stream, gout, N, in, C, F->tpart, g, B,
+                           kChunk);
+        hipLaunchKernelGGL(k_flow_sum_parts, dim3((N * K + 255) / 256), dim3(256), 0, F->stream, (const float*)F->tpart,
+                           nchunk, (uint32_t)(N * K), gw);
+        hipLaunchKernelGGL(k_flow_colsum, dim3(N), dim3(256), 0, F->stream, gout, N, R, gw + N * K);
+    };
+    using Hid = std::integral_constant<int, kHidden>;
+    using Out = std::integral_constant<int, kOut>;
+    using In0 = std::integral_constant<int, kCin0>;
+    hipLaunchKernelGGL(k_flow_w2_transpose, dim3((unsigned)((kW2 + 255) / 256), (unsigned)F->d.layers), dim3(256), 0, F->stream,
+                       (const uint16_t*)F->w2, F->tw2t);
     for (int l = 0; l < F->d.layers; ++l) {
         const int mu = l % 4, par = (l / 4) % 2;
         float* gl = F->tgrad + (size_t)l * kLayerParams;   // W1, b1, W2, b2 of layer l
@@ -1425,40 +1696,18 @@ int train_grad(qcd_flow* F, const float* links, int batch, double* loss)
         });
         conditioner(F, l, R, F->stream);
         // -log q_a and its gradient with respect to the spline parameters
-        with_mu(mu, [&](auto m) {
-            hipLaunchKernelGGL(k_flow_nll_grad<decltype(m)::value>, dim3(nb), dim3(256), 0, F->stream,
-                               (const float4*)F->links, F->prm, F->tg, F->tloss, g, B, par, F->d.bins);
+        with_mu_bins(mu, F->d.bins, [&](auto m, auto k) {
+            hipLaunchKernelGGL((k_flow_nll_grad<decltype(m)::value, decltype(k)::value>), site_grid(R), site_block(R), 0,
+                               F->stream, (const float4*)F->links, F->prm, F->tg, F->tloss, g, B, par);
         });
         hipLaunchKernelGGL((k_flow_rowsum<float>), dim3(B), dim3(256), 0, F->stream, F->tloss, g.V,
                            F->tsums + (size_t)l * F->d.max_batch);
-        // conv2: weight and bias gradients, then the hidden gradient through the transposed convolution
-        {
-            const uint32_t tiles = (uint32_t)(kStencil * kHidden / 16) * (kOut / 16) * nchunk;
-            hipLaunchKernelGGL(k_flow_wgrad, dim3((tiles + 3) / 4), dim3(256), 0, F->stream, (const uint16_t*)F->tg, kOut,
-                               (const uint16_t*)F->hid, kHidden, F->tpart, g, B, kChunk);
-            const uint32_t n2 = (uint32_t)kW2;
-            hipLaunchKernelGGL(k_flow_sum_parts, dim3((n2 + 255) / 256), dim3(256), 0, F->stream, (const float*)F->tpart,
-                               nchunk, n2, gl + kW1 + kHidden);
-            hipLaunchKernelGGL(k_flow_colsum, dim3(kOut), dim3(256), 0, F->stream, (const uint16_t*)F->tg, kOut, R,
-                               gl + kW1 + kHidden + kW2);
-            const uint32_t nt = (uint32_t)(kHidden * kStencil * kOut);
-            hipLaunchKernelGGL(k_flow_w2_transpose, dim3((nt + 255) / 256), dim3(256), 0, F->stream,
-                               (const uint16_t*)(F->w2 + l * kW2), F->tw2t);
-            launch_conv<kOut, false>(F->tg, F->tw2t, F->tzero, nullptr, F->tdhid, g, R, F->stream);
-            hipLaunchKernelGGL(k_flow_tanh_back, dim3((R * kHidden + 255) / 256), dim3(256), 0, F->stream,
-                               (const float*)F->tdhid, (const uint16_t*)F->hid, F->tdpre, R * (uint32_t)kHidden);
-        }
+        // conv2: weight and bias gradients, then the gradient before tanh
+        // through the transposed convolution
+        weight_grad(Hid{}, Out{}, F->tg, F->hid, lds2, gl + kW1 + kHidden);
+        launch_conv<kOut, CONV_TANH_BACK>(F->tg, F->tw2t + l * kW2, F->tzero, F->hid, F->tdpre, nullptr, g, R, F->stream);
         // conv1: weight and bias gradients (the features are data: no further gradient)
-        {
-            const uint32_t K1 = kStencil * kCin0, tiles = ((K1 + 15) / 16) * (kHidden / 16) * nchunk;
-            hipLaunchKernelGGL(k_flow_wgrad, dim3((tiles + 3) / 4), dim3(256), 0, F->stream, (const uint16_t*)F->tdpre,
-                               kHidden, (const uint16_t*)F->feat, kCin0, F->tpart, g, B, kChunk);
-            const uint32_t n1 = (uint32_t)kW1;
-            hipLaunchKernelGGL(k_flow_sum_parts, dim3((n1 + 255) / 256), dim3(256), 0, F->stream, (const float*)F->tpart,
-                               nchunk, n1, gl);
-            hipLaunchKernelGGL(k_flow_colsum, dim3(kHidden), dim3(256), 0, F->stream, (const uint16_t*)F->tdpre, kHidden,
-                               R, gl + kW1);
-        }
+        weight_grad(In0{}, Hid{}, F->tdpre, F->feat, lds1, gl);
     }
     FCHK(hipGetLastError());
     if (loss) {
