@@ -29,13 +29,17 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
 #include <ctime>
+#include <mutex>
 #include <string>
+#include <system_error>
+#include <thread>
 #include <vector>
 
 #include "../../include/qcd_hip.h"
@@ -1828,6 +1832,14 @@ __global__ __launch_bounds__(kBlock) void k_finalize_batch(const ChainDesc* cd, 
 // ============================================================================
 __device__ __align__(256) double scratch[kScratchBytesDev / sizeof(double)];
 
+// One of the lattices that keep the pinned transfer buffer alive.
+struct StageUser {
+    StageUser();
+    ~StageUser();
+    StageUser(const StageUser&) = delete;
+    StageUser& operator=(const StageUser&) = delete;
+};
+
 struct qcd_lattice {
     qcd_params p;
     Geom g;
@@ -1907,6 +1919,7 @@ struct qcd_lattice {
     // lattice's buffers and stream sizing, so neither may change (no
     // re-sizing start, no destroy except through the batch).
     bool batch_owned = false;
+    StageUser stage_user;
     // x-slab (one GPU's share of a lattice cut along x): the slices x = 0 and
     // x = N1 - 1 are halos that the updates read and never write; they are
     // refreshed through qcd_slab_face.
@@ -3243,106 +3256,273 @@ int qcd_prng_init(qcd_lattice* L)
     return QCD_OK;
 }
 
+}  // extern "C"
+
+// ---- links to and from host memory -----------------------------------------
+// The caller's array is [site][direction][N*N] complex doubles, the table
+// planes of one complex per (parity, direction, component).  The stored
+// components travel in the caller's order and the table's type through pinned
+// memory, up to 2 MiB at a time: k_links_move transposes in LDS and reads or writes
+// the pinned memory itself, in whole lines, and up to eight host threads, each
+// with a slot of its own, convert to or from doubles and fill in what is not
+// stored, while the other slots' transfers run.  Bound by the host's first
+// touch of the caller's pages.  One thread that walked the planes site by site
+// after a pageable copy: export of 32^3 x 8 SU(3) FP32 (151 MB) 35.6 ms, now
+// 3.1; import of 16^4 (38 MB) 2.1 ms, now 0.62.
+constexpr size_t kLinkSlotMin = 512u << 10, kLinkSlotMax = 2u << 20;
+constexpr uint32_t kLinkSlots = 8, kMovePairs = 32;
+
+template <typename C, int NP, bool IN>
+__global__ __launch_bounds__(256) void k_links_move(C* table, C* host, Geom g, uint32_t i0, uint32_t npairs)
+{
+    // 32 site pairs (y even, y odd) per workgroup; an odd pitch keeps the
+    // plane-wise accesses of neighbouring sites in different banks
+    constexpr uint32_t R = 4u * NP, PITCH = R + 1u, PER = 16u / sizeof(C);
+    __shared__ C sm[2u * kMovePairs * PITCH];
+    const uint32_t b0 = blockIdx.x * kMovePairs, np = min(kMovePairs, npairs - b0);
+    const uint32_t ii = threadIdx.x & 31u, row = threadIdx.x >> 5, i = i0 + b0 + ii;
+    const uint32_t q = g.dh.div(i), r = g.d3.div(q), x = g.d4.div(r);
+    const uint32_t par0 = (x + (q - r * (uint32_t)g.n3) + (r - x * (uint32_t)g.n4)) & 1u;   // parity of the pair's first site
+    uint4* hv = reinterpret_cast<uint4*>(host + (size_t)b0 * 2u * R);
+    const uint32_t nv = 2u * np * R / PER;
+    if constexpr (IN) {
+#pragma unroll 5
+        for (uint32_t j = threadIdx.x; j < nv; j += 256u) {
+            const uint4 v = hv[j];
+            C c[PER];
+            __builtin_memcpy(c, &v, 16);
+#pragma unroll
+            for (uint32_t k = 0; k < PER; ++k) {
+                const uint32_t o = j * PER + k;
+                sm[o / R * PITCH + o % R] = c[k];
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (uint32_t pl = row; pl < 2u * R; pl += 8u)
+            if (ii < np) table[(size_t)pl * g.vh_pad + i] = sm[(2u * ii + ((pl >= R ? 1u : 0u) ^ par0)) * PITCH + pl % R];
+    } else {
+        C v[R / 4u];
+#pragma unroll
+        for (uint32_t k = 0; k < R / 4u; ++k)
+            if (ii < np) v[k] = table[(size_t)(row + 8u * k) * g.vh_pad + i];
+#pragma unroll
+        for (uint32_t k = 0; k < R / 4u; ++k) {
+            const uint32_t pl = row + 8u * k;
+            if (ii < np) sm[(2u * ii + ((pl >= R ? 1u : 0u) ^ par0)) * PITCH + pl % R] = v[k];
+        }
+        __syncthreads();
+        for (uint32_t j = threadIdx.x; j < nv; j += 256u) {
+            C c[PER];
+            uint4 v;
+#pragma unroll
+            for (uint32_t k = 0; k < PER; ++k) {
+                const uint32_t o = j * PER + k;
+                c[k] = sm[o / R * PITCH + o % R];
+            }
+            __builtin_memcpy(&v, c, 16);
+            hv[j] = v;
+        }
+    }
+}
+
+// Pinned memory for one transfer; one buffer is kept between calls as long as
+// any lattice lives.
+static std::mutex stage_mutex;
+static void* stage_kept = nullptr;
+static size_t stage_kept_bytes = 0;
+static int stage_users = 0;
+
+StageUser::StageUser()
+{
+    std::lock_guard<std::mutex> lock(stage_mutex);
+    ++stage_users;
+}
+
+StageUser::~StageUser()
+{
+    std::lock_guard<std::mutex> lock(stage_mutex);
+    if (--stage_users == 0 && stage_kept) {
+        (void)hipHostFree(stage_kept);
+        stage_kept = nullptr;
+    }
+}
+
+struct Stage {
+    void* mem = nullptr;
+    size_t bytes;
+    explicit Stage(size_t n) : bytes(n)
+    {
+        {
+            std::lock_guard<std::mutex> lock(stage_mutex);
+            if (stage_kept && stage_kept_bytes >= n) {
+                mem = stage_kept;
+                bytes = stage_kept_bytes;
+                stage_kept = nullptr;
+            }
+        }
+        if (!mem && hipHostMalloc(&mem, n, hipHostMallocPortable) != hipSuccess) mem = nullptr;
+    }
+    ~Stage()
+    {
+        if (!mem) return;
+        {
+            std::lock_guard<std::mutex> lock(stage_mutex);
+            if (!stage_kept || stage_kept_bytes < bytes) {
+                std::swap(mem, stage_kept);
+                std::swap(bytes, stage_kept_bytes);
+            }
+        }
+        if (mem) (void)hipHostFree(mem);
+    }
+};
+
+// `sites` sites of stored components to the caller's doubles, and back.
+template <typename F> static void unpack_links(const F* src, double* dst, size_t sites, int N, int np)
+{
+    if (np == N * N) {
+        for (size_t j = 0; j < sites * 8 * (size_t)np; ++j) dst[j] = (double)src[j];
+        return;
+    }
+    for (size_t l = 0; l < sites * 4; ++l) {
+        const F* u0 = src + l * 2 * (size_t)np;
+        double* m = dst + l * 2 * (size_t)(N * N);
+        for (int j = 0; j < 2 * np; ++j) m[j] = (double)u0[j];
+        if (N == 2) {
+            m[4] = -m[2];
+            m[5] = m[3];
+            m[6] = m[0];
+            m[7] = -m[1];
+            continue;
+        }
+        // row 3 = conj(row1 x row2)
+        const double *u = m, *v = m + 6;
+        double* w = m + 12;
+        auto cm = [](double ar, double ai, double br, double bi, double& cr, double& ci) {
+            cr = ar * br - ai * bi;
+            ci = ar * bi + ai * br;
+        };
+        double p1r, p1i, p2r, p2i;
+        cm(u[2], u[3], v[4], v[5], p1r, p1i);
+        cm(u[4], u[5], v[2], v[3], p2r, p2i);
+        w[0] = p1r - p2r;
+        w[1] = -(p1i - p2i);
+        cm(u[4], u[5], v[0], v[1], p1r, p1i);
+        cm(u[0], u[1], v[4], v[5], p2r, p2i);
+        w[2] = p1r - p2r;
+        w[3] = -(p1i - p2i);
+        cm(u[0], u[1], v[2], v[3], p1r, p1i);
+        cm(u[2], u[3], v[0], v[1], p2r, p2i);
+        w[4] = p1r - p2r;
+        w[5] = -(p1i - p2i);
+    }
+}
+
+template <typename F> static void pack_links(const double* src, F* dst, size_t sites, int N, int np)
+{
+    if (np == N * N) {
+        for (size_t j = 0; j < sites * 8 * (size_t)np; ++j) dst[j] = (F)src[j];
+        return;
+    }
+    for (size_t l = 0; l < sites * 4; ++l)
+        for (int j = 0; j < 2 * np; ++j) dst[l * 2 * (size_t)np + j] = (F)src[l * 2 * (size_t)(N * N) + j];
+}
+
+template <typename C, bool IN>
+static void launch_links_move(qcd_lattice* L, void* host, uint32_t i0, uint32_t npairs)
+{
+    const dim3 nb((npairs + kMovePairs - 1) / kMovePairs);
+    C *t = (C*)L->table, *h = (C*)host;
+    if (L->np == 9) hipLaunchKernelGGL((k_links_move<C, 9, IN>), nb, dim3(256), 0, L->stream, t, h, L->g, i0, npairs);
+    else if (L->np == 6) hipLaunchKernelGGL((k_links_move<C, 6, IN>), nb, dim3(256), 0, L->stream, t, h, L->g, i0, npairs);
+    else hipLaunchKernelGGL((k_links_move<C, 2, IN>), nb, dim3(256), 0, L->stream, t, h, L->g, i0, npairs);
+}
+
+// Export (out) or import (in); returns when the transfer is complete.
+static int move_links(qcd_lattice* L, double* out, const double* in)
+{
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    HIPCHK(hipStreamIsCapturing(L->stream, &cap));
+    if (cap != hipStreamCaptureStatusNone) return fail(QCD_E_HIP, "links cannot be copied while the stream is recorded");
+    int dev = 0;
+    HIPCHK(hipGetDevice(&dev));
+    const int N = L->p.sun, np = L->np;
+    const bool f32 = L->elem == 8;
+    const size_t V = 2 * (size_t)L->g.vh, per_site = 4 * (size_t)np * L->elem;
+    // an eighth of the links per slot: 16^4 SU(2) (4 MB) exports in 0.6 ms by
+    // half megabytes as by two, imports in 0.24 against 0.50 by one; 32^3 x 8
+    // in 3.1 ms by 2 MiB, 3.7 by half, 4.3 by a quarter
+    const size_t slot_bytes = std::clamp(V * per_site / kLinkSlots, kLinkSlotMin, kLinkSlotMax);
+    const size_t chunk = std::min(slot_bytes / per_site / (2 * kMovePairs) * (2 * kMovePairs), V);   // sites
+    const size_t nchunks = (V + chunk - 1) / chunk;
+    const uint32_t workers = (uint32_t)std::min<size_t>(kLinkSlots, nchunks);
+    Stage st(chunk * per_site * workers);
+    if (!st.mem) return fail(QCD_E_NOMEM, "pinned memory for the links (%zu bytes)", chunk * per_site * workers);
+    hipEvent_t ev[kLinkSlots] = {};
+    std::atomic<int> err{(int)hipSuccess};
+    auto keep = [&](hipError_t e) {
+        int ok = (int)hipSuccess;
+        if (e != hipSuccess) err.compare_exchange_strong(ok, (int)e);
+        return e == hipSuccess;
+    };
+    for (uint32_t w = 0; w < workers; ++w) keep(hipEventCreateWithFlags(&ev[w], hipEventDisableTiming));
+    std::atomic<size_t> next{0};
+    auto work = [&](uint32_t w) {
+        if (w && !keep(hipSetDevice(dev))) return;
+        unsigned char* slot = (unsigned char*)st.mem + w * chunk * per_site;
+        bool used = false;
+        for (size_t c; err.load() == (int)hipSuccess && (c = next.fetch_add(1)) < nchunks;) {
+            const size_t s0 = c * chunk, ns = std::min(chunk, V - s0), at = s0 * 8 * (size_t)(N * N);
+            if (in) {
+                if (used && !keep(hipEventSynchronize(ev[w]))) return;
+                if (f32) pack_links(in + at, (float*)slot, ns, N, np);
+                else pack_links(in + at, (double*)slot, ns, N, np);
+                if (f32) launch_links_move<float2, true>(L, slot, (uint32_t)(s0 / 2), (uint32_t)(ns / 2));
+                else launch_links_move<double2, true>(L, slot, (uint32_t)(s0 / 2), (uint32_t)(ns / 2));
+                if (!keep(hipGetLastError()) || !keep(hipEventRecord(ev[w], L->stream))) return;
+                used = true;
+            } else {
+                if (f32) launch_links_move<float2, false>(L, slot, (uint32_t)(s0 / 2), (uint32_t)(ns / 2));
+                else launch_links_move<double2, false>(L, slot, (uint32_t)(s0 / 2), (uint32_t)(ns / 2));
+                if (!keep(hipGetLastError()) || !keep(hipEventRecord(ev[w], L->stream)) || !keep(hipEventSynchronize(ev[w])))
+                    return;
+                if (f32) unpack_links((const float*)slot, out + at, ns, N, np);
+                else unpack_links((const double*)slot, out + at, ns, N, np);
+            }
+        }
+    };
+    std::thread th[kLinkSlots];
+    if (err.load() == (int)hipSuccess) {
+        for (uint32_t w = 1; w < workers; ++w) {
+            try {
+                th[w] = std::thread(work, w);
+            } catch (const std::system_error&) {
+                break;   // no more threads: those there are take all chunks
+            }
+        }
+        work(0);
+    }
+    for (uint32_t w = 1; w < workers; ++w)
+        if (th[w].joinable()) th[w].join();
+    keep(hipStreamSynchronize(L->stream));   // the slots are free again, also after an error
+    for (uint32_t w = 0; w < workers; ++w)
+        if (ev[w]) (void)hipEventDestroy(ev[w]);
+    const hipError_t e = (hipError_t)err.load();
+    return e == hipSuccess ? QCD_OK : fail(QCD_E_HIP, "%s of the links: %s", in ? "import" : "export", hipGetErrorString(e));
+}
+
+extern "C" {
+
 int qcd_lattice_import(qcd_lattice* L, const double* links)
 {
     if (!L || !links) return fail(QCD_E_ARG, "null argument");
-    const int N = L->p.sun;
-    std::vector<unsigned char> host(L->table_bytes, 0);
-    const uint32_t vh = L->g.vh, vp = L->g.vh_pad;
-    const uint64_t V = 2ull * vh;
-    for (uint64_t s = 0; s < V; ++s) {
-        uint32_t y = (uint32_t)(s % L->g.n2);
-        uint64_t r = s / L->g.n2;
-        uint32_t z = (uint32_t)(r % L->g.n3);
-        r /= L->g.n3;
-        uint32_t t = (uint32_t)(r % L->g.n4);
-        uint32_t x = (uint32_t)(r / L->g.n4);
-        int par = (int)((x + y + z + t) & 1);
-        uint64_t i = s >> 1;
-        for (int d = 0; d < 4; ++d)
-            for (int k = 0; k < L->np; ++k) {
-                const double* src = links + 2 * (((size_t)s * 4 + d) * N * N + k);
-                size_t off = ((size_t)((par * 4 + d) * L->np + k) * vp + i);
-                if (L->elem == 8) {
-                    float* dst = (float*)host.data() + 2 * off;
-                    dst[0] = (float)src[0];
-                    dst[1] = (float)src[1];
-                } else {
-                    double* dst = (double*)host.data() + 2 * off;
-                    dst[0] = src[0];
-                    dst[1] = src[1];
-                }
-            }
-    }
-    HIPCHK(hipMemcpyAsync(L->table, host.data(), L->table_bytes, hipMemcpyHostToDevice, L->stream));
-    HIPCHK(hipStreamSynchronize(L->stream));
-    return QCD_OK;
+    return move_links(L, nullptr, links);
 }
 
 int qcd_lattice_export(qcd_lattice* L, double* links)
 {
     if (!L || !links) return fail(QCD_E_ARG, "null argument");
-    const int N = L->p.sun;
-    std::vector<unsigned char> host(L->table_bytes);
-    HIPCHK(hipMemcpyAsync(host.data(), L->table, L->table_bytes, hipMemcpyDeviceToHost, L->stream));
-    HIPCHK(hipStreamSynchronize(L->stream));
-    const uint32_t vh = L->g.vh, vp = L->g.vh_pad;
-    const uint64_t V = 2ull * vh;
-    for (uint64_t s = 0; s < V; ++s) {
-        uint32_t y = (uint32_t)(s % L->g.n2);
-        uint64_t r = s / L->g.n2;
-        uint32_t z = (uint32_t)(r % L->g.n3);
-        r /= L->g.n3;
-        uint32_t t = (uint32_t)(r % L->g.n4);
-        uint32_t x = (uint32_t)(r / L->g.n4);
-        int par = (int)((x + y + z + t) & 1);
-        uint64_t i = s >> 1;
-        for (int d = 0; d < 4; ++d) {
-            double* m = links + 2 * (((size_t)s * 4 + d) * N * N);
-            for (int k = 0; k < L->np; ++k) {
-                size_t off = ((size_t)((par * 4 + d) * L->np + k) * vp + i);
-                if (L->elem == 8) {
-                    const float* src = (const float*)host.data() + 2 * off;
-                    m[2 * k] = src[0];
-                    m[2 * k + 1] = src[1];
-                } else {
-                    const double* src = (const double*)host.data() + 2 * off;
-                    m[2 * k] = src[0];
-                    m[2 * k + 1] = src[1];
-                }
-            }
-            if (N == 3 && L->np == 6) {
-                // row 3 = conj(row1 x row2)
-                double* u = m;
-                double* v = m + 6;
-                double* w = m + 12;
-                auto cm = [](double ar, double ai, double br, double bi, double& cr, double& ci) {
-                    cr = ar * br - ai * bi;
-                    ci = ar * bi + ai * br;
-                };
-                double p1r, p1i, p2r, p2i;
-                cm(u[2], u[3], v[4], v[5], p1r, p1i);
-                cm(u[4], u[5], v[2], v[3], p2r, p2i);
-                w[0] = p1r - p2r;
-                w[1] = -(p1i - p2i);
-                cm(u[4], u[5], v[0], v[1], p1r, p1i);
-                cm(u[0], u[1], v[4], v[5], p2r, p2i);
-                w[2] = p1r - p2r;
-                w[3] = -(p1i - p2i);
-                cm(u[0], u[1], v[2], v[3], p1r, p1i);
-                cm(u[2], u[3], v[0], v[1], p2r, p2i);
-                w[4] = p1r - p2r;
-                w[5] = -(p1i - p2i);
-            }
-            if (N == 2) {
-                m[4] = -m[2];
-                m[5] = m[3];
-                m[6] = m[0];
-                m[7] = -m[1];
-            }
-        }
-    }
-    return QCD_OK;
+    return move_links(L, links, nullptr);
 }
 
 static int halfstep_impl(qcd_lattice* L, int parity, int mu, int kind, const LaunchOpt& o)
