@@ -936,6 +936,14 @@ __global__ __launch_bounds__(kRlWaves * 64) void k_ranlux_jump(float4* state, ui
     rl_produce(state, n, samples, keep, quads, blockIdx.x, tab, rl_lds, blockDim.x / 64u);
 }
 
+// kRlAhead of them in one launch, blockIdx.y the number of the produce().
+__global__ __launch_bounds__(kRlWaves * 64) void k_ranlux_ahead(const float4* state, float4* next, uint32_t n, uint32_t samples,
+                                                                uint32_t keep, float4* quads, const uint4* tab)
+{
+    extern __shared__ uint32_t rl_lds[];
+    rl_ahead(state, next, n, samples, keep, quads, blockIdx.x, blockIdx.y, tab, rl_lds, blockDim.x / 64u);
+}
+
 // produce() of `samples` quads per stream; the first `keep` go to `quads`
 // (null: none).  tab: the lattice's jump tables.
 void launch_ranlux_produce(int lux, float4* state, uint32_t n, uint32_t samples, uint32_t keep, float4* quads,
@@ -958,7 +966,7 @@ void launch_ranlux_produce(int lux, float4* state, uint32_t n, uint32_t samples,
     }
 }
 
-// Device copy of the jump tables of one luxury level (96 kB).
+// Device copy of the jump tables of one luxury level (253 kB).
 bool alloc_rl_tables(int lux, uint4** tab)
 {
     const std::vector<uint32_t>& h = rl_tables(lux >= 0 && lux < 4 ? lux : 4);   // as the kernels take it
@@ -1850,6 +1858,9 @@ struct qcd_lattice {
     uint4* rng_buf[2] = {nullptr, nullptr};   // generator states; rng_buf[rng_cur] is current
     uint4* jump_cols = nullptr;               // XOR128 jump-ahead matrix: 128 columns, then the 4-bit table
     float4* rl_state = nullptr;               // RANLUX: 7 float4 per stream
+    float4* rl_next = nullptr;                // its other half when a sweep's quads are produced ahead
+    float4* ahead_buf = nullptr;              // quads of kRlAhead half-steps, ahead_quads per stream and half-step
+    uint32_t ahead_quads = 0;
     uint4* rl_tab = nullptr;                  // RANLUX: jump tables of its luxury level
     float4* prn_buf = nullptr;                // RANLUX: produced quads, prn_quads per stream
     uint32_t prn_quads = 0;
@@ -2006,6 +2017,7 @@ struct LaunchOpt {
     hipEvent_t e0 = nullptr;
     hipEvent_t e1 = nullptr;
     uint32_t lds = 0;   // extra dynamic LDS per workgroup (caps workgroups per CU)
+    const float4* prn = nullptr;   // this half-step's quads, produced already
 };
 
 template <typename Kern, typename... Args>
@@ -2203,6 +2215,46 @@ void produce_quads_into(qcd_lattice* L, uint32_t samples, uint32_t keep, float4*
     }
 }
 
+// RANLUX: the quads of kRlAhead half-steps of a heatbath sweep in one launch
+// (they follow each other whatever the links are).  A single produce() is bound
+// by its latency, 4 to 5 us of loads, one jump and up to 24 steps; kRlAhead at
+// once fill the chip instead.  Heatbath half-step with its produce(): 8^4 SU(2)
+// 11.5 to 7.7 us, 16^4 12.5 to 9.5; SU(3) 8^4 15.3 to 11.0, 20 x 12 x 28 x 10
+// 24.9 to 20.5, 24^3 x 12 (175 MB of quads) 40.4 to 35.0.  Beyond what the last-level
+// cache holds the quads come back from memory: SU(2) 32^4 (369 MB) 63.3 to 69.1.
+constexpr size_t kAheadBytes = size_t(192) << 20;
+bool ahead_fits(const qcd_lattice* L)
+{
+    if (L->p.prng != QCD_PRNG_RANLUX || !L->quad_buffer || L->batch_owned) return false;
+    const uint32_t keep = update_quads(L);
+    return rl_waves(L->p.ranlux_luxury, L->s_quads, keep, L->n_inst) && rl_ahead_waves(L->s_quads, keep) &&
+           sizeof(float4) * kRlAhead * keep * (size_t)L->n_inst <= kAheadBytes;
+}
+// Its buffers, before a sweep or a capture of sweeps; without them (no memory,
+// or a capture under way) every half-step produces for itself.
+void ahead_prepare(qcd_lattice* L)
+{
+    if (!ahead_fits(L) || (L->ahead_buf && L->ahead_quads >= update_quads(L))) return;
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(L->stream, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) return;
+    (void)hipStreamSynchronize(L->stream);
+    (void)hipFree(L->ahead_buf);
+    L->ahead_buf = nullptr;
+    L->ahead_quads = update_quads(L);
+    if ((!L->rl_next && hipMalloc((void**)&L->rl_next, sizeof(float4) * 7 * L->n_inst) != hipSuccess) ||
+        hipMalloc((void**)&L->ahead_buf, sizeof(float4) * kRlAhead * L->ahead_quads * (size_t)L->n_inst) != hipSuccess) {
+        (void)hipGetLastError();
+        L->ahead_buf = nullptr;
+    }
+}
+void launch_ahead(qcd_lattice* L)
+{
+    const uint32_t keep = update_quads(L), W = rl_ahead_waves(L->s_quads, keep);
+    hipLaunchKernelGGL(k_ranlux_ahead, dim3((L->n_inst + 63u) / 64u, kRlAhead), dim3(64u * W), rl_lds_bytes(W), L->stream,
+                       L->rl_state, L->rl_next, L->n_inst, L->s_quads, keep, L->ahead_buf, L->rl_tab);
+    std::swap(L->rl_state, L->rl_next);
+}
+
 template <typename R, int N, int NREAL>
 int launch_update_rn(qcd_lattice* L, int parity, int mu, int kind, int start_gid, const LaunchOpt& o)
 {
@@ -2249,11 +2301,11 @@ int launch_update_rn(qcd_lattice* L, int parity, int mu, int kind, int start_gid
         if (L->quad_buffer) {
             // the reference's produce() into the PRN buffer, then the update
             // reads quad k of link i at k * PRNGSTEP + i
-            {
+            if (!o.prn) {
                 ProfScope ps(L, "PRNG produce");
                 produce_quads_into(L, L->s_quads, update_quads(L), L->prn_buf);
             }
-            a.prn = L->prn_buf;
+            a.prn = o.prn ? o.prn : L->prn_buf;
             a.prn_stride = L->n_streams;
             ProfScope ps(L, o.meas_mode ? "heatbath half-step + plaquette" : "heatbath half-step");
             launch_update_t<R, N, NREAL, false, RK_BUF>(L, a, ol);
@@ -2703,6 +2755,8 @@ int qcd_lattice_destroy(qcd_lattice* L)
     (void)hipFree(L->rng_buf[1]);
     (void)hipFree(L->jump_cols);
     (void)hipFree(L->rl_state);
+    (void)hipFree(L->rl_next);
+    (void)hipFree(L->ahead_buf);
     (void)hipFree(L->rl_tab);
     (void)hipFree(L->prn_buf);
     (void)hipFree(L->partials);
@@ -2935,6 +2989,7 @@ int qcd_graph_begin(qcd_lattice* L)
     if (L->profiling) return fail(QCD_E_STATE, "kernel timing waits for every kernel: no graph while it is on");
     drop_cycle_graphs(L);
     HIPCHK(hipStreamSynchronize(L->stream));
+    ahead_prepare(L);
     HIPCHK(hipStreamBeginCapture(L->stream, hipStreamCaptureModeThreadLocal));
     L->graph_open = true;
     L->graph_counter0 = L->prng_counter;
@@ -3302,15 +3357,9 @@ __global__ __launch_bounds__(256) void k_links_move(C* table, C* host, Geom g, u
         for (uint32_t pl = row; pl < 2u * R; pl += 8u)
             if (ii < np) table[(size_t)pl * g.vh_pad + i] = sm[(2u * ii + ((pl >= R ? 1u : 0u) ^ par0)) * PITCH + pl % R];
     } else {
-        C v[R / 4u];
 #pragma unroll
-        for (uint32_t k = 0; k < R / 4u; ++k)
-            if (ii < np) v[k] = table[(size_t)(row + 8u * k) * g.vh_pad + i];
-#pragma unroll
-        for (uint32_t k = 0; k < R / 4u; ++k) {
-            const uint32_t pl = row + 8u * k;
-            if (ii < np) sm[(2u * ii + ((pl >= R ? 1u : 0u) ^ par0)) * PITCH + pl % R] = v[k];
-        }
+        for (uint32_t pl = row; pl < 2u * R; pl += 8u)   // past the end the last pair again, into unread places
+            sm[(2u * ii + ((pl >= R ? 1u : 0u) ^ par0)) * PITCH + pl % R] = table[(size_t)pl * g.vh_pad + min(i, g.vh - 1u)];
         __syncthreads();
         for (uint32_t j = threadIdx.x; j < nv; j += 256u) {
             C c[PER];
@@ -3543,20 +3592,36 @@ int qcd_halfstep(qcd_lattice* L, int parity, int mu, int kind)
 static int sweep_impl(qcd_lattice* L, int kind, bool fuse_plaquette, std::vector<hipEvent_t>* ev, int* ev_used,
                       hipEvent_t join_before_odd_t = nullptr)
 {
+    // kernel timing counts one produce() per half-step, as the reference does
+    const bool ahead = kind == QCD_HEATBATH && !L->gid_updates && L->rng_ready && !L->profiling && ahead_fits(L) &&
+                       L->ahead_buf && L->ahead_quads >= update_quads(L);
+    static_assert(8 % kRlAhead == 0 && (8 / kRlAhead) % 2 == 0, "a sweep leaves the states in the buffer it found them in");
+    const float4* const states = L->rl_state;
+    auto half = [&](int parity, int mu) {
+        // the odd T half-step is the first to write links a measurement
+        // of the previous cycle (plaquette sums, Polyakov loop) reads
+        if (join_before_odd_t && parity == 1 && mu == 3) HIPCHK(hipStreamWaitEvent(L->stream, join_before_odd_t, 0));
+        LaunchOpt o;
+        if (fuse_plaquette && parity == 0 && mu >= 1) o.meas_mode = mu;   // 1, 2, 3
+        if (ev) {
+            o.e0 = (*ev)[2 * (*ev_used)];
+            o.e1 = (*ev)[2 * (*ev_used) + 1];
+            ++*ev_used;
+        }
+        if (ahead) {
+            const int j = (4 * (1 - parity) + mu) % kRlAhead;
+            if (j == 0) launch_ahead(L);
+            o.prn = L->ahead_buf + (size_t)j * update_quads(L) * L->n_inst;
+        }
+        return halfstep_impl(L, parity, mu, kind, o);
+    };
     for (int parity = 1; parity >= 0; --parity)
         for (int mu = 0; mu < 4; ++mu) {
-            // the odd T half-step is the first to write links a measurement
-            // of the previous cycle (plaquette sums, Polyakov loop) reads
-            if (join_before_odd_t && parity == 1 && mu == 3) HIPCHK(hipStreamWaitEvent(L->stream, join_before_odd_t, 0));
-            LaunchOpt o;
-            if (fuse_plaquette && parity == 0 && mu >= 1) o.meas_mode = mu;   // 1, 2, 3
-            if (ev) {
-                o.e0 = (*ev)[2 * (*ev_used)];
-                o.e1 = (*ev)[2 * (*ev_used) + 1];
-                ++*ev_used;
+            const int rc = half(parity, mu);
+            if (rc) {
+                if (L->rl_state != states) std::swap(L->rl_state, L->rl_next);
+                return rc;
             }
-            int rc = halfstep_impl(L, parity, mu, kind, o);
-            if (rc) return rc;
         }
     return QCD_OK;
 }
@@ -3564,6 +3629,7 @@ static int sweep_impl(qcd_lattice* L, int kind, bool fuse_plaquette, std::vector
 int qcd_sweep(qcd_lattice* L, int kind)
 {
     if (!L) return fail(QCD_E_ARG, "null lattice");
+    if (kind == QCD_HEATBATH) ahead_prepare(L);
     return sweep_impl(L, kind, false, nullptr, nullptr);
 }
 
@@ -3863,6 +3929,7 @@ int qcd_cycle_capture(qcd_lattice* L, int n_hb, int n_or, int mask)
     if (n_hb < 0 || n_or < 0) return fail(QCD_E_ARG, "negative sweep count");
     drop_cycle_graphs(L);
     HIPCHK(hipStreamSynchronize(L->stream));
+    if (n_hb) ahead_prepare(L);
     // K = QCD_TUNE_CYCLES_PER_GRAPH consecutive cycles as one graph, each
     // cycle's measurement beside the next cycle's first half-steps (replays
     // of whole K-blocks); the single cycle below covers the rest
@@ -3912,6 +3979,7 @@ int qcd_cycle_run(qcd_lattice* L, int n_hb, int n_or, int mask)
 {
     if (!L) return fail(QCD_E_ARG, "null lattice");
     if (n_hb < 0 || n_or < 0) return fail(QCD_E_ARG, "negative sweep count");
+    if (n_hb) ahead_prepare(L);
     return enqueue_cycle(L, n_hb, n_or, mask, nullptr, nullptr);
 }
 

@@ -30,7 +30,9 @@
 
 namespace qcd {
 
-constexpr int kRlTasks = 12;       // blocks a produce() may span on this path
+constexpr int kRlTasks = 24;       // blocks with a table: four produce() of 33 quads
+constexpr int kRlSpan = 12;        // blocks a single produce() may span on this path
+constexpr int kRlAhead = 4;        // produce() of one launch of rl_ahead
 constexpr int kRlWaves = 8;        // wavefronts of a workgroup: 60 kB of LDS
 constexpr int kRlTaskVec = 660;    // 16-byte entries of one block's table: 2 x 320 + 20
 constexpr int kRlIn = 28, kRlOut = 26;   // words per stream in LDS
@@ -402,6 +404,68 @@ __device__ __forceinline__ void rl_produce(float4* state, uint32_t n, uint32_t s
     if (last && valid) rl_store(state, n, g, s, carry, k1);
 }
 
+// produce() number h of kRlAhead that follow each other, `samples` quads each
+// with the first `keep` of every one stored ([h][quad][stream]): every
+// workgroup starts from the states before the first, and the last one's writes
+// those after the last to `next`, a buffer of its own.
+__device__ __forceinline__ void rl_ahead(const float4* state, float4* next, uint32_t n, uint32_t samples, uint32_t keep,
+                                         float4* quads, uint32_t unit, uint32_t h, const uint4* tab, uint32_t* lds,
+                                         uint32_t W)
+{
+    const uint32_t w = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const uint32_t lane = threadIdx.x & 63, g0 = unit * 64u + lane;
+    const bool valid = g0 < n;
+    const uint32_t g = valid ? g0 : n - 1u;
+    const float4 c6 = state[(size_t)6 * n + g];
+    const uint32_t k = min((uint32_t)__builtin_amdgcn_readfirstlane((int)c6.z), 6u);
+    const uint32_t first = 6u - k, total = (uint32_t)kRlAhead * samples, start = h * samples, stop = start + keep;
+    const uint32_t nb = (total - first + 5u) / 6u;
+    // blocks after the current one that hold quads start .. stop - 1
+    const uint32_t lo = start < first ? 1u : 1u + (start - first) / 6u, hi = stop <= first ? 0u : 1u + (stop - 1u - first) / 6u;
+    const bool end = h == (uint32_t)kRlAhead - 1u && w == W - 1u && hi < nb;   // a last block that is not kept
+    const uint32_t t = end ? nb : lo + w;
+    const bool idle = !end && t > hi;
+    RlTab table;
+    if (!idle) rl_load(table, tab + (size_t)(t - 1u) * kRlTaskVec);
+    quads += (size_t)h * keep * n;
+    uint32_t s[24], carry;
+    if (w == 0) {
+#pragma unroll
+        for (int q = 0; q < 6; ++q) {
+            const float4 v = state[(size_t)q * n + g];
+            s[4 * q] = (uint32_t)(v.x * 16777216.0f);
+            s[4 * q + 1] = (uint32_t)(v.y * 16777216.0f);
+            s[4 * q + 2] = (uint32_t)(v.z * 16777216.0f);
+            s[4 * q + 3] = (uint32_t)(v.w * 16777216.0f);
+        }
+        carry = c6.w > 0.0f ? 1u : 0u;
+        rl_block(s, carry, k, 6u, 0u - start, keep, quads, n, g, valid);   // numbers below 0 wrap: not kept
+        uint32_t* o = lds + lane * kRlIn;
+#pragma unroll
+        for (int q = 0; q < 6; ++q)
+            *reinterpret_cast<uint4*>(o + 4 * q) =
+                make_uint4((s[4 * q] ^ 0x808080u) | (q == 0 ? carry << 24 : 0u), s[4 * q + 1] ^ 0x808080u,
+                           s[4 * q + 2] ^ 0x808080u, s[4 * q + 3] ^ 0x808080u);
+    }
+    __syncthreads();
+    if (idle) return;
+    rl_jump(table, lds, lds + 64 * kRlIn + w * 64u * kRlOut, s, carry);
+    const uint32_t m = first + 6u * (t - 1u);
+    const uint32_t k1 = min(6u, (t == nb ? total : stop) - m);
+    rl_block(s, carry, 0u, k1, m - start, keep, quads, n, g, valid);
+    if (t == nb && valid) rl_store(next, n, g, s, carry, k1);
+}
+
+// Wavefronts of rl_ahead: the blocks that `keep` quads can touch, and one for
+// the last block when the last produce() keeps less than all; 0: not on this path.
+inline uint32_t rl_ahead_waves(uint32_t samples, uint32_t keep)
+{
+    const uint32_t W = (keep + 4u) / 6u + 1u + (keep < samples ? 1u : 0u);
+    const bool fits = samples >= 6u && keep >= 1u && keep <= samples && ((uint32_t)kRlAhead * samples + 5u) / 6u <= (uint32_t)kRlTasks &&
+                      W <= (uint32_t)kRlWaves;
+    return fits ? W : 0u;
+}
+
 // Wavefronts per 64 streams for a produce() of `samples` quads that keeps
 // `keep` of them, for n streams; 0: step through the blocks instead.  That is
 // for lengths that the tables or a workgroup do not reach, and for many
@@ -416,7 +480,7 @@ inline uint32_t rl_waves(int lux, uint32_t samples, uint32_t keep, uint64_t n)
     const uint32_t nb = (samples + 5u) / 6u, kept = (keep + 5u) / 6u + 1u;
     const uint32_t W = nb < kept ? (nb ? nb : 1u) : kept;
     const uint64_t most = rl_skip_count(lux) >= 223 ? 98304u : 40960u;
-    if (nb > (uint32_t)kRlTasks || W > (uint32_t)kRlWaves || (W > 4u && n > most)) return 0u;
+    if (nb > (uint32_t)kRlSpan || W > (uint32_t)kRlWaves || (W > 4u && n > most)) return 0u;
     return W;
 }
 inline uint32_t rl_lds_bytes(uint32_t W) { return 4u * 64u * ((uint32_t)kRlIn + W * (uint32_t)kRlOut); }
