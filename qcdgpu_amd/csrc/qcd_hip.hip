@@ -936,12 +936,20 @@ __global__ __launch_bounds__(kRlWaves * 64) void k_ranlux_jump(float4* state, ui
     rl_produce(state, n, samples, keep, quads, blockIdx.x, tab, rl_lds, blockDim.x / 64u);
 }
 
-// kRlAhead of them in one launch, blockIdx.y the number of the produce().
+// kRlAhead of them in one launch, blockIdx.y the number of the produce(): a unit
+// of 64 streams per workgroup, or several in turn.
 __global__ __launch_bounds__(kRlWaves * 64) void k_ranlux_ahead(const float4* state, float4* next, uint32_t n, uint32_t samples,
                                                                 uint32_t keep, float4* quads, const uint4* tab)
 {
     extern __shared__ uint32_t rl_lds[];
     rl_ahead(state, next, n, samples, keep, quads, blockIdx.x, blockIdx.y, tab, rl_lds, blockDim.x / 64u);
+}
+__global__ __launch_bounds__(kRlWaves * 64) void k_ranlux_ahead_turns(const float4* state, float4* next, uint32_t n,
+                                                                      uint32_t samples, uint32_t keep, float4* quads,
+                                                                      const uint4* tab)
+{
+    extern __shared__ uint32_t rl_lds[];
+    rl_ahead_turns(state, next, n, samples, keep, quads, blockIdx.x, gridDim.x, blockIdx.y, tab, rl_lds, blockDim.x / 64u - 1u);
 }
 
 // produce() of `samples` quads per stream; the first `keep` go to `quads`
@@ -2282,8 +2290,8 @@ void produce_quads_into(qcd_lattice* L, uint32_t samples, uint32_t keep, float4*
 // (they follow each other whatever the links are).  A single produce() is bound
 // by its latency, 4 to 5 us of loads, one jump and up to 24 steps; kRlAhead at
 // once fill the chip instead.  Heatbath half-step with its produce(): 8^4 SU(2)
-// 11.5 to 7.7 us, 16^4 12.5 to 9.5; SU(3) 8^4 15.3 to 11.0, 20 x 12 x 28 x 10
-// 24.9 to 20.5, 24^3 x 12 (175 MB of quads) 40.4 to 35.0.  Beyond what the last-level
+// 11.5 to 7.7 us, 16^4 12.5 to 9.3; SU(3) 8^4 15.3 to 11.0, 20 x 12 x 28 x 10
+// 24.9 to 18.7, 24^3 x 12 (175 MB of quads) 40.4 to 30.6.  Beyond what the last-level
 // cache holds the quads come back from memory: SU(2) 32^4 (369 MB) 63.3 to 69.1.
 constexpr size_t kAheadBytes = size_t(192) << 20;
 bool ahead_fits(const qcd_lattice* L)
@@ -2313,8 +2321,13 @@ void ahead_prepare(qcd_lattice* L)
 void launch_ahead(qcd_lattice* L)
 {
     const uint32_t keep = update_quads(L), W = rl_ahead_waves(L->s_quads, keep);
-    hipLaunchKernelGGL(k_ranlux_ahead, dim3((L->n_inst + 63u) / 64u, kRlAhead), dim3(64u * W), rl_lds_bytes(W), L->stream,
-                       L->rl_state, L->rl_next, L->n_inst, L->s_quads, keep, L->ahead_buf, L->rl_tab);
+    if (keep == L->s_quads)
+        hipLaunchKernelGGL(k_ranlux_ahead_turns, dim3(rl_turns_groups(L->n_inst, W), kRlAhead), dim3(64u * (W + 1u)),
+                           rl_turns_lds(W), L->stream, L->rl_state, L->rl_next, L->n_inst, L->s_quads, keep, L->ahead_buf,
+                           L->rl_tab);
+    else
+        hipLaunchKernelGGL(k_ranlux_ahead, dim3((L->n_inst + 63u) / 64u, kRlAhead), dim3(64u * W), rl_lds_bytes(W), L->stream,
+                           L->rl_state, L->rl_next, L->n_inst, L->s_quads, keep, L->ahead_buf, L->rl_tab);
     std::swap(L->rl_state, L->rl_next);
 }
 

@@ -23,6 +23,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <algorithm>
 #include <mutex>
 #include <vector>
 
@@ -456,14 +457,96 @@ __device__ __forceinline__ void rl_ahead(const float4* state, float4* next, uint
     if (t == nb && valid) rl_store(next, n, g, s, carry, k1);
 }
 
-// Wavefronts of rl_ahead: the blocks that `keep` quads can touch, and one for
-// the last block when the last produce() keeps less than all; 0: not on this path.
+// The same for the units first_unit, first_unit + step, ..: wavefronts
+// 0 .. W - 1 keep the table of their block and make it for one unit after the
+// other, wavefront W meanwhile finishes the block that the next unit's streams
+// stand in.  LDS: two buffers of rings, then the W wavefronts' own words.
+// For produce() that keep all quads, where every wavefront has a block for
+// every h: heatbath half-step SU(3) 20 x 12 x 28 x 10 19.9 (a unit per workgroup) /
+// 18.7 us, 16^3 x 32 28.2 / 24.7, 24^3 x 12 34.2 / 30.6; SU(2) (11 of 33 kept, a
+// wavefront in five idle) 16^4 9.3 / 10.8, 32^3 x 16 32.4 / 38.2.
+__device__ __forceinline__ void rl_ahead_turns(const float4* state, float4* next, uint32_t n, uint32_t samples, uint32_t keep,
+                                         float4* quads, uint32_t first_unit, uint32_t step, uint32_t h, const uint4* tab,
+                                         uint32_t* lds, uint32_t W)
+{
+    const uint32_t w = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const uint32_t lane = threadIdx.x & 63, units = (n + 63u) / 64u;
+    const float4 c0 = state[(size_t)6 * n];   // every stream stands at the same place of its block
+    const uint32_t k = min((uint32_t)__builtin_amdgcn_readfirstlane((int)c0.z), 6u);
+    const uint32_t first = 6u - k, total = (uint32_t)kRlAhead * samples, start = h * samples, stop = start + keep;
+    const uint32_t nb = (total - first + 5u) / 6u;
+    quads += (size_t)h * keep * n;
+    auto ring = [&](uint32_t it) { return lds + (it & 1u) * 64u * kRlIn; };
+    if (w == W) {
+        auto finish = [&](uint32_t unit, uint32_t* in) {
+            const uint32_t g0 = unit * 64u + lane, g = min(g0, n - 1u);
+            uint32_t s[24];
+#pragma unroll
+            for (int q = 0; q < 6; ++q) {
+                const float4 v = state[(size_t)q * n + g];
+                s[4 * q] = (uint32_t)(v.x * 16777216.0f);
+                s[4 * q + 1] = (uint32_t)(v.y * 16777216.0f);
+                s[4 * q + 2] = (uint32_t)(v.z * 16777216.0f);
+                s[4 * q + 3] = (uint32_t)(v.w * 16777216.0f);
+            }
+            uint32_t carry = state[(size_t)6 * n + g].w > 0.0f ? 1u : 0u;
+            rl_block(s, carry, k, 6u, 0u - start, keep, quads, n, g, g0 < n);   // numbers below 0 wrap: not kept
+            uint32_t* o = in + lane * kRlIn;
+#pragma unroll
+            for (int q = 0; q < 6; ++q)
+                *reinterpret_cast<uint4*>(o + 4 * q) =
+                    make_uint4((s[4 * q] ^ 0x808080u) | (q == 0 ? carry << 24 : 0u), s[4 * q + 1] ^ 0x808080u,
+                               s[4 * q + 2] ^ 0x808080u, s[4 * q + 3] ^ 0x808080u);
+        };
+        finish(first_unit, ring(0));
+        __syncthreads();
+        uint32_t it = 0;
+        for (uint32_t u = first_unit; u < units; u += step, ++it) {
+            if (u + step < units) finish(u + step, ring(it + 1u));
+            __syncthreads();
+        }
+        return;
+    }
+    // blocks after the current one that hold quads start .. stop - 1
+    const uint32_t lo = start < first ? 1u : 1u + (start - first) / 6u, hi = stop <= first ? 0u : 1u + (stop - 1u - first) / 6u;
+    const bool end = h == (uint32_t)kRlAhead - 1u && w == W - 1u && hi < nb;   // a last block that is not kept
+    const uint32_t t = end ? nb : lo + w, m = first + 6u * (t - 1u);
+    const bool idle = !end && t > hi;
+    RlTab table;
+    if (!idle) rl_load(table, tab + (size_t)(t - 1u) * kRlTaskVec);
+    const uint32_t k1 = idle ? 0u : min(6u, (t == nb ? total : stop) - m);
+    __syncthreads();
+    uint32_t it = 0;
+    for (uint32_t u = first_unit; u < units; u += step, ++it) {
+        if (!idle) {
+            const uint32_t g0 = u * 64u + lane, g = min(g0, n - 1u);
+            uint32_t s[24], carry;
+            rl_jump(table, ring(it), lds + 128u * kRlIn + w * 64u * kRlOut, s, carry);
+            rl_block(s, carry, 0u, k1, m - start, keep, quads, n, g, g0 < n);
+            if (t == nb && g0 < n) rl_store(next, n, g, s, carry, k1);
+        }
+        __syncthreads();
+    }
+}
+
+// Wavefronts W that make blocks: the blocks that `keep` quads can touch, and
+// one for the last block when the last produce() keeps less than all; 0: not on
+// this path.
 inline uint32_t rl_ahead_waves(uint32_t samples, uint32_t keep)
 {
     const uint32_t W = (keep + 4u) / 6u + 1u + (keep < samples ? 1u : 0u);
-    const bool fits = samples >= 6u && keep >= 1u && keep <= samples && ((uint32_t)kRlAhead * samples + 5u) / 6u <= (uint32_t)kRlTasks &&
-                      W <= (uint32_t)kRlWaves;
+    const bool fits = samples >= 6u && keep >= 1u && keep <= samples &&
+                      ((uint32_t)kRlAhead * samples + 5u) / 6u <= (uint32_t)kRlTasks && W < (uint32_t)kRlWaves;
     return fits ? W : 0u;
+}
+// rl_ahead_turns: its LDS, and workgroups per produce(): as many as run at once
+// (16 wavefronts per CU), each with the same number of units.
+inline uint32_t rl_turns_lds(uint32_t W) { return 4u * 64u * (2u * (uint32_t)kRlIn + W * (uint32_t)kRlOut); }
+inline uint32_t rl_turns_groups(uint32_t n, uint32_t W)
+{
+    const uint32_t units = (n + 63u) / 64u, once = 256u * std::min(16u / (W + 1u), 163840u / rl_turns_lds(W)) / (uint32_t)kRlAhead;
+    const uint32_t turns = (units + once - 1u) / once;
+    return (units + turns - 1u) / turns;
 }
 
 // Wavefronts per 64 streams for a produce() of `samples` quads that keeps

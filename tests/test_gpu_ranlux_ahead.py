@@ -34,6 +34,7 @@ def _by_halfsteps(lat):
     dict(sun=3, dims=(4, 4, 4, 4), nhit=3, ranlux_luxury=0),     # 12 of 12
     dict(sun=3, dims=(4, 4, 4, 4), nhit=2, ranlux_luxury=4),     # 9 of 9: blocks shared by half-steps
     dict(sun=2, dims=(4, 4, 4, 4), nhit=11),                     # 36 quads
+    dict(sun=3, dims=(8, 12, 8, 22), storage_reals=12),          # 132 units: two in turn, the last workgroups one
     dict(sun=2, dims=(32, 16, 32, 34)),                          # 197 MB: half-steps produce for themselves
 ])
 def test_sweeps_equal_halfsteps(kw):
