@@ -825,49 +825,28 @@ __global__ __launch_bounds__(256) void k_flow_imh_couple(float4* L, const float*
 // only, and the gradient flows back through conv2, tanh and conv1 alone.
 
 // -log q_a of one active link in double precision (the map of make_spline /
-// spline_inv / log_jac, written for double) and its gradient gr with respect to
-// the 3K + 1 raw spline parameters r; th = angle of U V.  In the bin of th with
-// corners (x0, y0), sizes (w, h), slope s = h / w and end derivatives d0, d1
+// spline_inv / log_jac, written for double) and its gradient gr with respect
+// to the 3K + 1 raw spline parameters r, from the formulas of bin `bin`;
+// pw, ph: the softmax of the widths and heights, th = angle of U V.  In the bin
+// with corners (x0, y0), sizes (w, h), slope s = h / w and end derivatives d0, d1
 // the inverse xi solves y0 + h A / den = th, and
 //   nll = log f' + 2 log(sin th / sin(x0 + xi w)),  f' = s^2 N / den^2,
 // so a parameter p moves it by its direct derivative plus, through xi,
 // -(dy/dp) / (w f') times the derivative in xi.  (Differences of nll at r +- h
-// were 27 evaluations per link: 231 us for 32768 sites, now 8 us.)
-template <int K> __device__ __forceinline__ double nll_grad_link(const float (&rf)[kOut], double th, float (&gr)[kOut])
+// were 27 evaluations per link: 231 us for 32768 sites, now 8 to 11 us.)
+template <int K>
+__device__ __forceinline__ double nll_grad_bin(const float (&rf)[kOut], const double (&pw)[K], const double (&ph)[K], double th,
+                                               int bin, float (&gr)[kOut])
 {
     const double pi = 3.14159265358979323846, ln2i = 1.4426950408889634;
-    double mw = rf[0], mh = rf[K];
-#pragma unroll
-    for (int i = 1; i < K; ++i) {
-        mw = fmax(mw, (double)rf[i]);
-        mh = fmax(mh, (double)rf[K + i]);
-    }
-    double pw[K], ph[K], sw = 0.0, sh = 0.0;
-#pragma unroll
-    for (int i = 0; i < K; ++i) {
-        pw[i] = exp((double)rf[i] - mw);
-        ph[i] = exp((double)rf[K + i] - mh);
-        sw += pw[i];
-        sh += ph[i];
-    }
-#pragma unroll
-    for (int i = 0; i < K; ++i) {
-        pw[i] /= sw;
-        ph[i] /= sh;
-    }
     const double scale = pi * (1.0 - K * (double)kMinW);
-    // the bin of th among the heights' knots, and its corners
     double x0 = 0.0, y0 = 0.0, w = 0.0, h = 0.0, xa = 0.0, ya = 0.0;
-    float r0 = rf[2 * K], r1 = rf[2 * K + 1];
-    int bin = 0;
-    bool go = true;
+    float r0 = 0.f, r1 = 0.f;
 #pragma unroll
     for (int i = 0; i < K; ++i) {
         const double xb = i == K - 1 ? pi : xa + pi * (double)kMinW + scale * pw[i];
         const double yb = i == K - 1 ? pi : ya + pi * (double)kMinW + scale * ph[i];
-        if (i > 0) go = go && th >= ya;
-        if (go) {
-            bin = i;
+        if (i == bin) {
             x0 = xa;
             y0 = ya;
             w = xb - xa;
@@ -922,6 +901,65 @@ template <int K> __device__ __forceinline__ double nll_grad_link(const float (&r
 #pragma unroll
     for (int i = 0; i <= K; ++i)
         gr[2 * K + i] = i == bin ? (float)(g_d0 * dk * sg((double)r0)) : (i == bin + 1 ? (float)(g_d1 * dk * sg((double)r1)) : 0.f);
+    return nll;
+}
+
+// The same in the bin of th.  At a knot nll has a kink in the heights: the
+// gradient is that of the symmetric difference over a step of kKinkStep, the
+// mean of both sides' derivatives weighted by the parts of the step in which the
+// knot lies above and below th.
+constexpr double kKinkStep = 1e-5;
+template <int K> __device__ __forceinline__ double nll_grad_link(const float (&rf)[kOut], double th, float (&gr)[kOut])
+{
+    const double pi = 3.14159265358979323846;
+    double mw = rf[0], mh = rf[K];
+#pragma unroll
+    for (int i = 1; i < K; ++i) {
+        mw = fmax(mw, (double)rf[i]);
+        mh = fmax(mh, (double)rf[K + i]);
+    }
+    double pw[K], ph[K], sw = 0.0, sh = 0.0;
+#pragma unroll
+    for (int i = 0; i < K; ++i) {
+        pw[i] = exp((double)rf[i] - mw);
+        ph[i] = exp((double)rf[K + i] - mh);
+        sw += pw[i];
+        sh += ph[i];
+    }
+#pragma unroll
+    for (int i = 0; i < K; ++i) {
+        pw[i] /= sw;
+        ph[i] /= sh;
+    }
+    const double scale = pi * (1.0 - K * (double)kMinW);
+    // the bin, and the knot (number edge, at y = ye, heights below it se) within reach of a step
+    double ya = 0.0, sa = 0.0, ye = 0.0, se = 0.0;
+    int bin = 0, edge = 0;
+#pragma unroll
+    for (int m = 1; m < K; ++m) {
+        ya += pi * (double)kMinW + scale * ph[m - 1];
+        sa += ph[m - 1];
+        if (th >= ya) bin = m;
+        if (fabs(th - ya) < kKinkStep) {   // |d ya / d r| <= scale / 4 < 1
+            edge = m;
+            ye = ya;
+            se = sa;
+        }
+    }
+    const double nll = nll_grad_bin<K>(rf, pw, ph, th, bin, gr);
+    if (edge) {
+        float go[kOut];
+        const bool up = bin == edge;   // th lies in the bin above the knot
+        (void)nll_grad_bin<K>(rf, pw, ph, th, up ? edge - 1 : edge, go);
+#pragma unroll
+        for (int i = 0; i < K; ++i) {
+            const double dy = scale * ph[i] * ((i < edge ? 1.0 : 0.0) - se);
+            // part of the step with the knot above th, where the lower bin holds
+            const double at = (th - ye) / (2.0 * kKinkStep * fabs(dy));
+            const double low = fmin(fmax(0.5 - at, 0.0), 1.0), other = up ? low : 1.0 - low;
+            if (dy != 0.0) gr[K + i] = (float)(gr[K + i] + other * ((double)go[K + i] - (double)gr[K + i]));
+        }
+    }
     return nll;
 }
 

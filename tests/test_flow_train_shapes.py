@@ -82,3 +82,46 @@ def test_bins_against_autograd(dims, bins):
     for (l, b, u), (_, _, v) in zip(_blocks(g), _blocks(want)):
         cos = float(np.dot(u, v) / (np.linalg.norm(u) * np.linalg.norm(v)))
         assert cos >= 0.99 and np.linalg.norm(u - v) <= 0.1 * np.linalg.norm(v), (l, b, cos)
+
+
+@pytest.mark.parametrize("below", [0.0, 2e-6])
+def test_gradient_at_a_knot(below):
+    """Links whose loop angle lies on the knot pi/2 of a spline with two equal
+    heights, or a part of a step below it: the gradient is the symmetric
+    difference's.  One value on all active sites; BF16 keeps 8 bits of it (2^-8),
+    and the knots' FP32 constants move the step's parts by 1e-3 at most."""
+    import math
+    import os
+    import sys
+
+    sys.path.insert(0, os.path.join(os.path.dirname(os.path.abspath(__file__)), "..", "oracle"))
+    import flow_ref as FR
+
+    print("[case] knot", below, flush=True)
+    dims, K = (4, 4, 4, 4), 2
+    r = np.array([0.7, -0.4, 0.2, 0.2, -0.5, 0.9, 0.3])
+    th = math.pi / 2 - below
+    links = np.zeros((1, 4, 256, 4), dtype=np.float32)
+    links[..., 0] = 1.0
+    for s in range(256):   # sites run y fastest, then z, t, x; direction x is active where y + z + t is even
+        y, z, t = s % 4, (s // 4) % 4, (s // 16) % 4
+        if (y + z + t) % 2 == 0:
+            links[0, 0, s] = (math.cos(th), 0.0, 0.0, math.sin(th))
+    p = np.zeros(QF.LAYER_PARAMS, dtype=np.float32)
+    p[-QF.COUT:-QF.COUT + 7] = r
+    with QF.Flow(dims=dims, layers=1, bins=K, max_batch=1) as f:
+        f.set_params(p)
+        loss, g = f.train_grad(links)
+
+    th = math.atan2(float(links[0, 0, 0, 3]), float(links[0, 0, 0, 0]))
+    r = p[-QF.COUT:-QF.COUT + 7].astype(np.float64)
+
+    def nll(q):
+        x, dlog = FR.spline(q, K, th, inverse=True)
+        return dlog + 2 * math.log(math.sin(th) / math.sin(x))
+
+    want = np.array([(nll(r + 1e-5 * e) - nll(r - 1e-5 * e)) / 2e-5 for e in np.eye(7)])
+    got = g[-QF.COUT:-QF.COUT + 7] / 128.0
+    print("  ", got, want)
+    assert abs(loss - 128 * nll(r)) <= 1e-4 * 128
+    assert np.all(np.abs(got - want) <= 2.0 ** -8 * np.abs(want) + 1e-3 * np.abs(want).max())
