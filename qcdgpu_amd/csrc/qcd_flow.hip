@@ -1017,11 +1017,11 @@ __global__ __launch_bounds__(256) void k_flow_nll_grad(const float4* L, const fl
 // workgroups share a plane's rows.  Wavefront w takes the offsets (oy, oz, ot) =
 // w, w + 8, .. with all three ox, and goes on to further units with the same
 // sums; one partial array per workgroup.
-// For 16 configurations of 8^3 x 4 (128 planes): 32 -> 16 channels 15 us, 8 ->
-// 32 channels 9 us, against 240 and 142 us of k_flow_wgrad, whose every operand
-// element is a load; 23 and 19 with one workgroup per plane and 16-row steps.
-// The matrix instructions take 2.6 us of the 15, the transposed reads 6 (25 of
-// 512 bytes per wavefront and 16 rows).
+// For 16 configurations of 8^3 x 4 (128 planes): 32 -> 16 channels 21 us, 8 ->
+// 32 channels 14.5 us, against 240 and 142 us of k_flow_wgrad, whose every operand
+// element is a load.  A good half of it is staging (57 kB per workgroup before the
+// first read) and the partial arrays (166 kB per workgroup, 42 MB in all, which
+// k_flow_sum_parts reads back in 9 us); the matrix instructions take 2.6 us.
 constexpr int kGradWaves = 8, kGradOffs = 4;   // 27 offsets over 8 wavefronts
 constexpr uint32_t kGradRows = 32;
 template <int C, int N>
@@ -1665,7 +1665,7 @@ int train_grad(qcd_flow* F, const float* links, int batch, double* loss)
     const size_t nmax = (size_t)F->d.max_batch * g.V;
     // weight gradients from x-planes in LDS where those fit, one partial
     // array per workgroup; else from chunks of rows
-    constexpr uint32_t kChunk = 512, kGradGroups = 256;   // one workgroup per CU
+    constexpr uint32_t kChunk = 512, kGradGroups = 256;   // one workgroup per CU; 128 cost 15 % at 64 configurations
     const uint32_t plane = g.V / (uint32_t)g.n1, lds2 = plane * (3u * 2 * kHidden + 2 * kOut),
                    lds1 = plane * (3u * 2 * kCin0 + 2 * kHidden);
     const bool by_plane = plane % 16 == 0 && lds2 <= 64u * 1024u;
