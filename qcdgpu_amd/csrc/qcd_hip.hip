@@ -2301,6 +2301,20 @@ bool ahead_fits(const qcd_lattice* L)
     return rl_waves(L->p.ranlux_luxury, L->s_quads, keep, L->n_inst) && rl_ahead_waves(L->s_quads, keep) &&
            sizeof(float4) * kRlAhead * keep * (size_t)L->n_inst <= kAheadBytes;
 }
+// Allocations and waits of a lattice while this thread records another one's
+// graph: those calls would end that recording otherwise.
+struct OutsideCapture {
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    bool ok;
+    OutsideCapture() : ok(hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess) {}
+    ~OutsideCapture()
+    {
+        if (ok) (void)hipThreadExchangeStreamCaptureMode(&mode);
+    }
+    OutsideCapture(const OutsideCapture&) = delete;
+    OutsideCapture& operator=(const OutsideCapture&) = delete;
+};
+
 // Its buffers, before a sweep or a capture of sweeps; without them (no memory,
 // or a capture under way) every half-step produces for itself.
 void ahead_prepare(qcd_lattice* L)
@@ -2308,6 +2322,7 @@ void ahead_prepare(qcd_lattice* L)
     if (!ahead_fits(L) || (L->ahead_buf && L->ahead_quads >= update_quads(L))) return;
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(L->stream, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) return;
+    const OutsideCapture outside;
     (void)hipStreamSynchronize(L->stream);
     (void)hipFree(L->ahead_buf);
     L->ahead_buf = nullptr;
@@ -3582,6 +3597,7 @@ static int move_links(qcd_lattice* L, double* out, const double* in)
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     HIPCHK(hipStreamIsCapturing(L->stream, &cap));
     if (cap != hipStreamCaptureStatusNone) return fail(QCD_E_HIP, "links cannot be copied while the stream is recorded");
+    const OutsideCapture outside;
     int dev = 0;
     HIPCHK(hipGetDevice(&dev));
     const int N = L->p.sun, np = L->np;

@@ -63,3 +63,27 @@ def test_sweeps_equal_halfsteps(kw):
             assert np.array_equal(a.save_state(), b.save_state())
     a.close()
     b.close()
+
+
+def test_beside_a_recording():
+    """A first sweep and an export of one lattice while another one's graph is recorded: both give
+    what they give alone."""
+    print("[case] beside a recording", flush=True)
+    kw = dict(sun=3, dims=(4, 4, 4, 4))
+    a, b, c = _lattice(**kw), _lattice(**kw), _lattice(**kw)
+    a.graph_begin()
+    a.sweep("hb")
+    b.sweep("hb")
+    links = b.export_links()
+    a.sweep("or")
+    a.graph_end()
+    for _ in range(3):
+        a.launch_cycle(1)
+        a.sync()
+        _by_halfsteps(c)
+        if _ == 0:
+            assert np.array_equal(links, c.export_links())
+        c.sweep("or")
+        assert np.array_equal(a.export_links(), c.export_links())
+    for lat in (a, b, c):
+        lat.close()
