@@ -36,9 +36,11 @@
 #include <cstdlib>
 #include <cstring>
 #include <ctime>
+#include <exception>
+#include <memory>
 #include <mutex>
+#include <new>
 #include <string>
-#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -3503,8 +3505,8 @@ StageUser::~StageUser()
 
 struct Stage {
     void* mem = nullptr;
-    size_t bytes;
-    explicit Stage(size_t n) : bytes(n)
+    size_t bytes = 0;
+    bool get(size_t n)
     {
         {
             std::lock_guard<std::mutex> lock(stage_mutex);
@@ -3512,9 +3514,16 @@ struct Stage {
                 mem = stage_kept;
                 bytes = stage_kept_bytes;
                 stage_kept = nullptr;
+                return true;
             }
         }
-        if (!mem && hipHostMalloc(&mem, n, hipHostMallocPortable) != hipSuccess) mem = nullptr;
+        if (hipHostMalloc(&mem, n, hipHostMallocPortable) != hipSuccess) {
+            (void)hipGetLastError();
+            mem = nullptr;
+            return false;
+        }
+        bytes = n;
+        return true;
     }
     ~Stage()
     {
@@ -3591,6 +3600,42 @@ static void launch_links_move(qcd_lattice* L, void* host, uint32_t i0, uint32_t 
     else hipLaunchKernelGGL((k_links_move<C, 2, IN>), nb, dim3(256), 0, L->stream, t, h, L->g, i0, npairs);
 }
 
+// Without pinned memory: the whole table in one copy to or from ordinary
+// memory, its planes walked site by site.
+template <typename F> static int move_links_pageable(qcd_lattice* L, double* out, const double* in)
+{
+    const int N = L->p.sun, np = L->np;
+    const Geom& g = L->g;
+    const size_t at = (size_t)N * N * 8, row = 8 * (size_t)np;   // doubles and stored reals of a site
+    std::unique_ptr<F[]> t(new (std::nothrow) F[L->table_bytes / sizeof(F)]());
+    if (!t) return fail(QCD_E_NOMEM, "host memory for the links (%zu bytes)", L->table_bytes);
+    if (out) {
+        HIPCHK(hipMemcpyAsync(t.get(), L->table, L->table_bytes, hipMemcpyDeviceToHost, L->stream));
+        HIPCHK(hipStreamSynchronize(L->stream));
+    }
+    F c[8 * 9];
+    for (uint32_t i = 0; i < g.vh; ++i) {
+        const uint32_t q = g.dh.div(i), r = g.d3.div(q), x = g.d4.div(r);
+        const uint32_t par0 = (x + (q - r * (uint32_t)g.n3) + (r - x * (uint32_t)g.n4)) & 1u;
+        for (uint32_t k = 0; k < 2; ++k) {   // the pair's sites, y even and odd
+            const size_t s = 2 * (size_t)i + k;
+            F* p = t.get() + 2 * ((size_t)(par0 ^ k) * 4 * (size_t)np * g.vh_pad + i);
+            if (in) pack_links(in + s * at, c, 1, N, np);
+            for (size_t j = 0; j < row; ++j) {
+                F& e = p[2 * (j / 2) * (size_t)g.vh_pad + j % 2];
+                if (in) e = c[j];
+                else c[j] = e;
+            }
+            if (out) unpack_links(c, out + s * at, 1, N, np);
+        }
+    }
+    if (in) {
+        HIPCHK(hipMemcpyAsync(L->table, t.get(), L->table_bytes, hipMemcpyHostToDevice, L->stream));
+        HIPCHK(hipStreamSynchronize(L->stream));
+    }
+    return QCD_OK;
+}
+
 // Export (out) or import (in); returns when the transfer is complete.
 static int move_links(qcd_lattice* L, double* out, const double* in)
 {
@@ -3609,9 +3654,10 @@ static int move_links(qcd_lattice* L, double* out, const double* in)
     const size_t slot_bytes = std::clamp(V * per_site / kLinkSlots, kLinkSlotMin, kLinkSlotMax);
     const size_t chunk = std::min(slot_bytes / per_site / (2 * kMovePairs) * (2 * kMovePairs), V);   // sites
     const size_t nchunks = (V + chunk - 1) / chunk;
-    const uint32_t workers = (uint32_t)std::min<size_t>(kLinkSlots, nchunks);
-    Stage st(chunk * per_site * workers);
-    if (!st.mem) return fail(QCD_E_NOMEM, "pinned memory for the links (%zu bytes)", chunk * per_site * workers);
+    uint32_t workers = (uint32_t)std::min<size_t>(kLinkSlots, nchunks);
+    Stage st;
+    while (workers && !st.get(chunk * per_site * workers)) workers /= 2;   // fewer slots where little can be pinned
+    if (!workers) return f32 ? move_links_pageable<float>(L, out, in) : move_links_pageable<double>(L, out, in);
     hipEvent_t ev[kLinkSlots] = {};
     std::atomic<int> err{(int)hipSuccess};
     auto keep = [&](hipError_t e) {
@@ -3650,7 +3696,7 @@ static int move_links(qcd_lattice* L, double* out, const double* in)
         for (uint32_t w = 1; w < workers; ++w) {
             try {
                 th[w] = std::thread(work, w);
-            } catch (const std::system_error&) {
+            } catch (const std::exception&) {
                 break;   // no more threads: those there are take all chunks
             }
         }

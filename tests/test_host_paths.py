@@ -1,0 +1,78 @@
+"""The library's host side without a GPU: libqcdhip.so on a stand-in for the HIP
+runtime (fake_hip.c: host memory for device memory, kernels not run, every call
+noted, allocations that can be made to fail).  Each test is a program of its own,
+since the stand-in has to be loaded before the library."""
+import os
+import shutil
+import subprocess
+import sys
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+REPO = os.path.dirname(HERE)
+
+pytestmark = [
+    pytest.mark.skipif(not os.path.exists(os.path.join(REPO, "qcdgpu_amd", "libqcdhip.so")), reason="libqcdhip.so not built"),
+    pytest.mark.skipif(shutil.which("gcc") is None, reason="gcc missing"),
+]
+
+PRELUDE = """
+import ctypes, sys
+fake = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
+fake.fake_log.restype = ctypes.c_char_p
+fake.fake_limits.argtypes = [ctypes.c_size_t, ctypes.c_size_t]
+ANY = 2 ** 64 - 1
+sys.path[:0] = %r
+def calls():
+    lines = fake.fake_log().decode().splitlines()
+    fake.fake_clear()
+    return lines
+import numpy as np
+import qcdgpu_amd as Q
+"""
+
+
+@pytest.fixture(scope="module")
+def fake(tmp_path_factory):
+    out = str(tmp_path_factory.mktemp("fake") / "libfakehip.so")
+    r = subprocess.run(["gcc", "-shared", "-fPIC", "-O1", "-o", out, os.path.join(HERE, "fake_hip.c"), "-lpthread"],
+                       capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr
+    return out
+
+
+def _run(fake, code):
+    r = subprocess.run([sys.executable, "-c", PRELUDE % [REPO, HERE] + code, fake], capture_output=True, text=True,
+                       timeout=120)
+    assert r.returncode == 0, r.stdout + r.stderr
+
+
+@pytest.mark.parametrize("precision", ["fp32", "fp64"])
+@pytest.mark.parametrize("sun,storage", [(2, 4), (3, 12), (3, 18)])
+def test_links_without_pinned_memory(fake, sun, storage, precision):
+    """Import and export need ordinary memory only: no slot can be pinned here."""
+    _run(fake, """
+from test_gpu_links_move import _links, _stored
+fake.fake_limits(ANY, 0)
+for dims in ((2, 2, 2, 2), (6, 10, 2, 4), (4, 6, 10, 6)):
+    with Q.Lattice(sun=%d, dims=dims, precision="%s", storage_reals=%d, max_measurements=2) as lat:
+        a = _links(lat, 3)
+        lat.import_links(a)
+        assert np.array_equal(lat.export_links(), _stored(a, %d, %d, "%s")), dims
+        assert not any("launch" in c for c in calls())
+""" % (sun, precision, storage, sun, storage, precision))
+
+
+def test_links_with_little_pinned_memory(fake):
+    """Where eight slots cannot be pinned, fewer are taken."""
+    _run(fake, """
+fake.fake_limits(ANY, 3 << 20)
+with Q.Lattice(sun=3, dims=(16, 16, 16, 16), max_measurements=2) as lat:
+    calls()
+    lat.export_links()
+    seen = calls()
+pinned = [c for c in seen if c.startswith("hostmalloc")]
+assert pinned and not pinned[-1].endswith("failed"), pinned
+assert sum(c.startswith("launch") for c in seen) > 8 and not any(c.startswith("copy") for c in seen)
+""")
