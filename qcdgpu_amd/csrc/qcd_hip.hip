@@ -1913,14 +1913,6 @@ __global__ __launch_bounds__(kBlock) void k_finalize_batch(const ChainDesc* cd, 
 // ============================================================================
 __device__ __align__(256) double scratch[kScratchBytesDev / sizeof(double)];
 
-// One of the lattices that keep the pinned transfer buffer alive.
-struct StageUser {
-    StageUser();
-    ~StageUser();
-    StageUser(const StageUser&) = delete;
-    StageUser& operator=(const StageUser&) = delete;
-};
-
 struct qcd_lattice {
     qcd_params p;
     Geom g;
@@ -2003,7 +1995,6 @@ struct qcd_lattice {
     // lattice's buffers and stream sizing, so neither may change (no
     // re-sizing start, no destroy except through the batch).
     bool batch_owned = false;
-    StageUser stage_user;
     // x-slab (one GPU's share of a lattice cut along x): the slices x = 0 and
     // x = N1 - 1 are halos that the updates read and never write; they are
     // refreshed through qcd_slab_face.
@@ -2603,6 +2594,8 @@ int qcdhip::lattice_dims(const qcd_lattice* L, int n[4])
     return QCD_OK;
 }
 
+static void stage_release();   // the pinned memory of the link transfers
+
 // ---------------------------------------------------------------- C ABI
 extern "C" {
 
@@ -2631,6 +2624,7 @@ int qcd_device_open(int platform, int device)
 int qcd_device_close(void)
 {
     if (g_device >= 0) HIPCHK(hipDeviceSynchronize());
+    stage_release();
     g_device = -1;
     return QCD_OK;
 }
@@ -3481,26 +3475,20 @@ __global__ __launch_bounds__(256) void k_links_move(C* table, C* host, Geom g, u
     }
 }
 
-// Pinned memory for one transfer; one buffer is kept between calls as long as
-// any lattice lives.
+// Pinned memory for one transfer; one buffer, at most kLinkSlots kLinkSlotMax
+// (16 MiB), is kept between calls until qcd_device_close.  (Given back with the
+// last lattice it cost programs that make a lattice per configuration: create,
+// import, destroy of SU(2) 16^3 x 8 1.4 to 1.7 ms, SU(3) 16^4 2.7 to 3.1 ms; kept,
+// 0.40 and 1.20 ms.)
 static std::mutex stage_mutex;
 static void* stage_kept = nullptr;
 static size_t stage_kept_bytes = 0;
-static int stage_users = 0;
 
-StageUser::StageUser()
+static void stage_release()
 {
     std::lock_guard<std::mutex> lock(stage_mutex);
-    ++stage_users;
-}
-
-StageUser::~StageUser()
-{
-    std::lock_guard<std::mutex> lock(stage_mutex);
-    if (--stage_users == 0 && stage_kept) {
-        (void)hipHostFree(stage_kept);
-        stage_kept = nullptr;
-    }
+    if (stage_kept) (void)hipHostFree(stage_kept);
+    stage_kept = nullptr;
 }
 
 struct Stage {

@@ -70,7 +70,11 @@ hipError_t hipFree(void* p)
     free(p);
     return hipSuccess;
 }
-hipError_t hipHostFree(void* p) { return hipFree(p); }
+hipError_t hipHostFree(void* p)
+{
+    free(p);
+    return note(hipSuccess, "hostfree", 0, 0, 0);
+}
 hipError_t hipMemcpy(void* d, const void* s, size_t n, int kind)
 {
     memcpy(d, s, n);

@@ -76,3 +76,20 @@ pinned = [c for c in seen if c.startswith("hostmalloc")]
 assert pinned and not pinned[-1].endswith("failed"), pinned
 assert sum(c.startswith("launch") for c in seen) > 8 and not any(c.startswith("copy") for c in seen)
 """)
+
+
+def test_pinned_memory_outlives_a_lattice(fake):
+    """A lattice per configuration: the pinned memory is had once and given back by
+    qcd_device_close, not with every last lattice."""
+    _run(fake, """
+from qcdgpu_amd import _abi
+calls()
+for _ in range(3):
+    with Q.Lattice(sun=2, dims=(16, 16, 16, 8), max_measurements=2) as lat:
+        lat.import_links(lat.export_links())
+seen = calls()
+assert sum(c.startswith("hostmalloc") for c in seen) == 1, seen
+assert "hostfree" not in seen
+assert _abi.lib().qcd_device_close() == 0
+assert calls().count("hostfree") == 1
+""")
