@@ -1543,13 +1543,25 @@ template <typename R, int N, int NREAL, bool TW>
 __device__ __forceinline__ M<R, N> line_product(const Table<R, N, NREAL>& T, const Geom& g, const Twist& tw, Site s,
                                                 int dir, int len)
 {
-    M<R, N> P;
-    for (int k = 0; k < len; ++k) {
+    auto ld = [&] {
         const uint32_t idx = cindex(g, s.x, s.y, s.z, s.t);
         M<R, N> m = T.load((s.x + s.y + s.z + s.t) & 1, dir, idx);
         if constexpr (TW) tbc(m, tw, dir, idx);
-        P = k ? m_mul(P, m) : m;
-        shift(g, s, dir, +1);
+        return m;
+    };
+    M<R, N> P;
+    if constexpr (sizeof(R) == 4 && (NREAL == 12) == TW) {   // fewer registers; SU(3) 16^4 7 x 2 35.2 us, else 36.3
+        P = ld();
+        for (int k = 1; k < len; ++k) {
+            shift(g, s, dir, +1);
+            P = m_mul(P, ld());
+        }
+    } else {   // the first load in the loop too: 12 reals 16^4 10 x 3 41.6 us, ahead of it 43.6
+        for (int k = 0; k < len; ++k) {
+            const M<R, N> m = ld();
+            P = k ? m_mul(P, m) : m;
+            shift(g, s, dir, +1);
+        }
     }
     return P;
 }
@@ -1587,8 +1599,16 @@ __device__ __forceinline__ void line_products(const Table<R, N, NREAL>& T, const
     }
 }
 
+// Wavefronts per SIMD that the registers of G = 1 leave room for.  A few more than
+// 64 or 128 registers cost one of them where the lattice fills the SIMDs: FP32
+// SU(2) 32^3 x 16 10 x 3 86.5 us (68 registers), now 74; SU(3) 12 reals 20 x 28 x
+// 12 x 30 125.7 (130), now 107; 18 reals 157.8 (132), now 154.  Twisted, only 12
+// reals gain (131 to 108); 18 reals 16^4 7 x 2 would take 38.5 us for 36.0.
 template <typename R, int N, int NREAL, bool TW, uint32_t G>
-__global__ __launch_bounds__(G * kBlock) void k_wilson(void* table, Geom g, int wr, int wt, double* partials, Twist tw)
+constexpr int kWilsonWaves = G != 1 || sizeof(R) != 4 || (TW && NREAL != 12) ? 1 : (N == 3 ? 4 : 8);
+
+template <typename R, int N, int NREAL, bool TW, uint32_t G>
+__global__ __launch_bounds__(G * kBlock, (kWilsonWaves<R, N, NREAL, TW, G>)) void k_wilson(void* table, Geom g, int wr, int wt, double* partials, Twist tw)
 {
     __shared__ double sums[G][kBlock], sm[kBlock / 64];
     const uint32_t blk = xcd_block(blockIdx.x, gridDim.x);
