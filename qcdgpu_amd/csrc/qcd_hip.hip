@@ -1608,10 +1608,11 @@ template <typename R, int N, int NREAL, bool TW, uint32_t G>
 constexpr int kWilsonWaves = G != 1 || sizeof(R) != 4 || (TW && NREAL != 12) ? 1 : (N == 3 ? 4 : 8);
 
 template <typename R, int N, int NREAL, bool TW, uint32_t G>
-__global__ __launch_bounds__(G * kBlock, (kWilsonWaves<R, N, NREAL, TW, G>)) void k_wilson(void* table, Geom g, int wr, int wt, double* partials, Twist tw)
+__global__ __launch_bounds__(G * kBlock, (kWilsonWaves<R, N, NREAL, TW, G>)) void k_wilson(
+    void* table, Geom g, int wr, int wt, bool by_xcd, double* partials, Twist tw)
 {
     __shared__ double sums[G][kBlock], sm[kBlock / 64];
-    const uint32_t blk = xcd_block(blockIdx.x, gridDim.x);
+    const uint32_t blk = by_xcd ? xcd_block(blockIdx.x, gridDim.x) : blockIdx.x;
     const uint32_t tid = threadIdx.x % kBlock, site = blk * kBlock + tid;
     const int d0 = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kBlock));
     double v = 0.0;
@@ -2479,10 +2480,19 @@ int launch_simple(qcd_lattice* L, int which, const LaunchOpt& o)
             // direction.  SU(3) is bound by its products and gains nothing
             // (16^4 7 x 2: 34.0 us against 33.9).
             const bool by_dir = N == 2 && L->wil_blocks <= 256u;
+            // One x-slab per XCD, but not for lines of five or more FP64 SU(3)
+            // links whose x-planes lie powers of two apart.  18 reals, slabs /
+            // hardware order: 32^3 x 16 1 x 1 87 / 104 us, 7 x 2 288 / 255, 10 x 3
+            // 394 / 343; 32^3 x 12 4 x 4 162 / 161, 5 x 2 164 / 149; but 32 x 24^3
+            // 7 x 2 241 / 270, 12 x 12 502 / 715, 32^3 x 4 7 x 2 65.5 / 68.6, 16^4
+            // 6 x 6 44 / 63.
+            const Geom& g = L->g;
+            const bool by_xcd = !(N == 3 && sizeof(R) == 8 && L->wil_R >= 5 && (uint32_t)g.n2 * g.n3 % 1024u == 0 &&
+                                  (uint64_t)g.n2 * g.n3 * g.n4 >= 8192u);
             auto wilson = [&](auto tw, auto groups) {
                 constexpr uint32_t G = decltype(groups)::value;
                 hipLaunchKernelGGL((k_wilson<R, N, NREAL, decltype(tw)::value, G>), dim3(L->wil_blocks), dim3(G * kBlock), 0,
-                                   L->stream, L->table, L->g, L->wil_R, L->wil_T, L->part_wil, L->tw);
+                                   L->stream, L->table, L->g, L->wil_R, L->wil_T, by_xcd, L->part_wil, L->tw);
             };
             auto with_tw = [&](auto groups) {
                 if (L->tw.on) wilson(std::true_type{}, groups);
