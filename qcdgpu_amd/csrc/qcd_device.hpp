@@ -496,6 +496,33 @@ __host__ __device__ __forceinline__ uint32_t step_bwd(const Step& s, uint32_t i,
     return i + (c > 0 ? in : s.wrap);
 }
 
+// The same steps as branches on the direction, whose sides the compiler keeps
+// apart: for the one-wavefront update, where a wavefront goes over three
+// directions and the selects above crowd out its gathers (staple_nu).
+__host__ __device__ __forceinline__ int extent(const Geom& g, int d)
+{
+    return d == 0 ? g.n1 : (d == 1 ? g.n2 : (d == 2 ? g.n3 : g.n4));
+}
+__host__ __device__ __forceinline__ uint32_t cstride(const Geom& g, int d)
+{
+    return d == 0 ? (uint32_t)g.h * (uint32_t)g.n3 * (uint32_t)g.n4
+                  : (d == 2 ? (uint32_t)g.h : (uint32_t)g.h * (uint32_t)g.n3);
+}
+__host__ __device__ __forceinline__ uint32_t step_fwd(const Geom& g, uint32_t i, int d, int c, uint32_t o)
+{
+    const int n = extent(g, d);
+    if (d == 1) return (c < n - 1) ? i + o : i - (uint32_t)(g.h - 1);
+    const uint32_t st = cstride(g, d);
+    return (c < n - 1) ? i + st : i - st * (uint32_t)(n - 1);
+}
+__host__ __device__ __forceinline__ uint32_t step_bwd(const Geom& g, uint32_t i, int d, int c, uint32_t o)
+{
+    const int n = extent(g, d);
+    if (d == 1) return (c > 0) ? i - (1u - o) : i + (uint32_t)(g.h - 1);
+    const uint32_t st = cstride(g, d);
+    return (c > 0) ? i - st : i + st * (uint32_t)(n - 1);
+}
+
 __host__ __device__ __forceinline__ uint32_t cindex(const Geom& g, int x, int y, int z, int t)
 {
     return (uint32_t)(y >> 1) + (uint32_t)g.h * ((uint32_t)z + (uint32_t)g.n3 * ((uint32_t)t + (uint32_t)g.n4 * (uint32_t)x));

@@ -330,7 +330,13 @@ __device__ __forceinline__ C<R> ua_entry(const M<R, 3>& U, const M<R, 3>& A, int
 // (suncpp/Update/sun_update.h:44-77; su3_update_cl.cl:341-565).  nu, mu and
 // the parity p are wavefront-uniform.  TW: apply the twisted boundary (a
 // separate instantiation, so the untwisted kernels carry none of its code).
-template <typename R, int N, int NREAL, bool TW = false>
+// BRANCH: neighbour steps as branches.  The one-wavefront update of SU(2) and of
+// FP32 18-real SU(3) is faster so (SU(3) PM heatbath half-step, selects / branches:
+// 8^4 17.9 / 12.8 us, 32^3 x 8 33.3 / 22.5, 20 x 12 x 28 x 10 28.4 / 15.4, 48 x 32^2 x
+// 24 118.6 / 91.0; SU(2) FP32 overrelaxation 48 x 32^2 x 24 19.3 / 17.1), the other
+// SU(3) storages slower (FP64 18 reals 8^4 overrelaxation 11.0 / 12.5, 12 reals FP32
+// 4^4 batch of 24 314 / 373 a sweep), as are all three-wavefront kernels.
+template <typename R, int N, int NREAL, bool TW = false, bool BRANCH = false>
 __device__ __forceinline__ M<R, N> staple_nu(const Table<R, N, NREAL>& T, const Geom& g, Site s, uint32_t i, int p,
                                              int mu, int nu, const Twist& tw = Twist{})
 {
@@ -341,11 +347,19 @@ __device__ __forceinline__ M<R, N> staple_nu(const Table<R, N, NREAL>& T, const 
     // matrices in flight at four wavefronts per SIMD.
     const int cmu = coord(s, mu), cnu = coord(s, nu);
     const uint32_t o = (uint32_t)s.y & 1u;
-    const Step smu = step_of(g, mu), snu = step_of(g, nu);
-    const uint32_t i_pmu = step_fwd(smu, i, cmu, o);
-    const uint32_t i_pnu = step_fwd(snu, i, cnu, o);
-    const uint32_t i_mnu = step_bwd(snu, i, cnu, o);
-    const uint32_t i_pmu_mnu = step_bwd(snu, i_pmu, cnu, o);
+    uint32_t i_pmu, i_pnu, i_mnu, i_pmu_mnu;
+    if constexpr (BRANCH) {
+        i_pmu = step_fwd(g, i, mu, cmu, o);
+        i_pnu = step_fwd(g, i, nu, cnu, o);
+        i_mnu = step_bwd(g, i, nu, cnu, o);
+        i_pmu_mnu = step_bwd(g, i_pmu, nu, cnu, o);
+    } else {
+        const Step smu = step_of(g, mu), snu = step_of(g, nu);
+        i_pmu = step_fwd(smu, i, cmu, o);
+        i_pnu = step_fwd(snu, i, cnu, o);
+        i_mnu = step_bwd(snu, i, cnu, o);
+        i_pmu_mnu = step_bwd(snu, i_pmu, cnu, o);
+    }
     M<R, N> S;
     if constexpr (N == 3 && NREAL == 12 && sizeof(R) == 4 && !TW) {
         // FP32, 12 reals: each product is formed before the gathers that
@@ -772,9 +786,10 @@ __device__ __forceinline__ void update1(const UpdArgs& a, uint32_t unit, uint32_
     m_zero(A);
     m_zero(Alow);
     if (active) {
+        constexpr bool kBranch = N == 2 || (NREAL == 18 && sizeof(R) == 4);
         for (int k = 0; k < 3; ++k) {
             const int nu = k + (k >= mu ? 1 : 0);
-            const M<R, N> S = staple_nu<R, N, NREAL>(Ts, a.g, s, i, p, mu, nu);
+            const M<R, N> S = staple_nu<R, N, NREAL, false, kBranch>(Ts, a.g, s, i, p, mu, nu);
             m_acc(A, S);
             if constexpr (MEAS) {
                 if (nu < mu) m_acc(Alow, S);

@@ -58,6 +58,9 @@ def _waves(vgprs):
     ("k_wilsonIfLi3ELi12ELb0ELj1E", 4),
     ("k_wilsonIfLi3ELi12ELb1ELj1E", 4),
     ("k_wilsonIfLi3ELi18ELb0ELj1E", 4),
+    ("k_update1IfLi3ELi18ELb0ELi2ELb1E", 4),        # one wavefront per 64 links, heatbath with the plaquette
+    ("k_update1IfLi3ELi18ELb0ELi3ELb1E", 4),
+    ("k_update_batch1IfLi3ELi18ELb0ELi2ELb1E", 4),
 ])
 def test_wavefronts_per_simd(registers, kernel, waves):
     found = [v for n, v in registers.items() if kernel in n]
