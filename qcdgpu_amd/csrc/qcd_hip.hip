@@ -601,7 +601,8 @@ __device__ __forceinline__ double update_link(const UpdArgs& a, const Table<R, N
 // MU >= 0: the direction is a compile-time constant (the neighbour steps
 // and plane bases fold away, shortening the scalar prologue before the
 // gathers); MU = -1 reads it from the arguments.
-template <typename R, int N, int NREAL, bool OVER, int RK, bool MEAS, bool TW = false, int MU = -1>
+template <typename R, int N, int NREAL, bool OVER, int RK, bool MEAS, bool TW = false, int MU = -1,
+          bool PIN = !(OVER && sizeof(R) == 8)>
 __device__ __forceinline__ void update3(const UpdArgs& a, uint32_t blk, uint32_t nunits)
 {
     using T = R;   // compute type of the SU(2) subgroup arithmetic
@@ -659,8 +660,9 @@ __device__ __forceinline__ void update3(const UpdArgs& a, uint32_t blk, uint32_t
     // of 78, and 2048 workgroups no longer fit the chip at once (32^3 x 8
     // FP32: overrelaxation 17.9 us, 16.9 with it; heatbath 21.0 and 20.1).
     // FP64 overrelaxation has too few wavefronts either way and gains from
-    // the loads in flight (24^3 x 12: 24.9 us with it, 22.7 without).
-    if constexpr (N == 3 && !(OVER && sizeof(R) == 8)) pin(S);
+    // the loads in flight (24^3 x 12: 24.9 us with it, 22.7 without), but for large
+    // batches (launch_batch_map).
+    if constexpr (N == 3 && PIN) pin(S);
     // Wavefront 0 issues the load of the link it updates before the
     // barrier, so its latency overlaps the wait for the other shares rather
     // than following it.
@@ -1875,7 +1877,7 @@ __device__ __forceinline__ UpdArgs chain_args(const ChainDesc* cd, uint32_t c, i
     return a;
 }
 
-template <typename R, int N, int NREAL, bool OVER, int RK, bool MEAS>
+template <typename R, int N, int NREAL, bool OVER, int RK, bool MEAS, bool PIN>
 __global__ __launch_bounds__(kUpdThreads) void k_update_batch3(const ChainDesc* cd, const uint2* map, int parity,
                                                                int mu, int meas_mode, int rng_cur)
 {
@@ -1883,7 +1885,7 @@ __global__ __launch_bounds__(kUpdThreads) void k_update_batch3(const ChainDesc* 
     const uint32_t u = __builtin_amdgcn_readfirstlane(map[blockIdx.x].y);
     if (c == ~0u) return;   // whole workgroup idle
     const UpdArgs a = chain_args(cd, c, parity, mu, meas_mode, rng_cur);
-    update3<R, N, NREAL, OVER, RK, MEAS>(a, u, cd[c].nunits);
+    update3<R, N, NREAL, OVER, RK, MEAS, false, -1, PIN>(a, u, cd[c].nunits);
 }
 
 template <typename R, int N, int NREAL, bool OVER, int RK, bool MEAS>
@@ -4674,6 +4676,7 @@ struct qcd_batch {
     };
     std::vector<Bucket> buckets;
     std::vector<uint2> h_map;              // host copy of d_map
+    size_t table_bytes = 0;                // links of all chains
     // Merged maps (merge on): per update kind [heatbath, overrelaxation] and
     // kernel shape [3, 1], the chosen maps of every bucket with that shape,
     // concatenated, so one launch per (parity, mu) and shape updates all
@@ -4859,12 +4862,26 @@ void launch_batch_map(qcd_batch* B, int shape, const uint2* map, uint32_t len, i
                    map, parity, mu, meas_mode, B->rng_cur);
     } else {
         const dim3 grid(len), block(kUpdThreads);
-        if (meas_mode)
-            launch(k_update_batch3<R, N, NREAL, OVER, RK, true>, grid, block, B->stream, o, (const ChainDesc*)B->d_desc,
-                   map, parity, mu, meas_mode, B->rng_cur);
-        else
-            launch(k_update_batch3<R, N, NREAL, OVER, RK, false>, grid, block, B->stream, o, (const ChainDesc*)B->d_desc,
-                   map, parity, mu, meas_mode, B->rng_cur);
+        auto go = [&](auto pinned) {
+            constexpr bool PIN = decltype(pinned)::value;
+            if (meas_mode)
+                launch(k_update_batch3<R, N, NREAL, OVER, RK, true, PIN>, grid, block, B->stream, o,
+                       (const ChainDesc*)B->d_desc, map, parity, mu, meas_mode, B->rng_cur);
+            else
+                launch(k_update_batch3<R, N, NREAL, OVER, RK, false, PIN>, grid, block, B->stream, o,
+                       (const ChainDesc*)B->d_desc, map, parity, mu, meas_mode, B->rng_cur);
+        };
+        if constexpr (NREAL == 18 && OVER && sizeof(R) == 8) {
+            // FP64 overrelaxation: two wavefronts per SIMD with all gathers in
+            // flight, or three with the share pinned, which gain where the links
+            // come from memory and not from the last-level cache (256 MB).  A
+            // sweep, without / with: 24 chains of 1.1 GB 10.2 / 10.0 ms, 36 of 220
+            // MB 1.88 / 2.10.  12 reals: 720 MB 7.55 / 6.91 ms, 146 MB 1.50 / 1.45.
+            if (B->table_bytes <= (size_t(256) << 20)) go(std::false_type{});
+            else go(std::true_type{});
+        } else {
+            go(std::true_type{});
+        }
     }
 }
 
@@ -5016,6 +5033,7 @@ int qcd_batch_create(const qcd_params* common, int nchains, const qcd_chain_desc
             return rc;
         }
         B->chains.push_back(L);
+        B->table_bytes += L->table_bytes;
         L->batch_owned = true;
         if (L->s_quads != B->chains[0]->s_quads) {   // one produce() size for the batched RANLUX launch
             qcd_batch_destroy(B);

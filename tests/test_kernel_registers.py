@@ -61,6 +61,9 @@ def _waves(vgprs):
     ("k_update1IfLi3ELi18ELb0ELi2ELb1E", 4),        # one wavefront per 64 links, heatbath with the plaquette
     ("k_update1IfLi3ELi18ELb0ELi3ELb1E", 4),
     ("k_update_batch1IfLi3ELi18ELb0ELi2ELb1E", 4),
+    ("k_update_batch3IdLi3ELi12ELb1ELi0ELb0ELb1E", 3),   # overrelaxation of large FP64 batches
+    ("k_update_batch3IdLi3ELi18ELb1ELi0ELb0ELb1E", 3),
+    ("k_update_batch3IdLi3ELi18ELb1ELi0ELb1ELb1E", 3),
 ])
 def test_wavefronts_per_simd(registers, kernel, waves):
     found = [v for n, v in registers.items() if kernel in n]
