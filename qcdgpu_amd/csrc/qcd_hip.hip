@@ -3552,7 +3552,9 @@ struct Stage {
                 return true;
             }
         }
-        if (hipHostMalloc(&mem, n, hipHostMallocPortable) != hipSuccess) {
+        // coherent: what k_links_move writes is in host memory when its event
+        // is done, whatever HIP_HOST_COHERENT says
+        if (hipHostMalloc(&mem, n, hipHostMallocPortable | hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess) {
             (void)hipGetLastError();
             mem = nullptr;
             return false;

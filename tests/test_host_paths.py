@@ -93,3 +93,15 @@ assert "hostfree" not in seen
 assert _abi.lib().qcd_device_close() == 0
 assert calls().count("hostfree") == 1
 """)
+
+
+def test_pinned_memory_is_coherent(fake):
+    """The transfer kernel's writes are read by the host after an event: the memory says
+    so itself (hipHostMallocCoherent), not an environment variable's default."""
+    _run(fake, """
+with Q.Lattice(sun=3, dims=(4, 4, 4, 4), max_measurements=2) as lat:
+    calls()
+    lat.export_links()
+    flags = [int(c.split()[3]) for c in calls() if c.startswith("hostmalloc")]
+assert flags and all(f & 0x40000000 for f in flags), flags
+""")
