@@ -1964,6 +1964,7 @@ struct qcd_lattice {
     float4* rl_next = nullptr;                // its other half when a sweep's quads are produced ahead
     float4* ahead_buf = nullptr;              // quads of kRlAhead half-steps, ahead_quads per stream and half-step
     uint32_t ahead_quads = 0;
+    uint32_t ahead_failed = 0;                // its size when there was no memory for it
     uint4* rl_tab = nullptr;                  // RANLUX: jump tables of its luxury level
     float4* prn_buf = nullptr;                // RANLUX: produced quads, prn_quads per stream
     uint32_t prn_quads = 0;
@@ -2347,21 +2348,28 @@ struct OutsideCapture {
 };
 
 // Its buffers, before a sweep or a capture of sweeps; without them (no memory,
-// or a capture under way) every half-step produces for itself.
-void ahead_prepare(qcd_lattice* L)
+// or a capture under way) every half-step produces for itself.  Sweeps do not
+// ask again for what could not be had, which would make each of them wait for
+// the stream; a recording, which waits for it anyway, does.
+void ahead_prepare(qcd_lattice* L, bool again)
 {
-    if (!ahead_fits(L) || (L->ahead_buf && L->ahead_quads >= update_quads(L))) return;
+    if (!ahead_fits(L)) return;
+    const uint32_t keep = update_quads(L);
+    if ((L->ahead_buf && L->ahead_quads >= keep) || (L->ahead_failed == keep && !again)) return;
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(L->stream, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) return;
     const OutsideCapture outside;
     (void)hipStreamSynchronize(L->stream);
     (void)hipFree(L->ahead_buf);
     L->ahead_buf = nullptr;
-    L->ahead_quads = update_quads(L);
+    L->ahead_quads = keep;
+    L->ahead_failed = 0;
     if ((!L->rl_next && hipMalloc((void**)&L->rl_next, sizeof(float4) * 7 * L->n_inst) != hipSuccess) ||
-        hipMalloc((void**)&L->ahead_buf, sizeof(float4) * kRlAhead * L->ahead_quads * (size_t)L->n_inst) != hipSuccess) {
+        hipMalloc((void**)&L->ahead_buf, sizeof(float4) * kRlAhead * keep * (size_t)L->n_inst) != hipSuccess) {
         (void)hipGetLastError();
-        L->ahead_buf = nullptr;
+        (void)hipFree(L->rl_next);
+        L->ahead_buf = L->rl_next = nullptr;
+        L->ahead_failed = keep;
     }
 }
 void launch_ahead(qcd_lattice* L)
@@ -3136,7 +3144,7 @@ int qcd_graph_begin(qcd_lattice* L)
     if (L->profiling) return fail(QCD_E_STATE, "kernel timing waits for every kernel: no graph while it is on");
     drop_cycle_graphs(L);
     HIPCHK(hipStreamSynchronize(L->stream));
-    ahead_prepare(L);
+    ahead_prepare(L, true);
     HIPCHK(hipStreamBeginCapture(L->stream, hipStreamCaptureModeThreadLocal));
     L->graph_open = true;
     L->graph_counter0 = L->prng_counter;
@@ -3817,7 +3825,7 @@ static int sweep_impl(qcd_lattice* L, int kind, bool fuse_plaquette, std::vector
 int qcd_sweep(qcd_lattice* L, int kind)
 {
     if (!L) return fail(QCD_E_ARG, "null lattice");
-    if (kind == QCD_HEATBATH) ahead_prepare(L);
+    if (kind == QCD_HEATBATH) ahead_prepare(L, false);
     return sweep_impl(L, kind, false, nullptr, nullptr);
 }
 
@@ -4117,7 +4125,7 @@ int qcd_cycle_capture(qcd_lattice* L, int n_hb, int n_or, int mask)
     if (n_hb < 0 || n_or < 0) return fail(QCD_E_ARG, "negative sweep count");
     drop_cycle_graphs(L);
     HIPCHK(hipStreamSynchronize(L->stream));
-    if (n_hb) ahead_prepare(L);
+    if (n_hb) ahead_prepare(L, true);
     // K = QCD_TUNE_CYCLES_PER_GRAPH consecutive cycles as one graph, each
     // cycle's measurement beside the next cycle's first half-steps (replays
     // of whole K-blocks); the single cycle below covers the rest
@@ -4167,7 +4175,7 @@ int qcd_cycle_run(qcd_lattice* L, int n_hb, int n_or, int mask)
 {
     if (!L) return fail(QCD_E_ARG, "null lattice");
     if (n_hb < 0 || n_or < 0) return fail(QCD_E_ARG, "negative sweep count");
-    if (n_hb) ahead_prepare(L);
+    if (n_hb) ahead_prepare(L, false);
     return enqueue_cycle(L, n_hb, n_or, mask, nullptr, nullptr);
 }
 

@@ -105,3 +105,31 @@ with Q.Lattice(sun=3, dims=(4, 4, 4, 4), max_measurements=2) as lat:
     flags = [int(c.split()[3]) for c in calls() if c.startswith("hostmalloc")]
 assert flags and all(f & 0x40000000 for f in flags), flags
 """)
+
+
+def test_sweeps_without_memory_for_quads_ahead(fake):
+    """Where the quads of several half-steps find no memory, sweeps go on as before they
+    were made ahead: no wait and no further attempt in each of them, and nothing kept."""
+    _run(fake, """
+with Q.Lattice(sun=3, dims=(8, 8, 8, 8), prng="RANLUX", max_measurements=2) as lat:
+    lat.prng_init()
+    lat.init("cold")
+    calls()
+    fake.fake_limits(4 << 20, ANY)
+    lat.sweep("hb")
+    first = calls()
+    assert sum(c.startswith("malloc") and c.endswith("failed") for c in first) == 1, first
+    for _ in range(3):
+        lat.sweep("hb")
+    lat.run_cycle(n_hb=1, n_or=0)
+    seen = calls()
+    assert not any(c.startswith(("malloc", "wait")) for c in seen), seen
+    assert sum(c.startswith("launch") for c in seen) >= 4 * 16   # a produce() and an update per half-step
+    fake.fake_limits(ANY, ANY)
+    lat.sweep("hb")   # as before, ...
+    assert sum(c.startswith("launch") for c in calls()) == 16
+    lat.capture_cycle(n_hb=1, n_or=0)   # ... until a recording asks again
+    assert sum(c.startswith("malloc") for c in calls()) == 2
+    lat.sweep("hb")
+    assert sum(c.startswith("launch") for c in calls()) == 10
+""")
