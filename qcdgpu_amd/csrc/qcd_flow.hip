@@ -1494,7 +1494,10 @@ int qcd_flow_create(const qcd_flow_desc* desc, qcd_flow** out)
     const size_t n = V * (size_t)d.max_batch;
     bool ok = hipStreamCreateWithFlags(&F->stream, hipStreamNonBlocking) == hipSuccess;
     ok = ok && hipMalloc((void**)&F->w1, sizeof(uint16_t) * kW1Pack * d.layers) == hipSuccess;
-    ok = ok && hipMemset(F->w1, 0, sizeof(uint16_t) * kW1Pack * d.layers) == hipSuccess;   // the padded k
+    // Cleared (the padded k, the counts) on the stream that packs the weights, which
+    // is not ordered with the null stream; qcd_flow_set_params, which everything else
+    // needs first, waits for it.
+    ok = ok && hipMemsetAsync(F->w1, 0, sizeof(uint16_t) * kW1Pack * d.layers, F->stream) == hipSuccess;
     ok = ok && hipMalloc((void**)&F->staged, sizeof(float) * F->nparam) == hipSuccess;
     ok = ok && hipMalloc((void**)&F->b1, sizeof(float) * kHidden * d.layers) == hipSuccess;
     ok = ok && hipMalloc((void**)&F->w2, sizeof(uint16_t) * kW2 * d.layers) == hipSuccess;
@@ -1507,7 +1510,7 @@ int qcd_flow_create(const qcd_flow_desc* desc, qcd_flow** out)
     ok = ok && hipMalloc((void**)&F->act, sizeof(double) * n) == hipSuccess;
     ok = ok && hipMalloc((void**)&F->sums, sizeof(double) * 2 * d.max_batch) == hipSuccess;
     ok = ok && hipMalloc((void**)&F->imh, 3 * sizeof(unsigned long long)) == hipSuccess;
-    ok = ok && hipMemset(F->imh, 0, 3 * sizeof(unsigned long long)) == hipSuccess;
+    ok = ok && hipMemsetAsync(F->imh, 0, 3 * sizeof(unsigned long long), F->stream) == hipSuccess;
     if (!ok) {
         qcd_flow_destroy(F);
         return err(QCD_E_NOMEM, "flow buffers");
@@ -1557,15 +1560,15 @@ int qcd_flow_set_params(qcd_flow* F, const float* p, size_t n)
     hipLaunchKernelGGL(k_flow_unpack_params, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, F->stream,
                        (const float*)F->staged, (uint32_t)F->d.layers, F->w1, F->b1, F->w2, F->b2);
     FCHK(hipGetLastError());
+    if (F->tp) {   // training continues from these parameters, fresh moments
+        FCHK(hipMemcpyAsync(F->tp, F->staged, sizeof(float) * n, hipMemcpyDeviceToDevice, F->stream));
+        FCHK(hipMemsetAsync(F->tm, 0, sizeof(float) * n, F->stream));
+        FCHK(hipMemsetAsync(F->tv, 0, sizeof(float) * n, F->stream));
+        F->tstep = 0;
+    }
     FCHK(hipStreamSynchronize(F->stream));
     F->host_params.assign(p, p + n);
     F->host_stale = false;
-    if (F->tp) {   // training continues from these parameters, fresh moments
-        FCHK(hipMemcpy(F->tp, p, sizeof(float) * n, hipMemcpyHostToDevice));
-        FCHK(hipMemset(F->tm, 0, sizeof(float) * n));
-        FCHK(hipMemset(F->tv, 0, sizeof(float) * n));
-        F->tstep = 0;
-    }
     return QCD_OK;
 }
 
@@ -1690,10 +1693,10 @@ int train_grad(qcd_flow* F, const float* links, int batch, double* loss)
         ok = ok && hipMalloc((void**)&F->tzero, sizeof(float) * kHidden) == hipSuccess;
         ok = ok && hipMalloc((void**)&F->tsums, sizeof(double) * F->d.layers * F->d.max_batch) == hipSuccess;
         if (!ok) return err(QCD_E_NOMEM, "flow training buffers");
-        FCHK(hipMemcpy(F->tp, F->host_params.data(), sizeof(float) * F->nparam, hipMemcpyHostToDevice));
-        FCHK(hipMemset(F->tm, 0, sizeof(float) * F->nparam));
-        FCHK(hipMemset(F->tv, 0, sizeof(float) * F->nparam));
-        FCHK(hipMemset(F->tzero, 0, sizeof(float) * kHidden));
+        FCHK(hipMemcpyAsync(F->tp, F->host_params.data(), sizeof(float) * F->nparam, hipMemcpyHostToDevice, F->stream));
+        FCHK(hipMemsetAsync(F->tm, 0, sizeof(float) * F->nparam, F->stream));
+        FCHK(hipMemsetAsync(F->tv, 0, sizeof(float) * F->nparam, F->stream));
+        FCHK(hipMemsetAsync(F->tzero, 0, sizeof(float) * kHidden, F->stream));
         F->tstep = 0;
     }
     const uint64_t nl = (uint64_t)B * 4 * g.V;
@@ -1768,7 +1771,10 @@ int qcd_flow_train_grad(qcd_flow* F, const float* links, int batch, double* loss
 {
     const int rc = train_grad(F, links, batch, loss);
     if (rc) return rc;
-    if (grad) FCHK(hipMemcpy(grad, F->tgrad, sizeof(float) * F->nparam, hipMemcpyDeviceToHost));
+    if (grad) {
+        FCHK(hipMemcpyAsync(grad, F->tgrad, sizeof(float) * F->nparam, hipMemcpyDeviceToHost, F->stream));
+        FCHK(hipStreamSynchronize(F->stream));
+    }
     return QCD_OK;
 }
 
@@ -1814,7 +1820,10 @@ int qcd_flow_imh_counts(qcd_flow* F, unsigned long long* accepted, unsigned long
     FCHK(hipMemcpy(a, F->imh, sizeof(a), hipMemcpyDeviceToHost));
     if (accepted) *accepted = a[0];
     if (proposed) *proposed = a[1] * (unsigned long long)F->d.layers * (F->g.V / 2);   // every layer proposes V/2 links
-    if (reset) FCHK(hipMemset(F->imh, 0, 2 * sizeof(unsigned long long)));   // the seed stays
+    if (reset) {   // the seed stays
+        FCHK(hipMemsetAsync(F->imh, 0, 2 * sizeof(unsigned long long), F->stream));
+        FCHK(hipStreamSynchronize(F->stream));
+    }
     return QCD_OK;
 }
 

@@ -133,3 +133,28 @@ with Q.Lattice(sun=3, dims=(8, 8, 8, 8), prng="RANLUX", max_measurements=2) as l
     lat.sweep("hb")
     assert sum(c.startswith("launch") for c in calls()) == 10
 """)
+
+
+def test_flow_works_on_its_own_stream(fake):
+    """The flow's stream does not wait for the null stream nor the null stream for it: what
+    is cleared, packed and copied follows in one order, and a gradient is waited for before
+    it is read, also when the loss is not asked for."""
+    _run(fake, """
+from qcdgpu_amd import flow as QF, _abi
+f = QF.Flow(dims=(4, 4, 4, 4), layers=2, max_batch=2)
+p = np.zeros(f.param_count(), np.float32)
+f.set_params(p)
+links = np.ones((2, 4, 256, 4), np.float32)
+f.train_grad(links)
+f.set_params(p)
+f.train_step(links, 1e-3)
+f.imh_counts(reset=True)
+seen = calls()
+assert not any(c.startswith("clear") and " on " not in c for c in seen), seen
+g = np.empty_like(p)
+P = ctypes.POINTER(ctypes.c_float)
+assert _abi.lib().qcd_flow_train_grad(f._h, links.ctypes.data_as(P), 2, None, g.ctypes.data_as(P)) == 0
+seen = calls()
+copy = [i for i, c in enumerate(seen) if c.startswith("copy kind 2")][-1]
+assert " on " in seen[copy] and seen[copy + 1].startswith("wait on"), seen[copy:]
+""")
