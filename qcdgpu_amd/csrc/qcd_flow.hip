@@ -1461,6 +1461,26 @@ int finish(qcd_flow* F, uint32_t B, double beta, double* logq, double* action)
     return QCD_OK;
 }
 
+// The training buffers; all are there or none.
+void free_training(qcd_flow* F)
+{
+    auto drop = [](auto*& q) {
+        (void)hipFree(q);
+        q = nullptr;
+    };
+    drop(F->tp);
+    drop(F->tgrad);
+    drop(F->tm);
+    drop(F->tv);
+    drop(F->tg);
+    drop(F->tdpre);
+    drop(F->tloss);
+    drop(F->tw2t);
+    drop(F->tpart);
+    drop(F->tzero);
+    drop(F->tsums);
+}
+
 int check_batch(const qcd_flow* F, int batch)
 {
     if (batch < 1 || batch > F->d.max_batch)
@@ -1536,9 +1556,7 @@ int qcd_flow_destroy(qcd_flow* F)
     (void)hipFree(F->act);
     (void)hipFree(F->sums);
     (void)hipFree(F->imh);
-    for (void* q : {(void*)F->tp, (void*)F->tgrad, (void*)F->tm, (void*)F->tv, (void*)F->tg, (void*)F->tdpre, (void*)F->tloss, (void*)F->tw2t, (void*)F->tpart, (void*)F->tzero,
-                    (void*)F->tsums})
-        (void)hipFree(q);
+    free_training(F);
     if (F->stream) (void)hipStreamDestroy(F->stream);
     delete F;
     return QCD_OK;
@@ -1692,7 +1710,11 @@ int train_grad(qcd_flow* F, const float* links, int batch, double* loss)
         ok = ok && hipMalloc((void**)&F->tpart, sizeof(float) * part_max) == hipSuccess;
         ok = ok && hipMalloc((void**)&F->tzero, sizeof(float) * kHidden) == hipSuccess;
         ok = ok && hipMalloc((void**)&F->tsums, sizeof(double) * F->d.layers * F->d.max_batch) == hipSuccess;
-        if (!ok) return err(QCD_E_NOMEM, "flow training buffers");
+        if (!ok) {
+            (void)hipGetLastError();
+            free_training(F);
+            return err(QCD_E_NOMEM, "flow training buffers");
+        }
         FCHK(hipMemcpyAsync(F->tp, F->host_params.data(), sizeof(float) * F->nparam, hipMemcpyHostToDevice, F->stream));
         FCHK(hipMemsetAsync(F->tm, 0, sizeof(float) * F->nparam, F->stream));
         FCHK(hipMemsetAsync(F->tv, 0, sizeof(float) * F->nparam, F->stream));

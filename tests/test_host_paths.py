@@ -158,3 +158,26 @@ seen = calls()
 copy = [i for i, c in enumerate(seen) if c.startswith("copy kind 2")][-1]
 assert " on " in seen[copy] and seen[copy + 1].startswith("wait on"), seen[copy:]
 """)
+
+
+def test_training_without_memory(fake):
+    """A gradient that finds no memory for its buffers is refused, each time, and works
+    once there is memory: never a launch on buffers that were not had."""
+    _run(fake, """
+from qcdgpu_amd import flow as QF
+f = QF.Flow(dims=(4, 4, 4, 4), layers=1, max_batch=64)
+f.set_params(np.zeros(f.param_count(), np.float32))
+links = np.ones((2, 4, 256, 4), np.float32)
+calls()
+fake.fake_limits(300000, ANY)   # parameters fit, the partial sums do not
+for _ in range(2):
+    try:
+        f.train_grad(links)
+        raise SystemExit("accepted")
+    except Q.QCDError as e:
+        assert "training buffers" in str(e)
+assert not any(c.startswith("launch") for c in calls())
+fake.fake_limits(ANY, ANY)
+f.train_grad(links)
+assert any(c.startswith("launch") for c in calls())
+""")
