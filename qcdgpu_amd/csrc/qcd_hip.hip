@@ -2431,6 +2431,7 @@ int launch_update_rn(qcd_lattice* L, int parity, int mu, int kind, int start_gid
         if (L->quad_buffer) {
             // the reference's produce() into the PRN buffer, then the update
             // reads quad k of link i at k * PRNGSTEP + i
+            if (!o.prn && !L->prn_buf) return fail(QCD_E_STATE, "no memory was found for the PRN quad buffer: start again");
             if (!o.prn) {
                 ProfScope ps(L, "PRNG produce");
                 produce_quads_into(L, L->s_quads, update_quads(L), L->prn_buf);
@@ -2758,7 +2759,7 @@ static int set_sizing(qcd_lattice* L, bool hot_run, bool* changed)
 {
     *changed = false;
     const uint32_t S = produce_quads(L->p, L->g.vh, hot_run);
-    if (S == L->s_quads && hot_run == L->hot_run) return QCD_OK;
+    if (S == L->s_quads && hot_run == L->hot_run && (!L->quad_buffer || L->prn_buf)) return QCD_OK;
     if (L->batch_owned)
         return fail(QCD_E_STATE, "a batched chain keeps its stream sizing (its batch holds the buffers): "
                                  "no reference hot start or resume of a hot run on it");
@@ -2770,9 +2771,13 @@ static int set_sizing(qcd_lattice* L, bool hot_run, bool* changed)
     if (L->quad_buffer && L->prn_quads < S) {
         (void)hipFree(L->prn_buf);
         L->prn_buf = nullptr;
-        L->prn_quads = S;
-        if (hipMalloc((void**)&L->prn_buf, sizeof(float4) * (size_t)S * L->n_inst) != hipSuccess)
+        L->prn_quads = 0;   // none, until a start or an image asks again
+        if (hipMalloc((void**)&L->prn_buf, sizeof(float4) * (size_t)S * L->n_inst) != hipSuccess) {
+            (void)hipGetLastError();
+            L->prn_buf = nullptr;
             return fail(QCD_E_NOMEM, "PRN quad buffer of %u quads per instance", S);
+        }
+        L->prn_quads = S;
     }
     return build_jumps(L);
 }

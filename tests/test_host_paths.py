@@ -181,3 +181,28 @@ fake.fake_limits(ANY, ANY)
 f.train_grad(links)
 assert any(c.startswith("launch") for c in calls())
 """)
+
+
+def test_start_without_memory_for_quads(fake):
+    """A hot start that finds no memory for its larger quad buffer is refused; so are
+    half-steps after it, until a start finds memory: never an update on no buffer."""
+    _run(fake, """
+def refused(f):
+    try:
+        f()
+    except Q.QCDError:
+        return
+    raise SystemExit("accepted")
+with Q.Lattice(sun=3, dims=(8, 8, 8, 8), prng="RANLUX", max_measurements=2) as lat:
+    lat.prng_init()
+    lat.init("cold")
+    fake.fake_limits(1200000, ANY)   # 33 quads per stream fit, 41 do not
+    refused(lambda: lat.init("random"))
+    calls()
+    refused(lambda: lat.halfstep(1, 0, "hb"))
+    refused(lambda: lat.init("random"))
+    assert not any(c.startswith("launch") for c in calls())
+    fake.fake_limits(ANY, ANY)
+    lat.init("random")
+    lat.halfstep(1, 0, "hb")
+""")
