@@ -4529,6 +4529,8 @@ int qcd_lattice_state_load(qcd_lattice* L, const void* buf, size_t bytes)
     if (r.u32() != L->p.prng_instances) return fail(QCD_E_ARG, "state image has another prng_instances than this lattice");
     r.p += 4;
     if (ready & ~3u) return fail(QCD_E_ARG, "state image with unknown start flags %#x", ready);
+    if ((int)wr < 1 || (int)wt < 1)   // as qcd_lattice_set_wilson; the kernel's lines have at least one link
+        return fail(QCD_E_ARG, "state image with a Wilson loop of %d x %d", (int)wr, (int)wt);
     bool changed = false;
     int rc = set_sizing(L, (ready & 2u) != 0, &changed);   // the run's produce() size
     if (rc) return rc;

@@ -206,3 +206,27 @@ with Q.Lattice(sun=3, dims=(8, 8, 8, 8), prng="RANLUX", max_measurements=2) as l
     lat.init("random")
     lat.halfstep(1, 0, "hb")
 """)
+
+
+def test_image_with_wilson_extents_of_none(fake):
+    """A state image whose Wilson loop has no extent, which no lattice can have set, is
+    refused: the loop kernel's lines start from a link and step by the extents."""
+    _run(fake, """
+with Q.Lattice(sun=2, dims=(4, 4, 4, 4), max_measurements=2) as lat:
+    lat.set_wilson(21, 34)
+    img = lat.save_state()
+    at = [i for i in range(0, 512, 4) if img[i:i + 8].tobytes() == np.array([21, 34], "<u4").tobytes()]
+    assert len(at) == 1, at
+    lat.load_state(img)
+    for field in (0, 4):
+        for value in (0, -3):
+            bad = img.copy()
+            bad[at[0] + field:at[0] + field + 4] = np.frombuffer(np.array([value], "<i4").tobytes(), np.uint8)
+            try:
+                lat.load_state(bad)
+            except Q.QCDError as e:
+                assert "Wilson" in str(e)
+            else:
+                raise SystemExit("accepted")
+    lat.load_state(img)
+""")
