@@ -1966,6 +1966,7 @@ struct qcd_lattice {
     uint32_t ahead_quads = 0;
     uint32_t ahead_failed = 0;                // its size when there was no memory for it
     uint4* rl_tab = nullptr;                  // RANLUX: jump tables of its luxury level
+    bool rl_tab_shared = false;               // those of its batch's first chain
     float4* prn_buf = nullptr;                // RANLUX: produced quads, prn_quads per stream
     uint32_t prn_quads = 0;
     uint32_t pm_ak = 1;                       // Park-Miller jump multiplier
@@ -2782,7 +2783,9 @@ static int set_sizing(qcd_lattice* L, bool hot_run, bool* changed)
     return build_jumps(L);
 }
 
-int qcd_lattice_create(const qcd_params* pp, qcd_lattice** out)
+// first: the batch's first chain, whose RANLUX tables the others use (253 kB and
+// a copy each otherwise: a batch of 96 chains 41 ms, with shared tables 34).
+static int lattice_create(const qcd_params* pp, const qcd_lattice* first, qcd_lattice** out)
 {
     if (!pp || !out) return fail(QCD_E_ARG, "null argument");
     const qcd_params& p = *pp;
@@ -2863,9 +2866,13 @@ int qcd_lattice_create(const qcd_params* pp, qcd_lattice** out)
         // One produce() per heatbath half-step (s_quads per instance) or, with
         // PRNGSTEP instances, per Haar start (8 links x 3 quads for SU(3)).
         L->prn_quads = L->s_quads > 24u ? L->s_quads : 24u;
+        if (first) {
+            L->rl_tab = first->rl_tab;
+            L->rl_tab_shared = true;
+        }
         if ((p.prng == QCD_PRNG_RANLUX &&
              (hipMalloc((void**)&L->rl_state, sizeof(float4) * 7 * L->n_inst) != hipSuccess ||
-              !alloc_rl_tables(p.ranlux_luxury, &L->rl_tab))) ||
+              (!first && !alloc_rl_tables(p.ranlux_luxury, &L->rl_tab)))) ||
             hipMalloc((void**)&L->prn_buf, sizeof(float4) * (size_t)L->prn_quads * L->n_inst) != hipSuccess) {
             qcd_lattice_destroy(L);
             return fail(QCD_E_NOMEM, "PRN quad buffer");
@@ -2898,6 +2905,8 @@ int qcd_lattice_create(const qcd_params* pp, qcd_lattice** out)
     return QCD_OK;
 }
 
+int qcd_lattice_create(const qcd_params* pp, qcd_lattice** out) { return lattice_create(pp, nullptr, out); }
+
 int qcd_lattice_destroy(qcd_lattice* L)
 {
     if (!L) return QCD_OK;
@@ -2917,7 +2926,7 @@ int qcd_lattice_destroy(qcd_lattice* L)
     (void)hipFree(L->rl_state);
     (void)hipFree(L->rl_next);
     (void)hipFree(L->ahead_buf);
-    (void)hipFree(L->rl_tab);
+    if (!L->rl_tab_shared) (void)hipFree(L->rl_tab);
     (void)hipFree(L->prn_buf);
     (void)hipFree(L->partials);
     (void)hipFree(L->rec_index);
@@ -5044,7 +5053,7 @@ int qcd_batch_create(const qcd_params* common, int nchains, const qcd_chain_desc
         q.beta = chains[c].beta;
         q.randseries = chains[c].randseries;
         qcd_lattice* L = nullptr;
-        const int rc = qcd_lattice_create(&q, &L);
+        const int rc = lattice_create(&q, c ? B->chains[0] : nullptr, &L);
         if (rc) {
             qcd_batch_destroy(B);
             return rc;
@@ -5108,9 +5117,9 @@ int qcd_batch_destroy(qcd_batch* B)
     if (B->stream) (void)hipStreamSynchronize(B->stream);
     if (B->exec) (void)hipGraphExecDestroy(B->exec);
     if (B->graph) (void)hipGraphDestroy(B->graph);
-    for (auto* L : B->chains) {
-        L->batch_owned = false;
-        qcd_lattice_destroy(L);
+    for (size_t c = B->chains.size(); c-- > 0;) {   // the first one, whose tables the others use, last
+        B->chains[c]->batch_owned = false;
+        qcd_lattice_destroy(B->chains[c]);
     }
     (void)hipFree(B->d_desc);
     (void)hipFree(B->d_map);

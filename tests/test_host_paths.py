@@ -230,3 +230,24 @@ with Q.Lattice(sun=2, dims=(4, 4, 4, 4), max_measurements=2) as lat:
                 raise SystemExit("accepted")
     lat.load_state(img)
 """)
+
+
+def test_batch_has_one_set_of_ranlux_tables(fake):
+    """The chains of a batch share the luxury level's tables instead of each allocating
+    and filling its own; they are freed once."""
+    _run(fake, """
+tables = "copy kind 1 bytes 253440"
+chains = [((4, 4, 4, 4), 5.7, k + 1) for k in range(5)]
+calls()
+for _ in range(2):
+    with Q.Batch(chains, sun=3, prng="RANLUX", max_measurements=2) as b:
+        assert calls().count(tables) == 1
+        b.init("cold")
+        b.sweep("hb")
+        b.sync()
+calls()
+with Q.Lattice(sun=3, dims=(4, 4, 4, 4), prng="RANLUX", max_measurements=2):
+    assert calls().count(tables) == 1
+with Q.Batch(chains, sun=3, prng="XOR128", max_measurements=2):
+    assert calls().count(tables) == 0
+""")
