@@ -2122,6 +2122,7 @@ struct LaunchOpt {
     hipEvent_t e1 = nullptr;
     uint32_t lds = 0;   // extra dynamic LDS per workgroup (caps workgroups per CU)
     const float4* prn = nullptr;   // this half-step's quads, produced already
+    bool produced = false;         // a batch's quads are in its chains' buffers
 };
 
 template <typename Kern, typename... Args>
@@ -4937,7 +4938,7 @@ template <typename R, int N, int NREAL>
 int batch_halfstep_rn(qcd_batch* B, int parity, int mu, int kind, int meas_mode, int only, const LaunchOpt& o)
 {
     const qcd_params& p = B->p;
-    if (kind == QCD_HEATBATH && p.prng == QCD_PRNG_RANLUX) {
+    if (kind == QCD_HEATBATH && p.prng == QCD_PRNG_RANLUX && !o.produced) {
         const uint32_t S = B->chains[0]->s_quads;
         const dim3 grid(B->len_units), block(kLinks);
         const uint2* map = B->d_map + B->off_units;
@@ -5256,9 +5257,26 @@ int qcd_batch_autotune(qcd_batch* B, int repeats, int* shapes_out)
         ok = ok && save(L->rl_state, L->rl_state ? sizeof(float4) * 7 * L->n_streams : 0);
     }
     const int rng_cur0 = B->rng_cur;
+    const size_t maps0 = B->mmap_old.size() + (B->d_mmap ? 1 : 0);   // a captured cycle may hold these
     hipEvent_t e0, e1;
     int rc = QCD_OK;
     if (ok && hipEventCreate(&e0) == hipSuccess && hipEventCreate(&e1) == hipSuccess) {
+        // one untimed half-step of bucket `only` (-1: all), then `repeats` timed
+        // ones, all on the quads of the first (RANLUX: their production is the
+        // same for every choice, and most of the time)
+        LaunchOpt o;
+        auto timed = [&](int kind, int only) {
+            const int k = kind == 0 ? QCD_HEATBATH : QCD_OVERRELAX;
+            rc = DISPATCH(B, batch_halfstep_rn, B, 1, 0, k, 0, only, o);
+            if (kind == 0) o.produced = true;
+            (void)hipEventRecord(e0, B->stream);
+            for (int r = 0; r < repeats && !rc; ++r) rc = DISPATCH(B, batch_halfstep_rn, B, r & 1, (r >> 1) & 3, k, 0, only, o);
+            (void)hipEventRecord(e1, B->stream);
+            (void)hipEventSynchronize(e1);
+            float t = 0.f;
+            (void)hipEventElapsedTime(&t, e0, e1);
+            return t;
+        };
         for (size_t k = 0; k < B->buckets.size() && !rc; ++k)
             for (int kind = 0; kind < 2 && !rc; ++kind) {
                 float best = 1e30f;
@@ -5267,17 +5285,7 @@ int qcd_batch_autotune(qcd_batch* B, int repeats, int* shapes_out)
                     const int shape = (cand % 2) ? 1 : 3, place = cand / 2;
                     B->buckets[k].shape[kind] = shape;
                     B->buckets[k].place[kind] = place;
-                    // one untimed launch, then `repeats` timed ones
-                    rc = DISPATCH(B, batch_halfstep_rn, B, 1, 0, kind == 0 ? QCD_HEATBATH : QCD_OVERRELAX, 0, (int)k,
-                                  LaunchOpt{});
-                    (void)hipEventRecord(e0, B->stream);
-                    for (int r = 0; r < repeats && !rc; ++r)
-                        rc = DISPATCH(B, batch_halfstep_rn, B, r & 1, (r >> 1) & 3,
-                                      kind == 0 ? QCD_HEATBATH : QCD_OVERRELAX, 0, (int)k, LaunchOpt{});
-                    (void)hipEventRecord(e1, B->stream);
-                    (void)hipEventSynchronize(e1);
-                    float t = 0.f;
-                    (void)hipEventElapsedTime(&t, e0, e1);
+                    const float t = timed(kind, (int)k);
                     if (t < best) {
                         best = t;
                         best_shape = shape;
@@ -5287,6 +5295,33 @@ int qcd_batch_autotune(qcd_batch* B, int repeats, int* shapes_out)
                 B->buckets[k].shape[kind] = best_shape;
                 B->buckets[k].place[kind] = best_place;
             }
+        // The buckets run merged, and a second launch for those of the other
+        // shape can cost more than they gain by it: their choices stand against
+        // every one for all, timed as it will run.  (36 chains of FP32 12-real
+        // SU(3), 8^3 x 4 to 16^3 x 6: a step of 1 + 2 sweeps took 537 to 630 us by
+        // which way single buckets fell; now 538 to 549.)
+        for (int kind = 0; kind < 2 && B->merge && B->buckets.size() > 1 && !rc; ++kind) {
+            std::vector<std::pair<int, int>> best;
+            float best_t = 1e30f;
+            for (int cand = -1; cand < 2 * qcd_batch::kPlacements && !rc; ++cand) {
+                if (cand >= 0)
+                    for (auto& bk : B->buckets) {
+                        bk.shape[kind] = (cand % 2) ? 1 : 3;
+                        bk.place[kind] = cand / 2;
+                    }
+                rc = build_merged(B);
+                const float t = rc ? 0.f : timed(kind, -1);
+                if (!rc && t < best_t) {
+                    best_t = t;
+                    best.clear();
+                    for (const auto& bk : B->buckets) best.emplace_back(bk.shape[kind], bk.place[kind]);
+                }
+            }
+            for (size_t k = 0; k < best.size(); ++k) {
+                B->buckets[k].shape[kind] = best[k].first;
+                B->buckets[k].place[kind] = best[k].second;
+            }
+        }
         (void)hipEventDestroy(e0);
         (void)hipEventDestroy(e1);
     } else {
@@ -5313,7 +5348,12 @@ int qcd_batch_autotune(qcd_batch* B, int repeats, int* shapes_out)
             shapes_out[2 * k + 1] = B->buckets[k].shape[1];
         }
     // a captured cycle keeps the shapes it was captured with
-    return build_merged(B);
+    rc = build_merged(B);
+    while (B->mmap_old.size() > maps0) {   // maps of the timing
+        (void)hipFree(B->mmap_old.back());
+        B->mmap_old.pop_back();
+    }
+    return rc;
 }
 
 int qcd_batch_set_tuning(qcd_batch* B, int bucket, int shape_hb, int shape_or, int place_hb, int place_or)

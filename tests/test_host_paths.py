@@ -251,3 +251,27 @@ with Q.Lattice(sun=3, dims=(4, 4, 4, 4), prng="RANLUX", max_measurements=2):
 with Q.Batch(chains, sun=3, prng="XOR128", max_measurements=2):
     assert calls().count(tables) == 0
 """)
+
+
+def test_autotune_times_what_will_run(fake):
+    """The buckets of a batch run merged, so the tuner times merged half-steps too, and the
+    choice is made on one production of the RANLUX quads; the maps it made are given back."""
+    _run(fake, """
+chains = [((8, 8, 8, 4), 5.7, 1), ((8, 8, 8, 6), 5.7, 2), ((6, 6, 6, 8), 5.7, 3)]
+grid = lambda c: int(c.split()[1])
+with Q.Batch(chains, sun=3, prng="RANLUX", max_measurements=2) as b:
+    b.init("cold")
+    b.sync()
+    calls()
+    b.sweep("or")
+    merged = {grid(c) for c in calls() if c.startswith("launch")}
+    assert len(merged) == 1
+    b.sweep("hb")
+    produce = {grid(c) for c in calls() if c.startswith("launch")} - merged
+    b.autotune(repeats=2)
+    seen = [grid(c) for c in calls() if c.startswith("launch")]
+    assert seen.count(next(iter(merged))) >= 2 * 3, seen
+    assert sum(seen.count(g) for g in produce) <= 1, (produce, seen)
+    b.sweep("or")
+    assert {grid(c) for c in calls() if c.startswith("launch")} == merged   # every time is equal here: the first choice
+""")
