@@ -275,3 +275,19 @@ with Q.Batch(chains, sun=3, prng="RANLUX", max_measurements=2) as b:
     b.sweep("or")
     assert {grid(c) for c in calls() if c.startswith("launch")} == merged   # every time is equal here: the first choice
 """)
+
+
+def test_flow_parameters_are_uploaded_by_a_plain_copy(fake):
+    """Parameters come from a caller's array that is often new; a plain copy stages it,
+    and is waited for before the flow's stream packs it."""
+    _run(fake, """
+from qcdgpu_amd import flow as QF
+f = QF.Flow(dims=(4, 4, 4, 4), layers=2, max_batch=2)
+p = np.zeros(f.param_count(), np.float32)
+calls()
+f.set_params(p)
+seen = calls()
+at = seen.index("copy kind 1 bytes %d" % p.nbytes)
+assert seen[at + 1].startswith("wait on 0") or seen[at + 1] == "wait on ", seen
+assert seen[at + 2].startswith("launch"), seen
+""")
