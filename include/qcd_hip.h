@@ -111,7 +111,8 @@ typedef struct {
 typedef struct qcd_lattice qcd_lattice;
 
 /* ---- device (GPU::device_select / device_initialize / device_finalize,
-        clinterface.cpp:347-459) ------------------------------------------ */
+        clinterface.cpp:347-459).  qcd_device_close gives back the pinned
+        memory kept between link copies (at most 16 MiB). ------------------ */
 int         qcd_device_open(int platform, int device);
 int         qcd_device_close(void);
 int         qcd_device_info(char *name, int name_len, int *compute_units, size_t *global_mem);
@@ -289,10 +290,17 @@ int  qcd_lattice_init(qcd_lattice *lat, int start);
 
 /* ---- PRNG (PRNG::initialize, random.cpp:216-277): seeds the per-site
         streams through glibc srand(RANDSERIES)/rand() in the reference order
-        and performs the initial produce().                                  */
+        and performs the initial produce().  A RANLUX lattice that sweeps
+        keeps, beside the quad buffer of one half-step, the quads of four
+        half-steps where these take at most 192 MiB, and a second state
+        buffer (112 B per stream); without that memory its half-steps produce
+        for themselves, with the same results.                               */
 int  qcd_prng_init(qcd_lattice *lat);
 
-/* ---- host copies (buffer_init / buffer_map, clinterface.cpp:1316-1433) */
+/* ---- host copies (buffer_init / buffer_map, clinterface.cpp:1316-1433),
+        through pinned memory (up to 16 MiB, kept until qcd_device_close) and
+        up to eight threads; without pinned memory through ordinary memory
+        of the table's size.                                                */
 int  qcd_lattice_import(qcd_lattice *lat, const double *links);
 int  qcd_lattice_export(qcd_lattice *lat, double *links);   /* synchronous */
 
@@ -517,7 +525,8 @@ int  qcd_batch_sync(qcd_batch *batch);
    units over the 8 XCDs (0: every chain whole on one XCD, units in index
    order; 1: the same in cross-section order, x fastest, then t, then z;
    2: every chain cut into eight slabs, one per XCD) and keeps the fastest
-   per bucket and update kind; chains are saved and restored around the
+   per bucket and update kind, or for all buckets where that is faster once
+   they run in one launch; chains are saved and restored around the
    timing, so results do not depend on it.  shapes_out (optional): 2 ints
    per bucket (heatbath, overrelaxation shape).  Capture the cycle after
    tuning.                                                                 */
@@ -578,7 +587,9 @@ int  qcd_flow_evaluate(qcd_flow *flow, const float *links, int batch, double bet
    independently replaced by the layer's map of a Haar draw with probability
    min(1, exp(-dS) q(U)/q(U')) -- exact Metropolis-within-Gibbs, since the
    layer's conditioners see frozen links only and no plaquette holds two
-   active links.  Eight layers visit every link once.  Asynchronous.        */
+   active links.  Eight layers visit every link once.  Asynchronous, and in
+   the flow's own buffers: qcd_lattice_sync comes before any other call of the
+   same flow but sweeps of this lattice and qcd_flow_imh_counts.             */
 int  qcd_flow_imh_sweep(qcd_flow *flow, qcd_lattice *lat, unsigned long long seed, double beta);
 /* The sweep's seed lives on the device: qcd_flow_imh_sweep sets it;
    qcd_flow_imh_sweep_next runs the sweep with the previous seed + 1, so a

@@ -426,7 +426,7 @@ __global__ __launch_bounds__(256) void k_flow_conv(const uint16_t* in, const uin
     }
 }
 
-// The same sums with the input in LDS: one workgroup of 4 wavefronts per
+// The same sums with the input in LDS: one workgroup of WV wavefronts per
 // x-plane of a configuration stages the plane and its two neighbours (`plane`
 // sites each, contiguous) and every one of the 81 gathers of a site reads
 // from there.  A wavefront takes MT tiles of 16 sites at a time.

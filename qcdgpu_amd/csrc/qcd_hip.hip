@@ -2180,8 +2180,9 @@ uint32_t update_unit0(const qcd_lattice* L) { return L->slab ? L->g.vh / (uint32
 // 1 / z-extent) of the table for a block that is cut along both
 // (periodic full extents have no halo).  A mode that does not apply falls
 // back to mode 1 (and to 0 when shape1 needs whole workgroups of four
-// units per XCD and does not get them).  Mode 1 takes any number of units
-// (the XCDs' ranges differ by at most one); 20 x 12 x 28 x 10, 525 units,
+// units per XCD and does not get them).  Mode 1 takes any number of units:
+// ranges of an eighth rounded up, what is left for the last ones (525 units: 7 x
+// 66 and 63; 12: 6 x 2 and none); 20 x 12 x 28 x 10, 525 units,
 // against hardware order: FP64 overrelaxation half-step 16.7 -> 11.4 us,
 // heatbath 23.3 -> 18.0 us, 12-real FP32 8.5 -> 7.7 and 10.7 -> 10.0 us.
 void dispatch_order(const qcd_lattice* L, int want, bool shape1, UpdArgs& a)
@@ -2326,7 +2327,9 @@ void produce_quads_into(qcd_lattice* L, uint32_t samples, uint32_t keep, float4*
 // once fill the chip instead.  Heatbath half-step with its produce(): 8^4 SU(2)
 // 11.5 to 7.7 us, 16^4 12.5 to 9.3; SU(3) 8^4 15.3 to 11.0, 20 x 12 x 28 x 10
 // 24.9 to 18.7, 24^3 x 12 (175 MB of quads) 40.4 to 30.6.  Beyond what the last-level
-// cache holds the quads come back from memory: SU(2) 32^4 (369 MB) 63.3 to 69.1.
+// cache holds the quads come back from memory: SU(2) 32^4 (369 MB) 63.3 to 69.1;
+// the limit lies between, not measured closer.  rl_waves' counts of streams, which
+// decide here too, were taken for single produce() calls.
 constexpr size_t kAheadBytes = size_t(192) << 20;
 bool ahead_fits(const qcd_lattice* L)
 {
